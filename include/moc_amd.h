@@ -208,8 +208,9 @@ int moc_gemm_residual_bf16(int64_t M, int64_t N, int64_t K, const void* A, int64
  * C1/C2 row-major (ldc1, ldc2).  The gate and up projections of the MoC FFN
  * input, G = x W_gate^T and U = x W_up^T (moc/ffn.py:141,146 for `moc`,
  * :389,394 for `moc_gcp`), which the reference runs as two library GEMMs.
- * Results equal two moc_gemm_ws calls bit for bit; pairs too small to fill
- * the CUs run as exactly those two calls (with the given workspace). */
+ * A pair that fills the CUs runs unsplit on 256-wide tiles, a smaller one
+ * unsplit on small tiles (the same k order of every sum), or as two
+ * moc_gemm_ws calls (with the given workspace). */
 int moc_gemm_pair(int64_t M, int64_t K, const void* A, int64_t lda, const void* W1, int64_t ldw1,
                   int64_t N1, void* C1, int64_t ldc1, const void* W2, int64_t ldw2, int64_t N2,
                   void* C2, int64_t ldc2, void* workspace, int64_t workspace_bytes, void* stream);

@@ -1249,6 +1249,182 @@ void gemm_pp_kernel(GemmArgs g) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Small-tile variant: BM x BN C tiles (64 or 128 each way), four waves, for
+// products whose 256x256 tiles would leave most CUs idle (a decode batch or
+// short prompt of 17 to a few hundred tokens, the short or narrow products of
+// small training batches).  Such a launch is bound by how many bytes it keeps
+// in flight and by the length of one workgroup's K loop, not by MFMA rate, so
+// it wants many workgroups with deep load queues rather than large tiles: two
+// or more workgroups share a CU, each with NS - 1 K tiles requested ahead by
+// direct-to-LDS loads into an NS-slot ring, and one barrier per K tile.
+//
+// Wave (wm, wn) of 2 x 2 owns a BM/2 x BN/2 block.  Tiles keep the layouts of
+// the 256-wide kernels (KC: 128-byte rows of 64 k; MN: k-rows of the tile's
+// columns) with the same fragment reads; an MN tile's row is 2 BN (or 2 BM)
+// bytes, and for 128-byte rows the chunk swizzle is {0, 0, 4, 4}: rows r and
+// r + 1 already lie on different halves of the 64 banks.
+// ---------------------------------------------------------------------------
+constexpr int kMidThreads = 256;
+
+template <bool KC, int EXT>
+struct MidMap {
+  static constexpr int kInstr = EXT / 32;            // wave loads per wave and K tile
+  static constexpr int kRowBytes = KC ? kBK * 2 : EXT * 2;
+  static constexpr int kRows = 1024 / kRowBytes;     // tile rows per wave load
+  static constexpr int kLanes = 64 / kRows;          // lanes (16-byte chunks) per row
+  uint32_t voff0;  // byte offset of load 0 at k = 0
+  int kchunk;      // KC: first k of this lane's chunk within a tile
+  uint32_t base;   // LDS byte of the lane's fragment of block 0, k16 step 0
+
+  static __device__ __forceinline__ int swz(int r) {
+    return KC ? kc_swz(r & 15) : (kRowBytes == 128 ? ((r >> 1) & 1) * 4 : mn_swz(r & 3));
+  }
+  __device__ __forceinline__ void init(const Operand& o, int row0, int wofs, uint32_t region, int wave, int lane) {
+    const int r = wave * kRows + lane / kLanes;  // load j: + 4 kRows j (a multiple of 16: same swizzle)
+    const int c = (lane % kLanes) ^ swz(r);
+    kchunk = KC ? 8 * c : 0;
+    const int64_t e = KC ? static_cast<int64_t>(row0 + r) * o.ld + 8 * c : static_cast<int64_t>(r) * o.ld + row0 + 8 * c;
+    voff0 = static_cast<uint32_t>(e * 2);
+    if (KC) {
+      base = region + static_cast<uint32_t>((wofs + (lane & 31)) * kRowBytes + (((lane >> 5) ^ swz(lane & 15)) * 16));
+    } else {
+      const int i = lane & 15, q = lane >> 4;
+      const int kr = 8 * (q >> 1) + (i >> 2);
+      const int ch = (wofs + 16 * (q & 1) + 4 * (i & 3)) >> 3;
+      base = region + static_cast<uint32_t>(kr * kRowBytes + 8 * (i & 1) + 16 * (ch ^ swz(i >> 2)));
+    }
+  }
+  // the K tile at k0 into the region at LDS byte `tile`; chunks or k-rows
+  // past K, and rows past the extent, read as zero (buffer range check)
+  __device__ __forceinline__ void issue(__amdgpu_buffer_rsrc_t rsrc, const Operand& o, int k0, uint32_t tile,
+                                        int wave) const {
+    uint32_t b = voff0 + (KC ? static_cast<uint32_t>(k0) * 2u : static_cast<uint32_t>(static_cast<int64_t>(k0) * o.ld * 2));
+    if (KC && k0 + kchunk >= o.K) b = kOob;
+    const uint32_t stride = static_cast<uint32_t>(4 * kRows * o.ld * 2);
+#pragma unroll
+    for (int j = 0; j < kInstr; ++j)
+      dma16(rsrc, __builtin_amdgcn_readfirstlane(tile + (j * 4 + wave) * 1024), b + j * stride);
+  }
+  // KC, K % 8 != 0: zero the elements k >= K of the chunk that straddles K
+  __device__ __forceinline__ void zero_straddle(char* lds, const Operand& o, int k0, uint32_t tile, int wave,
+                                                int lane) const {
+    const int k = k0 + kchunk;
+    if (!KC || !(k < o.K && o.K < k + 8)) return;
+    const int valid = o.K - k;
+#pragma unroll
+    for (int j = 0; j < kInstr; ++j) {
+      uint16_t* q = reinterpret_cast<uint16_t*>(lds + tile + (j * 4 + wave) * 1024 + lane * 16);
+      for (int e = valid; e < 8; ++e) q[e] = 0;
+    }
+  }
+  // so: byte offset of the ring slot (a multiple of 1 KB)
+  __device__ __forceinline__ bf16x8_t read(const char* lds, int blk, int ks, uint32_t so) const {
+    if (KC) {
+      const char* p = lds + ((base + so) ^ (32u * ks)) + blk * (32 * kRowBytes);
+      return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(p));
+    }
+    const char* p = lds + ((base + so) ^ (64u * blk)) + ks * (16 * kRowBytes);
+    const i16x4_t v[2] = {__builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)p),
+                          __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t*)(p + 4 * kRowBytes))};
+    return __builtin_bit_cast(bf16x8_t, v);
+  }
+};
+
+template <bool A_KC, bool B_KC, bool OUT_F32, int BM, int BN, int NS>
+__global__ __launch_bounds__(kMidThreads) void gemm_mid_kernel(GemmArgs g) {
+  constexpr int MI = BM / 64, NJ = BN / 64;         // 32-wide blocks of a wave's tile
+  constexpr int kABytes = BM * kBK * 2, kStage = kABytes + BN * kBK * 2;
+  constexpr int kPer = BM / 32 + BN / 32;           // loads per thread and K tile
+  constexpr int kStore = 4 * 32 * (32 * NJ * (OUT_F32 ? 4 : 2) + 16);
+  constexpr int kLds = NS * kStage > kStore ? NS * kStage : kStore;
+  __shared__ __attribute__((aligned(1024))) char lds[kLds];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int bid = static_cast<int>(blockIdx.x);
+  const int split = g.ksplit > 1 ? bid % g.ksplit : 0;
+  int tm, tn;
+  tile_coords(g.ksplit > 1 ? bid / g.ksplit : bid, g.tiles_m, g.tiles_n, tm, tn);
+  if (g.ncat_tn > 0 && tn >= g.ncat_tn) {  // the pair's second product
+    tn -= g.ncat_tn;
+    g.b[0] = g.b[1];
+    g.C = g.C2;
+    g.N = g.N2;
+    g.ldc = g.ldc2;
+    g.vec_store = g.vec_store2;
+  }
+  const int row0 = tm * BM, col0 = tn * BN;
+  const int wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
+  const int nk0 = g.nk[0], nk_all = nk0 + g.nk[1];
+  const int kt0 = split * g.kper, nk = min(nk_all, kt0 + g.kper);
+  const uint32_t lds0 = lds_addr(lds);
+
+  MidMap<A_KC, BM> ma0, ma1;
+  MidMap<B_KC, BN> mb0, mb1;
+  ma0.init(g.a[0], row0, wm, 0, wave, lane);
+  mb0.init(g.b[0], col0, wn, kABytes, wave, lane);
+  ma1.init(g.a[1], row0, wm, 0, wave, lane);
+  mb1.init(g.b[1], col0, wn, kABytes, wave, lane);
+  const __amdgpu_buffer_rsrc_t ra0 = make_rsrc(g.a[0]), rb0 = make_rsrc(g.b[0]);
+  const __amdgpu_buffer_rsrc_t ra1 = make_rsrc(g.a[1]), rb1 = make_rsrc(g.b[1]);
+  auto load = [&](int t) {
+    const uint32_t so = lds0 + static_cast<uint32_t>((t - kt0) % NS) * kStage;
+    if (t < nk0) {
+      ma0.issue(ra0, g.a[0], t * kBK, so, wave);
+      mb0.issue(rb0, g.b[0], t * kBK, so + kABytes, wave);
+    } else {
+      ma1.issue(ra1, g.a[1], (t - nk0) * kBK, so, wave);
+      mb1.issue(rb1, g.b[1], (t - nk0) * kBK, so + kABytes, wave);
+    }
+  };
+  f32x16_t acc[MI][NJ];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s)
+    if (kt0 + s < nk) load(kt0 + s);
+  for (int t = kt0; t < nk; ++t) {
+    // tile t has landed once only the loads of the min(NS - 2, nk - 1 - t)
+    // newer tiles are in flight (vector memory loads complete in issue order)
+    const int newer = min(NS - 2, nk - 1 - t);
+    if (newer == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (newer == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPer) : "memory");
+    else if (newer == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kPer) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * kPer) : "memory");
+    const uint32_t so = static_cast<uint32_t>((t - kt0) % NS) * kStage;
+    const bool p1 = t >= nk0;
+    const Operand& oa = p1 ? g.a[1] : g.a[0];
+    const int k0 = (p1 ? t - nk0 : t) * kBK;
+    if ((A_KC || B_KC) && k0 + kBK > oa.K && (oa.K & 7) != 0) {
+      if (A_KC) ma0.zero_straddle(lds, oa, k0, so, wave, lane);
+      if (B_KC) mb0.zero_straddle(lds, p1 ? g.b[1] : g.b[0], k0, so + kABytes, wave, lane);
+    }
+    __syncthreads();  // tile t is whole; every wave is past its reads of tile t - 1
+    if (t + NS - 1 < nk) load(t + NS - 1);
+#pragma unroll
+    for (int ks = 0; ks < kBK / 16; ++ks) {
+      bf16x8_t fa[MI], fb[NJ];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) fa[i] = ma0.read(lds, i, ks, so);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) fb[j] = mb0.read(lds, j, ks, so);
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
+    }
+  }
+  __syncthreads();  // the ring becomes the epilogue's staging
+  if (g.ksplit > 1) g.C = static_cast<float*>(g.C) + split * g.ws_stride;
+  store_tile_w<OUT_F32, NJ, MI>(g, lds, acc, row0, col0, wm, wn, wave, lane);
+}
+
 // Sum of the ksplit f32 partial tiles of a split-K GEMM, in split order (the
 // result does not depend on timing), converted to the output type.  One
 // thread per four consecutive columns of a row.
@@ -1618,6 +1794,34 @@ void launch_bf16(const GemmArgs& a, bool out_f32, hipStream_t st, bool short_m =
   }
 }
 
+// Small-tile launch (gemm_mid_kernel) of a product described for tiles of
+// MidPlan's size.
+struct MidPlan {
+  int bm = 0, bn = 0;  // 0: not used
+  int ksplit = 1, kper = 0;
+  int64_t ldw = 0, bytes = 0;  // f32 partials (ksplit > 1), as SplitPlan
+  double us = 0;               // predicted time
+};
+
+template <bool A_KC, bool B_KC, bool OUT_F32>
+void launch_mid_tile(const GemmArgs& a, const MidPlan& p, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(a.tiles_m) * a.tiles_n * a.ksplit)), block(kMidThreads);
+  if (p.bm == 64 && p.bn == 64) gemm_mid_kernel<A_KC, B_KC, OUT_F32, 64, 64, 4><<<grid, block, 0, st>>>(a);
+  else if (p.bm == 64) gemm_mid_kernel<A_KC, B_KC, OUT_F32, 64, 128, 3><<<grid, block, 0, st>>>(a);
+  else if (p.bn == 64) gemm_mid_kernel<A_KC, B_KC, OUT_F32, 128, 64, 3><<<grid, block, 0, st>>>(a);
+  else gemm_mid_kernel<A_KC, B_KC, OUT_F32, 128, 128, 2><<<grid, block, 0, st>>>(a);
+}
+
+void launch_mid(const GemmArgs& a, const MidPlan& p, bool a_kc, bool b_kc, bool out_f32, hipStream_t st) {
+#define MOC_MID(AK, BK)                                        \
+  (out_f32 ? launch_mid_tile<AK, BK, true>(a, p, st) : launch_mid_tile<AK, BK, false>(a, p, st))
+  if (a_kc && b_kc) MOC_MID(true, true);
+  else if (a_kc) MOC_MID(true, false);
+  else if (b_kc) MOC_MID(false, true);
+  else MOC_MID(false, false);
+#undef MOC_MID
+}
+
 // Returns +1 for K-contiguous, 0 for MN-contiguous, -1 if neither.
 int layout_of(int64_t s_mn, int64_t s_k, int64_t mn, int64_t k) {
   if (s_k == 1 || k <= 1) return 1;
@@ -1664,6 +1868,70 @@ F32Split plan_f32(int64_t M, int64_t N, int64_t K, int64_t K2) {
   p.ksplit = static_cast<int>((steps + best_per - 1) / best_per);
   p.ldw = (N + 3) / 4 * 4;
   p.bytes = static_cast<int64_t>(p.ksplit) * M * p.ldw * 4;
+  return p;
+}
+
+// The small-tile plan of a product [M, N] (with n2 > 0: of the pair [M, N],
+// [M, n2] side by side, never split over K), bm = 0 where the 256-wide tiles
+// are as fast or faster.  Measured on both sides (bf16, cold weights):
+//   M x N x K              256-wide plans      small tiles
+//   pair   48 x 5461 x 2048   39.1 us      64 x 64          15.6 us
+//   pair  200 x 5461 x 2048   52.1         128 x 64         25.2
+//   pair 1000 x 2736 x 1024   39.8         128 x 128        19.6
+//   pair  800 x 5461 x 2048   59.5         128 x 128        58.3
+//         48 x 2048 x 5461    20.5         64 x 64, K in 8  11.8
+//       1000 x 1024 x 5472    35.9         128 x 64, in 4   24.3
+//       1024 x 2736 x 4096    42.6         128 x 128, in 2  36.5
+//       8192 x 768 x 2048     32.0         128 x 128        33.7
+//       2048 x 2048 x 10912   95.3         128 x 128, in 2  99.5
+//       4096 x 2736 x 1024    27.6         128 x 128        33.7
+// so a product takes small tiles while its 256x256 tiles are at most 0.35 of
+// the CUs (a pair: fewer than the CUs) and hold at most 24 K tiles per CU
+// together.  Among the small tiles the least predicted time wins: a K tile
+// takes t1 us with one workgroup on a CU and t2 with two, each workgroup t0
+// more, a K split one reduction launch and its partials' bytes; the model
+// is within 10 % of the table above and of 40 shapes around it.
+MidPlan plan_mid(int64_t M, int64_t N, int nk, int64_t n2, int64_t ws_bytes) {
+  struct Tile {
+    int bm, bn;
+    double t1, t2, t0;
+  };
+  constexpr Tile kTiles[] = {{64, 64, 0.37, 0.50, 2.5}, {64, 128, 0.45, 0.71, 3.0}, {128, 64, 0.48, 0.70, 3.0},
+                             {128, 128, 0.72, 1.16, 3.0}};
+  constexpr double kReduce = 3.0, kPartRate = 7.4e6;  // us, bytes a us
+  MidPlan p;
+  const int cus = cu_count();
+  auto tiles = [](int64_t m, int64_t n, int bm, int bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
+  const int64_t big = tiles(M, N, kBM, kBN) + (n2 > 0 ? tiles(M, n2, kBM, kBN) : 0);
+  if (M < 1 || N < 1 || nk < 1 || big * nk > 24 * cus) return p;
+  if (n2 > 0 ? big >= cus : 20 * big > 7 * cus) return p;
+  const int64_t ldw = (N + 3) & ~3LL;
+  const double part_us = 2.0 * M * ldw * 4 / kPartRate;
+  double best = 0;
+  for (const Tile& t : kTiles) {
+    const int n = static_cast<int>(tiles(M, N, t.bm, t.bn) + (n2 > 0 ? tiles(M, n2, t.bm, t.bn) : 0));
+    const int ks_max = n2 > 0 ? 1 : std::min(16, std::max(1, std::min(nk / 4, 3 * cus / n)));
+    for (int ks = 1; ks <= ks_max; ++ks) {
+      const int kper = (nk + ks - 1) / ks;
+      if (kper * (ks - 1) >= nk) continue;  // the last part would be empty
+      const int64_t bytes = ks > 1 ? kFixCounterBytes + ks * M * ldw * 4 : 0;
+      if (bytes > ws_bytes) break;
+      const int full = n * ks / (2 * cus), rem = n * ks - full * 2 * cus;
+      const double two = kper * t.t2 + t.t0, one = kper * t.t1 + t.t0;
+      double cost = full * two + (rem == 0 ? 0.0 : rem <= cus ? one : two);
+      if (ks > 1) cost += kReduce + ks * part_us;
+      if (p.bm == 0 || cost < best) {
+        best = cost;
+        p.bm = t.bm;
+        p.bn = t.bn;
+        p.ksplit = ks;
+        p.kper = kper;
+        p.ldw = ldw;
+        p.bytes = bytes;
+        p.us = best;
+      }
+    }
+  }
   return p;
 }
 
@@ -1798,6 +2066,10 @@ PairSplitPlan plan_split_pair(int64_t M1, int64_t N1, int nk1, int64_t M2, int64
     }
   }
   if (pick[0] == 0) return r;
+  // the two products apart on small tiles, where both take them
+  const MidPlan mid[2] = {plan_mid(M1, N1, nk1, 0, INT64_MAX), plan_mid(M2, N2, nk2, 0, INT64_MAX)};
+  constexpr double kTileUs = 1.2;
+  if (mid[0].bm > 0 && mid[1].bm > 0 && mid[0].us + mid[1].us < best * kTileUs) return r;
   r.bytes = kFixCounterBytes;
   for (int i = 0; i < 2; ++i) {
     r.p[i].ksplit = pick[i];
@@ -1871,7 +2143,8 @@ extern "C" int64_t moc_gemm_workspace_size(int dtype, int64_t M, int64_t N, int6
   }
   if (dtype != MOC_BF16) return 0;
   const int nk = static_cast<int>((K + kBK - 1) / kBK + (K2 + kBK - 1) / kBK);
-  return std::max({plan_split(M, N, nk).bytes, plan_fix(M, N, nk).bytes, plan_fix_short(M, N, nk).bytes});
+  return std::max({plan_split(M, N, nk).bytes, plan_fix(M, N, nk).bytes, plan_fix_short(M, N, nk).bytes,
+                   plan_mid(M, N, nk, 0, INT64_MAX).bytes});
 }
 
 // MoC 2:8 compacted Down on the structured-sparse MFMA:
@@ -1977,8 +2250,7 @@ extern "C" int moc_gemm_pair(int64_t M, int64_t K, const void* A, int64_t lda, c
   if (M == 0) return MOC_OK;
   const int64_t tm = (M + kBM - 1) / kBM, tn1 = (N1 + kBN - 1) / kBN, tn2 = (N2 + kBN - 1) / kBN;
   GemmArgs a{};
-  bool pair = K > 0 && N1 > 0 && N2 > 0 && tm * (tn1 + tn2) >= cu_count() &&
-              tm * (tn1 + tn2) < (1LL << 31) && C1 != nullptr && C2 != nullptr && A != nullptr &&
+  bool pair = K > 0 && N1 > 0 && N2 > 0 && tm * (tn1 + tn2) < (1LL << 31) && C1 != nullptr && C2 != nullptr && A != nullptr &&
               W1 != nullptr && W2 != nullptr && aligned16(A) && aligned16(W1) && aligned16(W2) &&
               lda % 8 == 0 && ldw1 % 8 == 0 && ldw2 % 8 == 0 && lda >= K && ldw1 >= K && ldw2 >= K;
   if (pair) {
@@ -1989,7 +2261,11 @@ extern "C" int moc_gemm_pair(int64_t M, int64_t K, const void* A, int64_t lda, c
     };
     pair = pair && no_wrap(a.a[0]) && no_wrap(a.b[0]) && no_wrap(a.b[1]);
   }
-  if (!pair) {
+  const bool pair_ok = pair;  // one launch can take both products
+  pair = pair && tm * (tn1 + tn2) >= cu_count();
+  // small tiles: the pair's tile columns side by side, whole K
+  const MidPlan mp = pair_ok && !pair ? plan_mid(M, N1, static_cast<int>((K + kBK - 1) / kBK), N2, 0) : MidPlan();
+  if (!pair && mp.bm == 0) {
     int rc = moc_gemm_ws(MOC_BF16, M, N1, K, A, lda, 1, W1, 1, ldw1, 0, nullptr, 0, 0, nullptr, 0, 0,
                          C1, ldc1, MOC_BF16, workspace, workspace_bytes, stream);
     if (rc == MOC_OK)
@@ -2015,6 +2291,13 @@ extern "C" int moc_gemm_pair(int64_t M, int64_t K, const void* A, int64_t lda, c
   a.C2 = C2;
   a.ldc2 = ldc2;
   a.vec_store2 = (reinterpret_cast<uintptr_t>(C2) % 16 == 0 && (ldc2 * 2) % 16 == 0) ? 1 : 0;
+  if (mp.bm > 0) {
+    a.tiles_m = static_cast<int>((M + mp.bm - 1) / mp.bm);
+    a.ncat_tn = static_cast<int>((N1 + mp.bn - 1) / mp.bn);
+    a.tiles_n = a.ncat_tn + static_cast<int>((N2 + mp.bn - 1) / mp.bn);
+    launch_mid(a, mp, true, true, false, as_stream(stream));
+    return check_launch("gemm_mid_kernel (pair)");
+  }
   const dim3 grid(static_cast<unsigned>(tm * (tn1 + tn2)));
   gemm_pp_kernel<true, true, false, false, false><<<grid, dim3(kPpThreads), 0, as_stream(stream)>>>(a);
   return check_launch("gemm_pp_kernel (pair)");
@@ -2173,6 +2456,36 @@ int gemm_ws_impl(int dtype, int64_t M, int64_t N, int64_t K, const void* A, int6
     return static_cast<int64_t>(o.bytes) + 512 * o.ld + 4096 < (1LL << 32) && 512 * o.ld < (1LL << 31);
   };
   a.pp = no_wrap(a.a[0]) && no_wrap(a.b[0]) && no_wrap(a.a[1]) && no_wrap(a.b[1]);
+  // small tiles (a K split only with a workspace for its partials)
+  const MidPlan mp = a.pp ? plan_mid(M, N, a.nk[0] + a.nk[1], 0,
+                                     workspace != nullptr && aligned16(workspace) ? workspace_bytes : 0)
+                          : MidPlan();
+  if (mp.bm > 0) {
+    GemmArgs run = a;
+    run.tiles_m = static_cast<int>((M + mp.bm - 1) / mp.bm);
+    run.tiles_n = static_cast<int>((N + mp.bn - 1) / mp.bn);
+    run.ksplit = mp.ksplit;
+    run.kper = mp.ksplit > 1 ? mp.kper : a.nk[0] + a.nk[1];
+    if (mp.ksplit > 1) {
+      run.ws_stride = M * mp.ldw;
+      run.C = static_cast<char*>(workspace) + kFixCounterBytes;
+      run.ldc = mp.ldw;
+      run.vec_store = 1;
+      run.res = nullptr;
+    }
+    launch_mid(run, mp, la == 1, lb == 1, mp.ksplit > 1 || of, st);
+    const int rc = check_launch("gemm_mid_kernel");
+    if (rc != MOC_OK || mp.ksplit == 1) return rc;
+    const dim3 grid(static_cast<unsigned>((M * ((N + 3) / 4) + 255) / 256));
+    const float* parts = static_cast<const float*>(run.C);
+    if (of)
+      splitk_reduce_kernel<true><<<grid, 256, 0, st>>>(parts, run.ws_stride, mp.ksplit, (int)M, (int)N, mp.ldw, C, ldc,
+                                                       a.vec_store);
+    else
+      splitk_reduce_kernel<false><<<grid, 256, 0, st>>>(parts, run.ws_stride, mp.ksplit, (int)M, (int)N, mp.ldw, C,
+                                                        ldc, a.vec_store, a.res, a.ldres);
+    return check_launch("splitk_reduce_kernel");
+  }
   // 128-row tiles when 256 x 256 tiles would fill more than a quarter but at
   // most half of the CUs and K is short (the 130m layer's D: 96 tiles, 32 K
   // tiles): twice the tiles run whole, where 256 x 256 tiles need a two-part
