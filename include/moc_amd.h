@@ -222,6 +222,22 @@ int moc_gemm_pair(int64_t M, int64_t K, const void* A, int64_t lda, const void* 
 int64_t moc_gemm_workspace_size(int dtype, int64_t M, int64_t N, int64_t K, int64_t K2);
 
 /* ----------------------------------------------------------------- layer */
+/* Inference of one FFN layer over `rows` tokens with dense MFMA products
+ * (the >16-token form of moc/inference/inference_ffn.py:182-203): y = Z W_down
+ * (+ res, added as bf16(bf16(Z W_down) + res) when not NULL), Z the selected
+ * channels' bf16 SiLU(G) U.  selection 0: Top-K of each token's gate row;
+ * 2: top-2 of every 8 channels (inter a multiple of 8, k = inter / 4).
+ * x, y, res: rows of ldx, ldy, ldres; wg, wu [inter, d] contiguous; wdt =
+ * W_down^T [inter, d] with rows ldwdt apart; all rows 16-byte aligned.
+ * scratch: moc_ffn_infer_scratch_size bytes, no contents kept; workspace:
+ * moc_ffn_infer_workspace_size bytes as moc_gemm_ws uses it (counters zero). */
+int64_t moc_ffn_infer_scratch_size(int64_t rows, int64_t inter, int64_t k, int selection);
+int64_t moc_ffn_infer_workspace_size(int64_t rows, int64_t d, int64_t inter);
+int moc_ffn_infer_bf16(int64_t rows, int64_t d, int64_t inter, int64_t k, int selection, const void* x,
+                       int64_t ldx, const void* wg, const void* wu, const void* wdt, int64_t ldwdt,
+                       const void* res, int64_t ldres, void* y, int64_t ldy, void* scratch,
+                       int64_t scratch_bytes, void* workspace, int64_t workspace_bytes, void* stream);
+
 /* GEMM workspace bytes of moc_ffn_forward_bf16 (0: none). */
 int64_t moc_ffn_forward_workspace_size(int64_t rows, int64_t d, int64_t inter);
 

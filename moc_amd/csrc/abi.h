@@ -46,6 +46,11 @@ int launch_gate_up_2of8(const void* x, int64_t nb, int64_t hidden, const void* w
                         int64_t inter, int64_t* idx, uint16_t* sz, hipStream_t st, uint16_t* ap = nullptr,
                         int64_t ld_ap = 0, uint32_t* meta = nullptr, int64_t meta_rows = 0);
 
+// MoC 2:8: the dense Z of G's and U's rows (pitch ld, a multiple of 8, 16-byte
+// aligned; inter a multiple of 8) in G's place: z of the top 2 of every 8
+// channels, zeros for the rest (moc28.hip).
+int select28_dense(void* g, const void* u, int64_t ld, int64_t rows, int64_t inter, hipStream_t st);
+
 // f32 pair C1 = A W1^T, C2 = A W2^T as one launch (gemm.hip); 1: shapes not
 // taken (nothing launched).
 int f32_gemm_pair(int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* W1,

@@ -90,6 +90,82 @@ int ffn_forward(int dt, const char* name, int64_t rows, int64_t d, int64_t inter
 
 }  // namespace
 
+// ---------------------------------------------------------------------------
+// Inference of one MoC FFN layer for more tokens than the decode kernels take
+// (moc/inference/inference_ffn.py:169-203): G and U on the MFMA GEMM (one
+// launch), the selection, the dense Z, y = Z W_down from the module's
+// W_down^T.  From 17 tokens on a token's selected rows of W_up and W_down
+// overlap the other tokens' so much that reading both weights once, densely,
+// beats gathering rows token by token: 200 tokens of 2048 -> 5461, K 1024:
+// 214 us in the gathered Up and Down alone (245 the layer), 48 here for the layer.
+// Scratch: G and U (rows of `pitch`), the selected gate values and indices;
+// Z takes G's place.
+// ---------------------------------------------------------------------------
+namespace {
+struct InferScratch {
+  int64_t pitch, g, u, vals, idx, bytes;
+};
+InferScratch infer_scratch(int64_t rows, int64_t inter, int64_t k, int selection) {
+  auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
+  InferScratch s;
+  s.pitch = inter >= 512 ? (inter + 63) / 64 * 64 : (inter + 7) / 8 * 8;
+  s.g = 0;
+  s.u = up(rows * s.pitch * 2);
+  s.vals = 2 * s.u;
+  s.idx = s.vals + (selection == 0 ? up(rows * k * 2) : 0);
+  s.bytes = s.idx + (selection == 0 ? up(rows * k * 2) : 0);
+  return s;
+}
+}  // namespace
+
+extern "C" int64_t moc_ffn_infer_scratch_size(int64_t rows, int64_t inter, int64_t k, int selection) {
+  if (rows <= 0 || inter <= 0 || k <= 0) return 0;
+  return infer_scratch(rows, inter, k, selection).bytes;
+}
+
+extern "C" int64_t moc_ffn_infer_workspace_size(int64_t rows, int64_t d, int64_t inter) {
+  if (rows <= 0 || d <= 0 || inter <= 0) return 0;
+  return std::max(gemm_ws(rows, inter, d, 0), gemm_ws(rows, d, inter, 0));
+}
+
+extern "C" int moc_ffn_infer_bf16(int64_t rows, int64_t d, int64_t inter, int64_t k, int selection, const void* x,
+                                  int64_t ldx, const void* wg, const void* wu, const void* wdt, int64_t ldwdt,
+                                  const void* res, int64_t ldres, void* y, int64_t ldy, void* scratch,
+                                  int64_t scratch_bytes, void* workspace, int64_t workspace_bytes, void* stream) {
+  MOC_REQUIRE(rows >= 1 && d >= 8 && d % 8 == 0 && inter >= 1 && k >= 1 && k <= inter, "moc_ffn_infer_bf16: bad shape");
+  MOC_REQUIRE(selection == 0 || (selection == 2 && inter % 8 == 0 && k == effective_2of8(inter)),
+              "moc_ffn_infer_bf16: selection 0 (Top-K) or 2 (top-2 of 8, intermediate a multiple of 8)");
+  MOC_REQUIRE(inter <= 32768, "moc_ffn_infer_bf16: intermediate size above 32768");
+  MOC_REQUIRE(ld_ok(x, ldx, d) && ld_ok(wg, d, d) && ld_ok(wu, d, d) && ld_ok(wdt, ldwdt, d) && ld_ok(y, ldy, d) &&
+                  (res == nullptr || ld_ok(res, ldres, d)),
+              "moc_ffn_infer_bf16: operands need 16-byte aligned rows");
+  const InferScratch s = infer_scratch(rows, inter, k, selection);
+  MOC_REQUIRE(scratch != nullptr && moc::aligned16(scratch) && scratch_bytes >= s.bytes,
+              "moc_ffn_infer_bf16: scratch of %lld bytes required", (long long)s.bytes);
+  const int64_t need = moc_ffn_infer_workspace_size(rows, d, inter);
+  MOC_REQUIRE(workspace_bytes >= need && (need == 0 || workspace != nullptr),
+              "moc_ffn_infer_bf16: workspace of %lld bytes required", (long long)need);
+  char* base = static_cast<char*>(scratch);
+  void *g = base + s.g, *u = base + s.u, *vals = base + s.vals, *idx = base + s.idx;
+  int rc = moc_gemm_pair(rows, d, x, ldx, wg, d, inter, g, s.pitch, wu, d, inter, u, s.pitch, workspace,
+                         workspace_bytes, stream);
+  if (rc != MOC_OK) return rc;
+  if (selection == 2) {
+    rc = moc::select28_dense(g, u, s.pitch, rows, inter, moc::as_stream(stream));
+  } else {
+    rc = moc_topk_rows(MOC_BF16, g, rows, inter, s.pitch, k, 0, vals, idx, MOC_I16, nullptr, 0, stream);
+    if (rc == MOC_OK)
+      rc = moc_sparse_forward_aux(MOC_BF16, vals, idx, MOC_I16, u, s.pitch, rows, k, inter, nullptr, nullptr,
+                                  nullptr, g, s.pitch, stream);
+  }
+  if (rc != MOC_OK) return rc;
+  if (res != nullptr)
+    return moc_gemm_residual_bf16(rows, d, inter, g, s.pitch, 1, wdt, ldwdt, 1, y, ldy, res, ldres, workspace,
+                                  workspace_bytes, stream);
+  return moc_gemm_ws(MOC_BF16, rows, d, inter, g, s.pitch, 1, wdt, ldwdt, 1, 0, nullptr, 0, 0, nullptr, 0, 0, y, ldy,
+                     MOC_BF16, workspace, workspace_bytes, stream);
+}
+
 // GEMM workspace of moc_ffn_forward_bf16: the G,U pair and D = Z W_down^T.
 extern "C" int64_t moc_ffn_forward_workspace_size(int64_t rows, int64_t d, int64_t inter) {
   if (rows <= 0 || d <= 0 || inter <= 0) return 0;

@@ -440,7 +440,42 @@ __global__ __launch_bounds__(256) void pack28_kernel(const uint16_t* __restrict_
     meta[(static_cast<int64_t>(ot) * meta_rows + orow) * 2 + (wi & 1)] = words[wt][wi];
 }
 
+// One thread per (row, group of 8 channels): two 16-byte loads, the top-2
+// tournament, one 16-byte store over G (bound by the 6 bytes a channel that
+// pass through it).
+__global__ __launch_bounds__(256) void select28_dense_kernel(uint4* __restrict__ g, const uint4* __restrict__ u,
+                                                             int64_t ld8, int groups, int64_t total) {
+  const int64_t gid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (gid >= total) return;
+  const int64_t o = gid / groups * ld8 + gid % groups;
+  const uint4 ga = g[o], ua = u[o];
+  const uint32_t gw[4] = {ga.x, ga.y, ga.z, ga.w}, uw[4] = {ua.x, ua.y, ua.z, ua.w};
+  int b1, b2;
+  uint16_t s1, s2;
+  select_group_top2_bits(gw, uw, b1, b2, s1, s2);
+  uint32_t z[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const uint32_t lo = b1 == 2 * e ? s1 : b2 == 2 * e ? s2 : 0u;
+    const uint32_t hi = b1 == 2 * e + 1 ? s1 : b2 == 2 * e + 1 ? s2 : 0u;
+    z[e] = lo | (hi << 16);
+  }
+  g[o] = make_uint4(z[0], z[1], z[2], z[3]);
+}
+
 }  // namespace
+
+int select28_dense(void* g, const void* u, int64_t ld, int64_t rows, int64_t inter, hipStream_t st) {
+  MOC_REQUIRE(g != nullptr && u != nullptr && aligned16(g) && aligned16(u) && ld % 8 == 0 && inter % 8 == 0 &&
+                  ld >= inter && inter >= 8 && rows >= 0,
+              "select28_dense: 16-byte aligned rows of whole groups of 8");
+  const int64_t total = rows * (inter / 8);
+  if (total == 0) return MOC_OK;
+  MOC_REQUIRE((total + 255) / 256 < (1LL << 31), "select28_dense: too many rows");
+  select28_dense_kernel<<<dim3(static_cast<unsigned>((total + 255) / 256)), 256, 0, st>>>(
+      static_cast<uint4*>(g), static_cast<const uint4*>(u), ld / 8, static_cast<int>(inter / 8), total);
+  return check_launch("select28_dense_kernel");
+}
 }  // namespace moc
 
 using namespace moc;

@@ -204,6 +204,19 @@ class InferenceMoCSwiGLUFFN(nn.Module):
         chans = within + self._group_offset(gate_values.device)
         return vals.reshape(rows, c.k), chans.reshape(rows, c.k)
 
+    def _dense_infer_ok(self, x_2d: torch.Tensor) -> bool:
+        """K.ffn_infer takes x_2d and this module's weights as they are."""
+        return K.ffn_infer_fits(x_2d, self.gate_proj.weight, self.up_proj.weight, self._down_weight_t)
+
+    def _dense28(self, nb: int) -> bool:
+        """2:8 batches that run as dense products (K.ffn_infer) instead of the
+        packed gate/up epilogue and the structured-sparse Down, whose tiles of
+        256 tokens leave CUs idle: 2048 -> 5464 at 48 / 200 / 512 / 700 tokens
+        80 / 64 / 75 / 77 us packed, 32 / 45 / 64 / 85 dense; 1024 -> 2736 at
+        1024 / 1500 tokens 51 / 58 and 43 / 60; 512 -> 1376 at 4096 45 and 41."""
+        c = self.config
+        return nb > 16 and (nb <= 512 or nb * c.hidden_size * c.intermediate_size <= 3 << 30)
+
     # -- modes
     def dense_baseline(self, x: torch.Tensor) -> torch.Tensor:
         x_2d, shp = self._flatten_decode_input(x)
@@ -236,6 +249,9 @@ class InferenceMoCSwiGLUFFN(nn.Module):
             y = K.global_decode(x_2d, self.gate_proj.weight, self.up_proj.weight,
                                 self._down_weight_t, self.config.k,
                                 workspace=self._global_decode_workspace(x_2d.shape[0], x_2d.device))
+            return self._restore_output_shape(y, shp)
+        if x_2d.shape[0] > 16 and self._dense_infer_ok(x_2d):
+            y = K.ffn_infer(x_2d, self.gate_proj.weight, self.up_proj.weight, self._down_weight_t, self.config.k)
             return self._restore_output_shape(y, shp)
         if x_2d.shape[0] <= 16:
             gate_full = K.gemv(x_2d, self.gate_proj.weight)
@@ -318,6 +334,15 @@ class InferenceMoCSwiGLUFFN(nn.Module):
 
             def _run():
                 K.moc28_decode(x_buf, wg, wu, self._down_weight_t, workspace=ws, out=y_buf)
+        elif self._dense28(batch_size) and K.ffn_infer_fits(x_buf, wg, wu, self._down_weight_t):
+            sbytes, wbytes = K.ffn_infer_bytes(batch_size, h, inter, k, grouped=True)
+            scratch = torch.empty(sbytes, dtype=torch.uint8, device=device)
+            ws = torch.zeros(max(wbytes, 1), dtype=torch.uint8, device=device)
+            buffers = (x_buf, y_buf, scratch, ws)
+
+            def _run():
+                K.ffn_infer(x_buf, wg, wu, self._down_weight_t, k, grouped=True, out=y_buf, scratch=scratch,
+                            workspace=ws)
         elif batch_size > 64 and dtype == torch.bfloat16:
             # prefill batches: the selection travels 2:4-packed from the
             # gate/up epilogue to the structured-sparse Down
@@ -387,6 +412,10 @@ class InferenceMoCSwiGLUFFN(nn.Module):
             x_2d = x_2d.contiguous()
             y = K.moc28_decode(x_2d, self.gate_proj.weight, self.up_proj.weight, self._down_weight_t,
                                workspace=self._moc28_decode_workspace(x_2d.shape[0], x_2d.device))
+            return self._restore_output_shape(y, shp)
+        if self._dense28(x_2d.shape[0]) and self._dense_infer_ok(x_2d):
+            y = K.ffn_infer(x_2d, self.gate_proj.weight, self.up_proj.weight, self._down_weight_t, c.k,
+                            grouped=True)
             return self._restore_output_shape(y, shp)
         if x_2d.shape[0] > 64 and x_2d.dtype == torch.bfloat16:
             # prefill: the gate/up epilogue writes the selection 2:4-packed and

@@ -663,13 +663,13 @@ def global_after_gate(x, gate_scores, up_weight, down_weight_t, k: int, *, works
         raise ValueError(f"idx_out must be a contiguous int32 [{nb}, {int(k)}] tensor")
     if nb > 16:
         # more tokens than the fused kernel takes: the same steps as separate
-        # launches (row Top-K, selected Up * SiLU, selected Down), like the
-        # reference's op, which accepts any batch (optimized_global_moc_ext.cu:457-540)
+        # launches, like the reference's op, which accepts any batch
+        # (optimized_global_moc_ext.cu:457-540).  U and Down as dense products:
+        # the tokens' selections overlap (see moc_ffn_infer_bf16)
         vals, idx, _ = topk_rows(g, int(k), idx_dtype=torch.int32)
-        z = selected_up_silu(x, vals, idx, wu)
-        yy = selected_down(z, idx, wdt)
-        if residual is not None:
-            yy = residual.reshape(yy.shape) + yy
+        u = linear(x, wu, out=padded_empty(nb, inter, torch.bfloat16, x.device))
+        z = sparse_forward_aux(vals, idx, u, inter, want_s=False, want_z=False)[3]
+        yy = gemm(z, wdt, residual=None if residual is None else residual.reshape(nb, hidden))
         if idx_out is not None:
             idx_out.copy_(idx)
         if out is None:
@@ -765,6 +765,60 @@ def global_decode_rmsnorm_residual(x, norm_weight, eps: float, gate_weight, up_w
 def global_decode_rmsnorm_residual_fits(nb: int, inter: int, k: int, hidden: int) -> bool:
     """Shapes moc_global_decode_rmsnorm_residual_bf16 takes."""
     return 1 <= nb <= 4 and hidden % 256 == 0 and hidden <= 4096 and inter <= 8192 and int(k) <= 4096
+
+
+# ------------------------------------------- inference, more than 16 tokens
+def ffn_infer_fits(x2d: torch.Tensor, gate_weight, up_weight, down_weight_t) -> bool:
+    """Operands moc_ffn_infer_bf16 takes as they are: bf16, contiguous gate and
+    up weights, 16-byte aligned rows."""
+    nb, hidden = x2d.shape
+    inter = gate_weight.shape[0]
+    return (x2d.is_cuda and nb >= 1 and hidden % 8 == 0 and inter <= 16384
+            and x2d.dtype == gate_weight.dtype == up_weight.dtype == down_weight_t.dtype == torch.bfloat16
+            and gate_weight.shape == up_weight.shape == down_weight_t.shape == (inter, hidden)
+            and gate_weight.is_contiguous() and up_weight.is_contiguous()
+            and x2d.stride(1) == 1 and (nb == 1 or (x2d.stride(0) % 8 == 0 and x2d.stride(0) >= hidden))
+            and down_weight_t.stride(1) == 1 and down_weight_t.stride(0) % 8 == 0
+            and down_weight_t.stride(0) >= hidden
+            and all(t.data_ptr() % 16 == 0 for t in (x2d, gate_weight, up_weight, down_weight_t)))
+
+
+def ffn_infer_bytes(nb: int, hidden: int, inter: int, k: int, grouped: bool = False) -> tuple[int, int]:
+    """Bytes of ffn_infer's scratch and of its workspace."""
+    k = moc28_effective_k(inter) if grouped else int(k)
+    return (N.query("moc_ffn_infer_scratch_size", nb, inter, k, 2 if grouped else 0),
+            N.query("moc_ffn_infer_workspace_size", nb, hidden, inter))
+
+
+def ffn_infer(x2d, gate_weight, up_weight, down_weight_t, k: int, *, grouped: bool = False,
+              residual: torch.Tensor | None = None, out: torch.Tensor | None = None,
+              scratch: torch.Tensor | None = None, workspace: torch.Tensor | None = None) -> torch.Tensor:
+    """One MoC FFN layer over many tokens with dense MFMA products
+    (moc_ffn_infer_bf16): global Top-K, or with `grouped` the top 2 of every 8
+    channels; with `residual`, residual + that.  ffn_infer_fits must hold.
+    `scratch` and `workspace` (zeroed before its first use): buffers of
+    ffn_infer_bytes() kept by the caller."""
+    N.require_device(x2d, gate_weight, up_weight, down_weight_t, residual)
+    nb, hidden = x2d.shape
+    inter = gate_weight.shape[0]
+    k = moc28_effective_k(inter) if grouped else int(k)
+    sel = 2 if grouped else 0
+    dev = x2d.device
+    r = None if residual is None else aligned_rows(residual.reshape(nb, hidden))
+    y = _empty((nb, hidden), torch.bfloat16, dev) if out is None else out
+    if y.shape != (nb, hidden) or y.dtype != torch.bfloat16 or not y.is_contiguous():
+        raise ValueError(f"out must be a contiguous bf16 [{nb}, {hidden}] tensor")
+    sbytes, wbytes = ffn_infer_bytes(nb, hidden, inter, k, grouped)
+    scratch = _empty((sbytes,), torch.uint8, dev) if scratch is None else scratch
+    ws = workspace if workspace is not None else _gemm_workspace(dev, wbytes) if wbytes > 0 else None
+    if scratch.numel() < sbytes or (ws is not None and ws.numel() < wbytes):
+        raise ValueError(f"ffn_infer needs {sbytes} bytes of scratch and a workspace of {wbytes}")
+    ld = lambda t: t.stride(0) if nb > 1 else hidden  # noqa: E731
+    N.call("moc_ffn_infer_bf16", nb, hidden, inter, k, sel, x2d.data_ptr(), ld(x2d), gate_weight.data_ptr(),
+           up_weight.data_ptr(), down_weight_t.data_ptr(), down_weight_t.stride(0), N.ptr(r),
+           0 if r is None else ld(r), y.data_ptr(), hidden, scratch.data_ptr(), sbytes, N.ptr(ws), wbytes,
+           N.stream_of(x2d))
+    return y
 
 
 # ----------------------------------------------------------------------- 2:8

@@ -1,0 +1,100 @@
+"""The dense many-token inference layer (K.ffn_infer and the module routes that
+take it) against 64-bit arithmetic on inputs whose gate scores are exact."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from moc_amd import kernels as K
+from moc_amd.inference.inference_ffn import InferenceMoCSwiGLUFFN
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+def _case(nb, hidden, inter, seed):
+    """x in {-1, 0, 1}, weights in {-2 .. 2} / 128: every gate and up sum is
+    exact in f32 and in bf16, so the selection has one right answer."""
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    ri = lambda lo, hi, s: torch.randint(lo, hi + 1, s, generator=gen, device="cuda")  # noqa: E731
+    x = ri(-1, 1, (nb, hidden)).to(BF)
+    w = [(ri(-2, 2, s).float() / 128).to(BF) for s in ((inter, hidden), (inter, hidden), (hidden, inter))]
+    return x, w
+
+
+def _reference(x, w, k, grouped):
+    wg, wu, wd = (t.double() for t in w)
+    g, u = x.double() @ wg.t(), x.double() @ wu.t()
+    nb, inter = g.shape
+    if grouped:
+        order = torch.sort(g.reshape(nb, -1, 8), dim=-1, descending=True, stable=True).indices[..., :2]
+        mask = torch.zeros(nb, inter // 8, 8, device=g.device).scatter_(-1, order, 1.0).reshape(nb, inter)
+        z = (F.silu(g) * u).to(BF).double()  # rounded once
+    else:
+        order = torch.sort(g, dim=-1, descending=True, stable=True).indices[:, :k]
+        mask = torch.zeros_like(g).scatter_(-1, order, 1.0)
+        z = (F.silu(g).to(BF).double() * u).to(BF).double()
+    z = z * mask
+    return z @ wd.t(), z.abs() @ wd.abs().t()
+
+
+def _check(y, ref, mags, inter, extra=0.0):
+    # one bf16 rounding of y; z may round the other way where f32 SiLU differs
+    # from the 64-bit one (half an ulp of z at most, on few channels)
+    bound = 2.0 ** -8 * (ref.abs() + extra) + (2.0 ** -9 + inter * 2.0 ** -24) * mags + 1e-30
+    assert ((y.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("nb,hidden,inter,k", [(17, 64, 200, 1), (64, 128, 333, 100), (65, 256, 1000, 1000),
+                                               (200, 512, 1376, 256), (300, 192, 5461, 1024)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_global(nb, hidden, inter, k, residual):
+    x, w = _case(nb, hidden, inter, nb + inter)
+    wdt = K.down_weight_t_for_decode(w[2])
+    ref, mags = _reference(x, w, k, False)
+    res = torch.randn(nb, hidden, device="cuda").to(BF) if residual else None
+    assert K.ffn_infer_fits(x, w[0], w[1], wdt)
+    y = K.ffn_infer(x, w[0], w[1], wdt, k, residual=res)
+    if residual:
+        _check(y, ref + res.double(), mags, inter, extra=ref.abs())
+    else:
+        _check(y, ref, mags, inter)
+        m = InferenceMoCSwiGLUFFN(hidden, inter, k).to("cuda", BF)
+        for p, t in zip((m.gate_proj, m.up_proj, m.down_proj), w):
+            p.weight.data.copy_(t)
+        assert torch.equal(m(x), y)
+        # the gate-given operator: the same steps from the gate scores
+        g = K.linear(x, w[0])
+        _check(K.global_after_gate(x, g, w[1], wdt, k), ref, mags, inter)
+
+
+@pytest.mark.parametrize("nb,hidden,inter", [(17, 64, 8), (33, 128, 200), (64, 256, 1000), (513, 64, 1376),
+                                             (200, 512, 2736)])
+def test_28(nb, hidden, inter):
+    x, w = _case(nb, hidden, inter, nb + inter)
+    wdt = K.down_weight_t_for_decode(w[2])
+    ref, mags = _reference(x, w, 0, True)
+    y = K.ffn_infer(x, w[0], w[1], wdt, 0, grouped=True)
+    _check(y, ref, mags, inter)
+    m = InferenceMoCSwiGLUFFN(hidden, inter, inter // 4, grouped_a=2, grouped_b=8).to("cuda", BF)
+    for p, t in zip((m.gate_proj, m.up_proj, m.down_proj), w):
+        p.weight.data.copy_(t)
+    assert torch.equal(m(x), y)
+    run = m.make_moc2_8_graph_runner(nb)
+    for s in range(3):  # replays with eager work between them
+        xs = x.roll(s, 0).contiguous()
+        got = run(xs).clone()
+        assert torch.equal(got, m(xs))
+
+
+def test_28_nan_rows_and_ties():
+    """NaN gates rank first and equal ones go to the lower channel, as in the
+    packed path; other tokens' rows are untouched by a NaN token."""
+    x, w = _case(20, 64, 64, 1)
+    x[3] = float("nan")
+    x[5] = 0  # all gates equal: channels 0 and 1 of each group
+    wdt = K.down_weight_t_for_decode(w[2])
+    y = K.ffn_infer(x, w[0], w[1], wdt, 0, grouped=True)
+    assert torch.isnan(y[3]).all() and (y[5] == 0).all()
+    ref, mags = _reference(torch.nan_to_num(x), w, 0, True)
+    keep = [i for i in range(20) if i != 3]
+    _check(y[keep], ref[keep], mags[keep], 64)
