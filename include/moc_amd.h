@@ -436,6 +436,22 @@ int moc_global_decode_bf16(const void* x, int64_t nb, int64_t hidden, const void
                            int64_t k, void* y, void* idx_out, void* workspace, int64_t workspace_bytes,
                            void* stream);
 
+/* The attention half of a decoder layer for one token
+ * (benchmarks/inference/benchmark_decode.py:128-303): y = x + out_proj(
+ * attention(RoPE(qkv_proj(RMSNorm(x))))) against a KV cache that the call
+ * extends at position *pos (a device int64; outside [0, max_seq) the cache is
+ * left alone and y is NaN).  x, y [hidden]; w_qkv [3 hidden, hidden] (rows of
+ * q, then k, then v, each by head), w_out [hidden, hidden]; cos, sin
+ * [max_seq, head_dim / 2] bf16, RoPE on pairs (2i, 2i + 1); k_t [heads,
+ * head_dim, max_seq], v [heads, max_seq, head_dim]; scale multiplies q k.
+ * workspace: moc_decode_attention_workspace_size(hidden) bytes, no contents
+ * kept. */
+int64_t moc_decode_attention_workspace_size(int64_t hidden);
+int moc_decode_attention_bf16(const void* x, int64_t hidden, int64_t heads, const void* norm_w, float eps,
+                              const void* w_qkv, const void* w_out, const void* cos, const void* sin,
+                              const int64_t* pos, int64_t max_seq, void* k_t, void* v, float scale, void* y,
+                              void* workspace, int64_t workspace_bytes, void* stream);
+
 /* The decoder layer's FFN half y = bf16(x + bf16(FFN(RMSNorm(x)))) for nb <= 4
  * tokens (benchmark_decode.py:101-109,303): the norm (rounding as in
  * moc_gemv_rmsnorm_bf16) inside the gate/up GEMV pair, the residual added in

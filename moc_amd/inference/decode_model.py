@@ -17,8 +17,10 @@ replayed per token: benchmark_decode.py:549-617).  The reference's
 torch.compile scope (:423-459) is not offered: Inductor would generate
 Triton kernels for the host's attention, which this build does not use.
 
-Attention, RMSNorm, RoPE, the embedding and the LM head are stock PyTorch
-(the host of the FFN).  Attention keeps K transposed in its cache
+A single-token step runs each layer's attention half (norm, q/k/v, RoPE,
+cache, attention, out_proj, residual) as three kernels and the final norm
+inside the LM head's GEMV (one bf16 token, no gradients or hooks; else stock
+PyTorch, as for the prompt).  Attention keeps K transposed in its cache
 ([1, heads, head_dim, max_seq]) and V as [1, heads, max_seq, head_dim], so
 both attention products are batched products of contiguous operands; the
 softmax runs in f32.
@@ -33,6 +35,7 @@ from typing import Callable
 import torch
 import torch.nn as nn
 
+from .. import kernels as K
 from .inference_ffn import InferenceMoCSwiGLUFFN
 
 HIDDEN = 2048
@@ -149,6 +152,26 @@ class StaticKVAttention(nn.Module):
         return self.out_proj(y.transpose(1, 2).reshape(b, 1, h))
 
 
+def _plain(*modules) -> bool:
+    """No forward hooks, and the linears plain bias-free nn.Linear: what a
+    fused step computes from the weights alone."""
+    for m in modules:
+        if m._forward_hooks or m._forward_pre_hooks:
+            return False
+        if isinstance(m, nn.Linear) and (type(m) is not nn.Linear or m.bias is not None):
+            return False
+    return True
+
+
+def _one_token_native(x: torch.Tensor, *weights) -> bool:
+    """One bf16 token of a gradient-free pass outside autocast, with
+    contiguous, aligned bf16 weights on its device."""
+    return (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[:2] == (1, 1) and not torch.is_grad_enabled()
+            and not torch.is_autocast_enabled("cuda")
+            and all(w.dtype == torch.bfloat16 and w.device == x.device and w.is_contiguous()
+                    and w.data_ptr() % 16 == 0 for w in weights))
+
+
 class DecoderLayer(nn.Module):
     def __init__(self, row: str, cfg: DecodeConfig, fuse: bool = True):
         super().__init__()
@@ -156,6 +179,9 @@ class DecoderLayer(nn.Module):
         # MoC decode: ffn_norm and the residual add run inside the FFN's two
         # kernels (InferenceMoCSwiGLUFFN.fused_decode_residual)
         self.fuse = fuse and row in ("global_moc", "moc_2_8")
+        # one token: the norm, q/k/v, RoPE, the cache update, attention, out_proj
+        # and the residual add as three kernels (K.decode_attention)
+        self.fuse_attn = True
         grouped = row == "moc_2_8"
         k = cfg.intermediate * 2 // 8 if grouped else cfg.k
         self.attn_norm = RMSNorm(cfg.hidden)
@@ -173,8 +199,22 @@ class DecoderLayer(nn.Module):
         x = x + self.attn.forward_prompt(self.attn_norm(x))
         return x + self._ffn(self.ffn_norm(x))
 
+    def _attn_native(self, x: torch.Tensor) -> bool:
+        a, n = self.attn, self.attn_norm
+        return (self.fuse_attn and type(a) is StaticKVAttention and type(n) is RMSNorm
+                and _plain(a, n, a.qkv_proj, a.out_proj) and a.k_t is not None and a.k_t.shape[0] == 1
+                and _one_token_native(x, n.weight, a.qkv_proj.weight, a.out_proj.weight, a.rope_cos, a.rope_sin,
+                                      a.k_t, a.v)
+                and K.decode_attention_fits(a.hidden, a.heads, a.max_seq))
+
     def forward_step(self, x: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
-        x = x + self.attn.forward_step(self.attn_norm(x), pos)
+        if self._attn_native(x):
+            a = self.attn
+            x = K.decode_attention(x.reshape(1, -1).contiguous(), self.attn_norm.weight, self.attn_norm.eps,
+                                   a.qkv_proj.weight, a.out_proj.weight, a.rope_cos, a.rope_sin, pos, a.k_t[0],
+                                   a.v[0], 1.0 / math.sqrt(a.head_dim)).reshape(x.shape)
+        else:
+            x = x + self.attn.forward_step(self.attn_norm(x), pos)
         if self.fuse and x.is_cuda:
             b, n, h = x.shape
             return self.ffn.fused_decode_residual(x.reshape(b * n, h), self.ffn_norm.weight,
@@ -188,6 +228,7 @@ class DecoderModel(nn.Module):
         if row not in ROWS:
             raise ValueError(f"unknown decode row {row!r}; expected one of {sorted(ROWS)}")
         self.row, self.cfg = row, cfg
+        self.fuse_head = True  # one token: the final norm inside the LM head's GEMV
         self.embed = nn.Embedding(cfg.vocab, cfg.hidden)
         self.layers = nn.ModuleList(DecoderLayer(row, cfg, fuse) for _ in range(cfg.layers))
         self.final_norm = RMSNorm(cfg.hidden)
@@ -227,7 +268,11 @@ class DecoderModel(nn.Module):
         x = self.embed(tokens)
         for layer in self.layers:
             x = layer.forward_step(x, pos)
-        return self.lm_head(self.final_norm(x))
+        n, head = self.final_norm, self.lm_head
+        if (self.fuse_head and type(n) is RMSNorm and _plain(n, head) and self.cfg.hidden % 8 == 0
+                and self.cfg.hidden <= 4096 and _one_token_native(x, n.weight, head.weight)):
+            return K.gemv_rmsnorm(x.reshape(1, -1), n.weight, n.eps, head.weight)[0][None]
+        return head(n(x))
 
 
 def make_step(model: DecoderModel, scope: str) -> Callable[[torch.Tensor, int], torch.Tensor]:

@@ -767,6 +767,37 @@ def global_decode_rmsnorm_residual_fits(nb: int, inter: int, k: int, hidden: int
     return 1 <= nb <= 4 and hidden % 256 == 0 and hidden <= 4096 and inter <= 8192 and int(k) <= 4096
 
 
+def decode_attention(x, norm_weight, eps: float, qkv_weight, out_weight, cos, sin, pos, k_t, v,
+                     scale: float) -> torch.Tensor:
+    """x + out_proj(attention(RoPE(qkv_proj(RMSNorm(x))))) of one token x
+    [1, hidden] at position `pos` (0-dim device int64), the caches k_t [heads,
+    head_dim, max_seq] and v [heads, max_seq, head_dim] extended in place
+    (moc_decode_attention_bf16)."""
+    ts = (x, norm_weight, qkv_weight, out_weight, cos, sin, k_t, v)
+    N.require_device(*ts, pos)
+    heads, head_dim, max_seq = k_t.shape
+    hidden = heads * head_dim
+    if any(t.dtype != torch.bfloat16 or not t.is_contiguous() for t in ts) or pos.dtype != torch.int64:
+        raise ValueError("decode_attention takes contiguous bf16 tensors and an int64 position")
+    if (x.shape != (1, hidden) or norm_weight.shape != (hidden,) or qkv_weight.shape != (3 * hidden, hidden)
+            or out_weight.shape != (hidden, hidden) or v.shape != (heads, max_seq, head_dim)
+            or cos.shape != (max_seq, head_dim // 2) or sin.shape != cos.shape or pos.numel() != 1):
+        raise ValueError("decode_attention shape mismatch")
+    y = torch.empty_like(x)
+    nbytes = N.query("moc_decode_attention_workspace_size", hidden)
+    ws = _empty((nbytes,), torch.uint8, x.device)
+    N.call("moc_decode_attention_bf16", x.data_ptr(), hidden, heads, norm_weight.data_ptr(), float(eps),
+           qkv_weight.data_ptr(), out_weight.data_ptr(), cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), max_seq,
+           k_t.data_ptr(), v.data_ptr(), float(scale), y.data_ptr(), ws.data_ptr(), nbytes, N.stream_of(x))
+    return y
+
+
+def decode_attention_fits(hidden: int, heads: int, max_seq: int) -> bool:
+    """Shapes moc_decode_attention_bf16 takes."""
+    return (hidden <= 4096 and heads >= 1 and hidden % heads == 0 and (hidden // heads) % 8 == 0
+            and hidden // heads <= 256 and 1 <= max_seq <= 8192)
+
+
 # ------------------------------------------- inference, more than 16 tokens
 def ffn_infer_fits(x2d: torch.Tensor, gate_weight, up_weight, down_weight_t) -> bool:
     """Operands moc_ffn_infer_bf16 takes as they are: bf16, contiguous gate and
