@@ -361,20 +361,14 @@ __global__ __launch_bounds__(256) void gemv16_kernel(const uint16_t* __restrict_
 // products and a wave reduction.  With ~one row per wave every byte of W is
 // in flight within one memory latency.
 // ---------------------------------------------------------------------------
-// NORM: the tokens go through RMSNorm first (the FFN's pre-norm,
-// benchmark_decode.py:101-109,303): xn = bf16(bf16(x * r) * w) with
-// r = 1 / sqrt(mean(x^2) + eps) in f32; every wave normalises its own copy
-// of x, and wave 0 of workgroup 0 also writes xn for the kernels after it.
 // Pair form (W2 != nullptr): the waves from row2_start on (a workgroup
 // boundary) take the rows of a second matrix W2 [rows2, hidden] into y2 (two
 // projections of the same tokens in one launch).
-template <int NB, int CHN, bool NORM>
+template <int NB, int CHN>
 __global__ __launch_bounds__(256) void gemv_rows_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                         const uint16_t* __restrict__ W, int64_t ldw,
                                                         int rows, int hidden,
                                                         uint16_t* __restrict__ y, int64_t ldy,
-                                                        const uint16_t* __restrict__ norm_w, float eps,
-                                                        uint16_t* __restrict__ xn, int64_t ldxn,
                                                         const uint16_t* __restrict__ W2, int64_t ldw2,
                                                         int row2_start, int rows2, uint16_t* __restrict__ y2,
                                                         int64_t ldy2) {
@@ -397,14 +391,6 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(const uint16_t* __restri
     wv[i] = c < nch ? *reinterpret_cast<const uint4*>(W + static_cast<int64_t>(row) * ldw + c * 8)
                     : make_uint4(0, 0, 0, 0);
   }
-  uint4 nwv[NORM ? CHN : 1];  // norm weight chunks, requested with the row
-  if (NORM) {
-#pragma unroll
-    for (int i = 0; i < CHN; ++i) {
-      const int c = lane + 64 * i;
-      nwv[i] = c < nch ? *reinterpret_cast<const uint4*>(norm_w + c * 8) : make_uint4(0, 0, 0, 0);
-    }
-  }
   float acc[NB];
 #pragma unroll
   for (int t = 0; t < NB; ++t) {
@@ -415,33 +401,94 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(const uint16_t* __restri
       const int c = lane + 64 * i;
       xv[i] = c < nch ? *reinterpret_cast<const uint4*>(x + t * ldx + c * 8) : make_uint4(0, 0, 0, 0);
     }
-    if (NORM) {
-      float ss = 0.f;
-#pragma unroll
-      for (int i = 0; i < CHN; ++i) {
-        const uint32_t a[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float lo = __uint_as_float(a[j] << 16), hi = __uint_as_float(a[j] & 0xFFFF0000u);
-          ss = fmaf(lo, lo, ss);
-          ss = fmaf(hi, hi, ss);
-        }
-      }
-      const float r = rsqrtf(wave_sum(ss) / static_cast<float>(hidden) + eps);
-#pragma unroll
-      for (int i = 0; i < CHN; ++i) {
-        const int c = lane + 64 * i;
-        xv[i] = rmsnorm8(xv[i], nwv[NORM ? i : 0], r);
-        if (blockIdx.x == 0 && threadIdx.x < 64 && c < nch)
-          *reinterpret_cast<uint4*>(xn + t * ldxn + c * 8) = xv[i];
-      }
-    }
 #pragma unroll
     for (int i = 0; i < CHN; ++i) acc[t] = dot8(wv[i], xv[i], acc[t]);
   }
 #pragma unroll
   for (int t = 0; t < NB; ++t) {
     const float tot = wave_sum(acc[t]);
+    if (lane == 0) y[t * ldy + row] = f32_to_bf16(tot);
+  }
+}
+
+// The same with the tokens going through RMSNorm first (the FFN's pre-norm,
+// benchmark_decode.py:101-109,303): xn = bf16(bf16(x * r) * w) with
+// r = 1 / sqrt(mean(x^2) + eps) in f32.  The workgroup's WAVES waves request
+// their rows, then normalise the tokens together into LDS and read xn from
+// there; workgroup 0 also writes xn for the kernels after it.  A wave that
+// normalises the tokens for itself spends more VALU time on that than its
+// row's bytes take: one token, gate and up of 2048 -> 5461 (44.7 MB from HBM)
+// 14.1 -> 9.9 us, a 32000 x 2048 LM head 32.5 -> 22.1 us.
+constexpr int kGnWaves = 8;
+template <int NB, int CHN>
+__global__ __launch_bounds__(64 * kGnWaves) void gemv_norm_rows_kernel(
+    const uint16_t* __restrict__ x, int64_t ldx, const uint16_t* __restrict__ W, int64_t ldw, int rows, int hidden,
+    uint16_t* __restrict__ y, int64_t ldy, const uint16_t* __restrict__ norm_w, float eps,
+    uint16_t* __restrict__ xn, int64_t ldxn, const uint16_t* __restrict__ W2, int64_t ldw2, int row2_start,
+    int rows2, uint16_t* __restrict__ y2, int64_t ldy2) {
+  __shared__ uint4 xs[NB][64 * CHN];
+  __shared__ float red[NB][kGnWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int row = blockIdx.x * kGnWaves + wave;
+  if (W2 != nullptr && row >= row2_start) {
+    row -= row2_start;
+    rows = rows2;
+    W = W2;
+    ldw = ldw2;
+    y = y2;
+    ldy = ldy2;
+  }
+  const int nch = hidden / 8;
+  const bool live = row < rows;
+  uint4 wv[CHN];
+#pragma unroll
+  for (int i = 0; i < CHN; ++i) {
+    const int c = lane + 64 * i;
+    wv[i] = live && c < nch ? *reinterpret_cast<const uint4*>(W + static_cast<int64_t>(row) * ldw + c * 8)
+                            : make_uint4(0, 0, 0, 0);
+  }
+  // thread tid: chunk tid of every token (hidden <= 4096: one chunk each)
+  const uint4 nw = tid < nch ? *reinterpret_cast<const uint4*>(norm_w + tid * 8) : make_uint4(0, 0, 0, 0);
+  uint4 xv[NB];
+#pragma unroll
+  for (int t = 0; t < NB; ++t)
+    xv[t] = tid < nch ? *reinterpret_cast<const uint4*>(x + t * ldx + tid * 8) : make_uint4(0, 0, 0, 0);
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    const uint32_t a[4] = {xv[t].x, xv[t].y, xv[t].z, xv[t].w};
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float lo = __uint_as_float(a[j] << 16), hi = __uint_as_float(a[j] & 0xFFFF0000u);
+      ss = fmaf(lo, lo, ss);
+      ss = fmaf(hi, hi, ss);
+    }
+    ss = wave_sum(ss);
+    if (lane == 0) red[t][wave] = ss;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    float ss = 0.f;
+#pragma unroll
+    for (int w = 0; w < kGnWaves; ++w) ss += red[t][w];
+    const uint4 n = rmsnorm8(xv[t], nw, rsqrtf(ss / static_cast<float>(hidden) + eps));
+    if (tid < nch) {
+      xs[t][tid] = n;
+      if (blockIdx.x == 0) *reinterpret_cast<uint4*>(xn + t * ldxn + tid * 8) = n;
+    }
+  }
+  __syncthreads();
+  if (!live) return;
+#pragma unroll
+  for (int t = 0; t < NB; ++t) {
+    float acc = 0.f;
+#pragma unroll
+    for (int i = 0; i < CHN; ++i) {
+      const int c = lane + 64 * i;
+      acc = dot8(wv[i], c < nch ? xs[t][c] : make_uint4(0, 0, 0, 0), acc);
+    }
+    const float tot = wave_sum(acc);
     if (lane == 0) y[t * ldy + row] = f32_to_bf16(tot);
   }
 }
@@ -508,26 +555,58 @@ void launch_gemv_dual_rows(const void* x, int64_t ldx, const void* W, const void
 #undef MOC_GD
 }
 
-template <int NB, bool NORM = false>
+template <int NB>
 void launch_gemv_rows(const void* x, int64_t ldx, const void* W, int64_t ldw, int rows, int hidden,
-                      void* y, int64_t ldy, hipStream_t st, const void* norm_w = nullptr,
-                      float eps = 0.f, void* xn = nullptr, int64_t ldxn = 0, const void* W2 = nullptr,
+                      void* y, int64_t ldy, hipStream_t st, const void* W2 = nullptr,
                       int64_t ldw2 = 0, int rows2 = 0, void* y2 = nullptr, int64_t ldy2 = 0) {
   // the pair's second row range starts at a workgroup boundary
   const int wg1 = (rows + 3) / 4, wg2 = W2 != nullptr ? (rows2 + 3) / 4 : 0;
   const dim3 grid(static_cast<unsigned>(wg1 + wg2)), block(256);
   const int chn = (hidden / 8 + 63) / 64;
 #define MOC_GR(C)                                                                                  \
-  gemv_rows_kernel<NB, C, NORM><<<grid, block, 0, st>>>((const uint16_t*)x, ldx, (const uint16_t*)W, \
-                                                         ldw, rows, hidden, (uint16_t*)y, ldy,       \
-                                                         (const uint16_t*)norm_w, eps, (uint16_t*)xn, ldxn, \
-                                                         (const uint16_t*)W2, ldw2, wg1 * 4, rows2, (uint16_t*)y2, \
-                                                         ldy2)
+  gemv_rows_kernel<NB, C><<<grid, block, 0, st>>>((const uint16_t*)x, ldx, (const uint16_t*)W,       \
+                                                  ldw, rows, hidden, (uint16_t*)y, ldy,              \
+                                                  (const uint16_t*)W2, ldw2, wg1 * 4, rows2, (uint16_t*)y2, ldy2)
   if (chn <= 1) MOC_GR(1);
   else if (chn <= 2) MOC_GR(2);
   else if (chn <= 4) MOC_GR(4);
   else MOC_GR(8);
 #undef MOC_GR
+}
+
+template <int NB>
+void launch_gemv_norm_rows(const void* x, int64_t ldx, const void* W, int64_t ldw, int rows, int hidden,
+                           void* y, int64_t ldy, hipStream_t st, const void* norm_w, float eps, void* xn,
+                           int64_t ldxn, const void* W2, int64_t ldw2, int rows2, void* y2, int64_t ldy2) {
+  const int wg1 = (rows + kGnWaves - 1) / kGnWaves, wg2 = W2 != nullptr ? (rows2 + kGnWaves - 1) / kGnWaves : 0;
+  const dim3 grid(static_cast<unsigned>(wg1 + wg2)), block(64 * kGnWaves);
+  const int chn = (hidden / 8 + 63) / 64;
+#define MOC_GN(C)                                                                                           \
+  gemv_norm_rows_kernel<NB, C><<<grid, block, 0, st>>>((const uint16_t*)x, ldx, (const uint16_t*)W, ldw, rows, \
+                                                       hidden, (uint16_t*)y, ldy, (const uint16_t*)norm_w, eps, \
+                                                       (uint16_t*)xn, ldxn, (const uint16_t*)W2, ldw2,          \
+                                                       wg1 * kGnWaves, rows2, (uint16_t*)y2, ldy2)
+  if (chn <= 1) MOC_GN(1);
+  else if (chn <= 2) MOC_GN(2);
+  else if (chn <= 4) MOC_GN(4);
+  else MOC_GN(8);
+#undef MOC_GN
+}
+
+// nb <= 4 tokens, hidden <= 4096 (checked by the callers)
+void gemv_norm_rows(int64_t nb, const void* x, int64_t ldx, const void* W, int64_t ldw, int rows, int hidden,
+                    void* y, int64_t ldy, hipStream_t st, const void* norm_w, float eps, void* xn, int64_t ldxn,
+                    const void* W2 = nullptr, int64_t ldw2 = 0, int rows2 = 0, void* y2 = nullptr,
+                    int64_t ldy2 = 0) {
+#define MOC_GNB(N) \
+  launch_gemv_norm_rows<N>(x, ldx, W, ldw, rows, hidden, y, ldy, st, norm_w, eps, xn, ldxn, W2, ldw2, rows2, y2, ldy2)
+  switch (nb) {
+    case 1: MOC_GNB(1); break;
+    case 2: MOC_GNB(2); break;
+    case 3: MOC_GNB(3); break;
+    default: MOC_GNB(4); break;
+  }
+#undef MOC_GNB
 }
 
 // ---------------------------------------------------------------------------
@@ -1170,10 +1249,10 @@ int gemv_launch(const void* x, int64_t ldx, int64_t nb, const void* W, int64_t l
                 int64_t ldy2, hipStream_t st) {
   if (nb <= 4 && hidden <= 4096) {
     switch (nb) {
-      case 1: launch_gemv_rows<1>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, nullptr, 0.f, nullptr, 0, W2, ldw2, (int)rows2, y2, ldy2); break;
-      case 2: launch_gemv_rows<2>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, nullptr, 0.f, nullptr, 0, W2, ldw2, (int)rows2, y2, ldy2); break;
-      case 3: launch_gemv_rows<3>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, nullptr, 0.f, nullptr, 0, W2, ldw2, (int)rows2, y2, ldy2); break;
-      default: launch_gemv_rows<4>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, nullptr, 0.f, nullptr, 0, W2, ldw2, (int)rows2, y2, ldy2); break;
+      case 1: launch_gemv_rows<1>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, W2, ldw2, (int)rows2, y2, ldy2); break;
+      case 2: launch_gemv_rows<2>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, W2, ldw2, (int)rows2, y2, ldy2); break;
+      case 3: launch_gemv_rows<3>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, W2, ldw2, (int)rows2, y2, ldy2); break;
+      default: launch_gemv_rows<4>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, W2, ldw2, (int)rows2, y2, ldy2); break;
     }
     return check_launch("gemv_rows_kernel");
   }
@@ -1253,13 +1332,8 @@ extern "C" int moc_gemv_rmsnorm_bf16(const void* x, int64_t ldx, int64_t nb, con
   MOC_REQUIRE(aligned16(x) && aligned16(W) && aligned16(norm_w) && aligned16(xn),
               "moc_gemv_rmsnorm_bf16: x, norm_w, xn and W must be 16-byte aligned");
   hipStream_t st = as_stream(stream);
-  switch (nb) {
-    case 1: launch_gemv_rows<1, true>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, norm_w, eps, xn, ldxn); break;
-    case 2: launch_gemv_rows<2, true>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, norm_w, eps, xn, ldxn); break;
-    case 3: launch_gemv_rows<3, true>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, norm_w, eps, xn, ldxn); break;
-    default: launch_gemv_rows<4, true>(x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, norm_w, eps, xn, ldxn); break;
-  }
-  return check_launch("gemv_rows_kernel (rmsnorm)");
+  gemv_norm_rows(nb, x, ldx, W, ldw, (int)rows, (int)hidden, y, ldy, st, norm_w, eps, xn, ldxn);
+  return check_launch("gemv_norm_rows_kernel");
 }
 
 extern "C" int moc_selected_up_silu_bf16(const void* x, int64_t nb, int64_t hidden,
@@ -1440,15 +1514,11 @@ int global_decode_sd(const void* x, int64_t nb, int64_t hidden, const void* norm
   const int in = static_cast<int>(inter), hd = static_cast<int>(hidden);
   int rc;
   if (norm_w != nullptr) {
-    // gate rows, then the up rows as the pair's second range; every wave
-    // normalises its own copy of x (nb <= 4, checked by the caller)
-    switch (nb) {
-      case 1: launch_gemv_rows<1, true>(x, hidden, w_gate, hidden, in, hd, gs, pitch, st, norm_w, eps, xn, hidden, w_up, hidden, in, u, pitch); break;
-      case 2: launch_gemv_rows<2, true>(x, hidden, w_gate, hidden, in, hd, gs, pitch, st, norm_w, eps, xn, hidden, w_up, hidden, in, u, pitch); break;
-      case 3: launch_gemv_rows<3, true>(x, hidden, w_gate, hidden, in, hd, gs, pitch, st, norm_w, eps, xn, hidden, w_up, hidden, in, u, pitch); break;
-      default: launch_gemv_rows<4, true>(x, hidden, w_gate, hidden, in, hd, gs, pitch, st, norm_w, eps, xn, hidden, w_up, hidden, in, u, pitch); break;
-    }
-    rc = check_launch("gemv_rows_kernel");
+    // gate rows, then the up rows as the pair's second range (nb <= 4,
+    // checked by the caller)
+    gemv_norm_rows(nb, x, hidden, w_gate, hidden, in, hd, gs, pitch, st, norm_w, eps, xn, hidden, w_up, hidden, in, u,
+                   pitch);
+    rc = check_launch("gemv_norm_rows_kernel");
   } else if (nb >= 3 && nb <= 4 && hidden <= 4096) {
     // 3-4 tokens: one wave per (gate row, up row) pair measured faster
     // (4 tokens 24.3 -> 23.1 us per layer); 1-2 tokens: the two-range form
