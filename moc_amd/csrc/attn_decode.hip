@@ -120,89 +120,94 @@ __global__ __launch_bounds__(kAdThreads) void decode_qkv_kernel(
   }
 }
 
-// One head per workgroup.  K^T [head_dim, max_seq]: thread (g, j) of 4 x 128
-// sums its quarter of the dimensions for positions 2j, 2j + 1 of each block
-// of 256; V [max_seq, head_dim]: thread (p, c) of P x head_dim / 8 sums the
-// positions p, p + P, ... of its eight dimensions.  The first V rows are
-// requested before the scores, so the two passes share one memory latency.
-constexpr int kAttnThreads = 512;
-constexpr int kAttnVPre = 8;       // V rows per thread requested ahead
+// One head per workgroup of 16 waves.  The launch is a chain of latencies, so
+// everything that does not depend on the scores is requested at once: q, the
+// position, the first 256 positions of K^T (which need no position: those past
+// it are masked) and of V.
+//   K^T [head_dim, max_seq]: thread (g, j) of 8 x 128 sums its eighth of the
+//     dimensions (at most DPT) for positions 2j, 2j + 1 of a block of 256;
+//   V [max_seq, head_dim]: thread (p, c) of P x head_dim / 8 sums positions p,
+//     p + P, ... of its eight dimensions.
+// One head of 128 dimensions, 129 positions, in the chain of a decode step:
+// 7.4 us (8 waves, four groups of dimensions, the loads behind the position:
+// 18.4 us).
+constexpr int kAttnThreads = 1024;
+constexpr int kAttnWaves = kAttnThreads / 64;
+constexpr int kAttnGroups = 8;     // groups of dimensions
+constexpr int kAttnVPre = 4;       // V rows per thread requested ahead
 constexpr int kAttnMaxSeq = 8192;  // scores held in LDS
 constexpr int kAttnMaxDim = 256;
 
+template <int DPT, bool EVEN>
 __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_t, const uint16_t* __restrict__ v,
     const int64_t* __restrict__ pos_p, int head_dim, int max_seq, float scale, uint16_t* __restrict__ y) {
   extern __shared__ __attribute__((aligned(16))) float lds[];
   __shared__ float qs[kAttnMaxDim];
-  __shared__ float part[4][256];
-  __shared__ float wred[2][kAttnThreads / 64];
+  __shared__ float part[kAttnGroups][256];
+  __shared__ float wred[2][kAttnWaves];
   float* sc = lds;  // [max_seq rounded to 256], then the V partial sums [P][head_dim]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int head = blockIdx.x;
-  const int64_t pos = *pos_p;
-  const int n = (pos < 0 || pos >= max_seq) ? 0 : static_cast<int>(pos) + 1;
   const uint16_t* kh = k_t + static_cast<int64_t>(head) * head_dim * max_seq;
   const uint16_t* vh = v + static_cast<int64_t>(head) * max_seq * head_dim;
+  const int g = tid >> 7, j2 = (tid & 127) * 2;
+  const int dpt = head_dim / kAttnGroups, d0 = g * dpt;
+  // two neighbouring positions of one dimension; 0 past the cache
+  auto load_k = [&](int d, int j) -> uint32_t {
+    const uint16_t* p = kh + static_cast<int64_t>(d0 + d) * max_seq + j;
+    if (EVEN) return j < max_seq ? *reinterpret_cast<const uint32_t*>(p) : 0u;
+    return j + 1 < max_seq ? p[0] | (static_cast<uint32_t>(p[1]) << 16) : j < max_seq ? p[0] : 0u;
+  };
+  uint32_t kk[DPT];
+#pragma unroll
+  for (int d = 0; d < DPT; ++d) kk[d] = d < dpt ? load_k(d, j2) : 0u;
+  const int64_t pos = *pos_p;
+  if (tid < head_dim) qs[tid] = bf16_to_f32(q[head * head_dim + tid]) * scale;
   const int cpr = head_dim / 8, P = kAttnThreads / cpr;
   const int vp = tid / cpr, vc = tid - vp * cpr;
   uint4 vv[kAttnVPre];
 #pragma unroll
   for (int i = 0; i < kAttnVPre; ++i) {
     const int j = vp + P * i;
-    vv[i] = vp < P && j < n ? *reinterpret_cast<const uint4*>(vh + static_cast<int64_t>(j) * head_dim + vc * 8)
-                            : make_uint4(0, 0, 0, 0);
+    vv[i] = vp < P && j < max_seq ? *reinterpret_cast<const uint4*>(vh + static_cast<int64_t>(j) * head_dim + vc * 8)
+                                  : make_uint4(0, 0, 0, 0);
   }
-  if (tid < head_dim) qs[tid] = bf16_to_f32(q[head * head_dim + tid]) * scale;
+  const int n = (pos < 0 || pos >= max_seq) ? 0 : static_cast<int>(pos) + 1;
   __syncthreads();
 
   // scores of blocks of 256 positions
-  const int g = tid >> 7, j2 = (tid & 127) * 2;
-  const int d_lo = g * head_dim / 4, d_hi = (g + 1) * head_dim / 4;
-  const bool even = (max_seq & 1) == 0;
   float mx = -INFINITY;
   for (int b0 = 0; b0 < n; b0 += 256) {
-    const int j = b0 + j2;
+    if (b0 > 0) {
+      __syncthreads();  // the block before is summed
+#pragma unroll
+      for (int d = 0; d < DPT; ++d) kk[d] = d < dpt ? load_k(d, b0 + j2) : 0u;
+    }
     float a0 = 0.f, a1 = 0.f;
-    if (j < n) {
-      const uint16_t* p = kh + j;
-      if (even) {
-#pragma unroll 16
-        for (int d = d_lo; d < d_hi; ++d) {
-          const uint32_t kk = *reinterpret_cast<const uint32_t*>(p + static_cast<int64_t>(d) * max_seq);
-          a0 = fmaf(qs[d], __uint_as_float(kk << 16), a0);
-          a1 = fmaf(qs[d], __uint_as_float(kk & 0xFFFF0000u), a1);
-        }
-      } else {
-        const int o = j + 1 < n ? 1 : 0;
-#pragma unroll 16
-        for (int d = d_lo; d < d_hi; ++d) {
-          const uint16_t* pd = p + static_cast<int64_t>(d) * max_seq;
-          a0 = fmaf(qs[d], bf16_to_f32(pd[0]), a0);
-          a1 = fmaf(qs[d], bf16_to_f32(pd[o]), a1);
-        }
+#pragma unroll
+    for (int d = 0; d < DPT; ++d)
+      if (d < dpt) {
+        a0 = fmaf(qs[d0 + d], __uint_as_float(kk[d] << 16), a0);
+        a1 = fmaf(qs[d0 + d], __uint_as_float(kk[d] & 0xFFFF0000u), a1);
       }
-    }
-    part[g][j2] = a0;
-    part[g][j2 + 1] = a1;
+    *reinterpret_cast<float2*>(&part[g][j2]) = make_float2(a0, a1);
     __syncthreads();
-    if (tid < 256) {
-      const float s = (part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]);
-      if (b0 + tid < n) {
-        sc[b0 + tid] = s;
-        mx = fmaxf(mx, s);
-      }
+    if (tid < 256 && b0 + tid < n) {
+      float s = 0.f;
+#pragma unroll
+      for (int i = 0; i < kAttnGroups; ++i) s += part[i][tid];
+      sc[b0 + tid] = s;
+      mx = fmaxf(mx, s);
     }
-    __syncthreads();
   }
-  // softmax (f32): NaN scores stay NaN through the sum
+  // softmax (a NaN score makes the sum NaN)
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
   if (lane == 0) wred[0][wave] = mx;
   __syncthreads();
-  mx = wred[0][0];
 #pragma unroll
-  for (int w = 1; w < kAttnThreads / 64; ++w) mx = fmaxf(mx, wred[0][w]);
+  for (int w = 0; w < 4; ++w) mx = fmaxf(mx, wred[0][w]);  // the waves that hold scores
   float sum = 0.f;
   for (int j = tid; j < n; j += kAttnThreads) {
     const float e = expf(sc[j] - mx);
@@ -214,7 +219,7 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
   __syncthreads();
   sum = 0.f;
 #pragma unroll
-  for (int w = 0; w < kAttnThreads / 64; ++w) sum += wred[1][w];
+  for (int w = 0; w < kAttnWaves; ++w) sum += wred[1][w];
 
   // weighted sum of V
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -237,13 +242,23 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attn_kernel(
   }
   __syncthreads();  // the scores' LDS becomes the partial sums
   if (vp < P) {
-#pragma unroll
-    for (int e = 0; e < 8; ++e) lds[vp * head_dim + vc * 8 + e] = acc[e];
+    float4* o = reinterpret_cast<float4*>(lds + vp * head_dim + vc * 8);
+    o[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    o[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+  }
+  __syncthreads();
+  // thread (s, d) of S x head_dim adds the partial sums s, s + S, ...
+  const int S = min(kAttnGroups, kAttnThreads / head_dim), sg = tid / head_dim, sd = tid - sg * head_dim;
+  float* fin = &part[0][0];  // S head_dim <= 2048 floats
+  if (sg < S) {
+    float t = 0.f;
+    for (int p = sg; p < P; p += S) t += lds[p * head_dim + sd];
+    fin[sg * head_dim + sd] = t;
   }
   __syncthreads();
   if (tid < head_dim) {
     float t = 0.f;
-    for (int p = 0; p < P; ++p) t += lds[p * head_dim + tid];
+    for (int s = 0; s < S; ++s) t += fin[s * head_dim + tid];
     y[head * head_dim + tid] = f32_to_bf16(t / sum);
   }
 }
@@ -317,8 +332,20 @@ extern "C" int moc_decode_attention_bf16(const void* x, int64_t hidden, int64_t 
   if (rc != MOC_OK) return rc;
   const size_t sc = static_cast<size_t>((S + 255) / 256 * 256) * 4;
   const size_t part = static_cast<size_t>(kAttnThreads / (dim / 8)) * dim * 4;
-  decode_attn_kernel<<<dim3(static_cast<unsigned>(heads)), dim3(kAttnThreads), std::max(sc, part), st>>>(
-      q, (const uint16_t*)k_t, (const uint16_t*)v, pos, dim, S, scale, o);
+  const dim3 ga(static_cast<unsigned>(heads)), ba(kAttnThreads);
+#define MOC_ATTN(D, E)                                                                                      \
+  decode_attn_kernel<D, E><<<ga, ba, std::max(sc, part), st>>>(q, (const uint16_t*)k_t, (const uint16_t*)v, \
+                                                               pos, dim, S, scale, o)
+  if (S % 2 == 0) {  // two positions of a dimension in one aligned word
+    if (dim <= 64) MOC_ATTN(8, true);
+    else if (dim <= 128) MOC_ATTN(16, true);
+    else MOC_ATTN(32, true);
+  } else {
+    if (dim <= 64) MOC_ATTN(8, false);
+    else if (dim <= 128) MOC_ATTN(16, false);
+    else MOC_ATTN(32, false);
+  }
+#undef MOC_ATTN
   rc = check_launch("decode_attn_kernel");
   if (rc != MOC_OK) return rc;
 #define MOC_OUT(C)                                                                                               \
