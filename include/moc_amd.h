@@ -495,6 +495,17 @@ int moc_grouped_top2_up_silu_bf16(const void* x, int64_t nb, int64_t hidden, con
                                   const void* w_up, int64_t inter, void* idx, void* sz,
                                   void* stream);
 
+/* A decoder layer's FFN half x + FFN(RMSNorm(x)) for at most 16 tokens
+ * (benchmarks/inference/benchmark_decode.py:101-109,303): global Top-K of k
+ * channels, or with g28 the top 2 of every 8 (k = inter / 4).  hidden a
+ * multiple of 256 up to 4096; y must not alias x; workspace:
+ * moc_moc28_decode_workspace_size(nb, max(inter, 8), hidden) bytes, no
+ * contents kept. */
+int moc_decode_block_bf16(const void* x, int64_t nb, int64_t hidden, const void* norm_w, float eps,
+                          const void* w_gate, const void* w_up, int64_t inter, const void* w_down_t,
+                          int64_t ldw_down, int64_t k, int g28, void* y, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+
 /* Workspace bytes of moc_moc28_decode_bf16 (no zeroing needed). */
 int64_t moc_moc28_decode_workspace_size(int64_t nb, int64_t inter, int64_t hidden);
 

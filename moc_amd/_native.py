@@ -74,6 +74,8 @@ SIGNATURES: dict[str, tuple] = {
                                            _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _i64,
                                            _int, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _i64, _int, _vp,
                                            _int, _vp, _i64, _vp]),
+    "moc_decode_block_bf16": (_int, [_vp, _i64, _i64, _vp, ctypes.c_float, _vp, _vp, _i64, _vp, _i64, _i64,
+                                     _int, _vp, _vp, _i64, _vp]),
     "moc_decode_attention_workspace_size": (_i64, [_i64]),
     "moc_decode_attention_bf16": (_int, [_vp, _i64, _i64, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _i64,
                                          _vp, _vp, ctypes.c_float, _vp, _vp, _i64, _vp]),

@@ -31,6 +31,9 @@
 #include "select.h"
 
 extern "C" int moc_fill_zero(void* dst, int64_t bytes, void* stream);
+extern "C" int moc_rmsnorm_rows_bf16(const void* x, int64_t ldx, int64_t rows, int64_t d, const void* w, float eps,
+                                     void* y, int64_t ldy, float* rstd, void* stream);
+extern "C" int64_t moc_moc28_decode_workspace_size(int64_t nb, int64_t inter, int64_t hidden);
 
 namespace moc {
 namespace {
@@ -1513,7 +1516,12 @@ int global_decode_sd(const void* x, int64_t nb, int64_t hidden, const void* norm
   void* xn = ws + kFusedCounterBytes + 2 * align256(nb * pitch * 2);
   const int in = static_cast<int>(inter), hd = static_cast<int>(hidden);
   int rc;
-  if (norm_w != nullptr) {
+  if (norm_w != nullptr && nb > 4) {
+    // the tokens normalised by a row kernel, then the MFMA GEMV pair
+    rc = moc_rmsnorm_rows_bf16(x, hidden, nb, hidden, norm_w, eps, xn, hidden, nullptr, st);
+    if (rc != MOC_OK) return rc;
+    rc = gemv_launch(xn, hidden, nb, w_gate, hidden, inter, hidden, gs, pitch, w_up, hidden, inter, u, pitch, st);
+  } else if (norm_w != nullptr) {
     // gate rows, then the up rows as the pair's second range (nb <= 4,
     // checked by the caller)
     gemv_norm_rows(nb, x, hidden, w_gate, hidden, in, hd, gs, pitch, st, norm_w, eps, xn, hidden, w_up, hidden, in, u,
@@ -1630,6 +1638,35 @@ extern "C" int moc_global_decode_rmsnorm_residual_bf16(const void* x, int64_t nb
               "moc_global_decode_rmsnorm_residual_bf16: workspace of %lld bytes required", (long long)need);
   return global_decode_sd(x, nb, hidden, norm_w, eps, w_gate, w_up, inter, w_down_t, ldw_down, k, x, y, idx_out,
                           static_cast<char*>(workspace), as_stream(stream));
+}
+
+// x + FFN(RMSNorm(x)) for up to 16 tokens: global Top-K, or (g28) the top 2 of
+// every 8 channels.  Up to 4 tokens the launches of the entry points above
+// and below; more: the norm as a row kernel in front of them.  16 tokens of
+// 2048 -> 5464, 2:8: the norm's seven and the residual's one elementwise
+// launch took 25 of 50 us a layer.
+extern "C" int moc_decode_block_bf16(const void* x, int64_t nb, int64_t hidden, const void* norm_w, float eps,
+                                     const void* w_gate, const void* w_up, int64_t inter, const void* w_down_t,
+                                     int64_t ldw_down, int64_t k, int g28, void* y, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+  MOC_REQUIRE(nb >= 0 && nb <= 16, "moc_decode_block_bf16: 0 <= nb <= 16 tokens");
+  MOC_REQUIRE(inter >= 1 && hidden >= 256 && hidden <= 4096 && k >= 1 && k <= inter &&
+                  sd_fits(nb < 1 ? 1 : nb, inter, k, hidden) && (!g28 || (inter % 8 == 0 && k == inter / 4)),
+              "moc_decode_block_bf16: hidden a multiple of 256 up to 4096, inter <= %d, k <= %d (2:8: inter a "
+              "multiple of 8, k = inter / 4)", kSdMaxInter, kSdMaxK);
+  MOC_REQUIRE(eps >= 0.f, "moc_decode_block_bf16: eps must be >= 0");
+  if (nb == 0) return MOC_OK;
+  MOC_REQUIRE(x && norm_w && w_gate && w_up && w_down_t && y && workspace, "moc_decode_block_bf16: null pointer");
+  MOC_REQUIRE(aligned16(x) && aligned16(norm_w) && aligned16(w_gate) && aligned16(w_up) && aligned16(w_down_t) &&
+                  aligned16(workspace),
+              "moc_decode_block_bf16: operands must be 16-byte aligned");
+  MOC_REQUIRE(ldw_down >= hidden && ldw_down % 8 == 0,
+              "moc_decode_block_bf16: ldw_down must be a multiple of 8 and >= hidden");
+  MOC_REQUIRE(y != x, "moc_decode_block_bf16: y must not alias x");
+  const int64_t need = moc_moc28_decode_workspace_size(nb, inter < 8 ? 8 : inter, hidden);
+  MOC_REQUIRE(workspace_bytes >= need, "moc_decode_block_bf16: workspace of %lld bytes required", (long long)need);
+  return global_decode_sd(x, nb, hidden, norm_w, eps, w_gate, w_up, inter, w_down_t, ldw_down, k, x, y, nullptr,
+                          static_cast<char*>(workspace), as_stream(stream), g28 != 0);
 }
 
 extern "C" int64_t moc_moc28_decode_workspace_size(int64_t nb, int64_t inter, int64_t hidden) {

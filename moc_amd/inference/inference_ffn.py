@@ -263,12 +263,13 @@ class InferenceMoCSwiGLUFFN(nn.Module):
 
     def fused_decode_residual(self, x: torch.Tensor, norm_weight: torch.Tensor,
                               eps: float) -> torch.Tensor:
-        """x + FFN(RMSNorm(x)) for a decoder layer's FFN half, <= 4 tokens,
+        """x + FFN(RMSNorm(x)) for a decoder layer's FFN half, up to 4 tokens
         in two launches: the pre-norm runs inside the gate GEMV (global MoC)
         or the fused gate/up + top-2-of-8 kernel (MoC 2:8), the residual add
         inside the last step of the after-gate kernel or of the selected
         Down (the layer of benchmark_decode.py:303 with RMSNorm of
-        :101-109).  Other shapes: the same result unfused."""
+        :101-109).  More tokens: the norm as one launch before the layer's.
+        Other shapes: the same result unfused."""
         x_2d, shp = self._flatten_decode_input(x)
         grouped28 = self.config.grouped and self.config.grouped_a == 2 and self.config.grouped_b == 8
         if grouped28 and x_2d.shape[0] <= 4 and x_2d.dtype == torch.bfloat16:
@@ -285,6 +286,27 @@ class InferenceMoCSwiGLUFFN(nn.Module):
                                              norm_weight=norm_weight, eps=eps)
             y = K.selected_grouped_down(sz, idx, self._down_weight_t, residual=x_2d)
             return self._restore_output_shape(y, shp)
+        nb, c = x_2d.shape[0], self.config
+        if nb > 4 and (grouped28 or not c.grouped) and x_2d.is_cuda and x_2d.dtype == norm_weight.dtype == torch.bfloat16 \
+                and self.gate_proj.weight.dtype == torch.bfloat16 \
+                and not (torch.is_grad_enabled() and (x.requires_grad or norm_weight.requires_grad)):
+            # more tokens: the norm as a row kernel in front of the layer's
+            # kernels, the residual added in the last of them
+            ensure_native_ops_ready()
+            self._ensure_down_weight_t()
+            x_2d = x_2d.contiguous()
+            if nb <= 16 and K.decode_block_fits(nb, c.intermediate_size, c.k, c.hidden_size):
+                ws = (self._moc28_decode_workspace(nb, x_2d.device) if grouped28
+                      else self._global_decode_workspace(nb, x_2d.device))
+                y = K.decode_block(x_2d, norm_weight, eps, self.gate_proj.weight, self.up_proj.weight,
+                                   self._down_weight_t, c.k, grouped=grouped28, workspace=ws)
+                return self._restore_output_shape(y, shp)
+            if nb > 16 and c.hidden_size % 8 == 0 and c.hidden_size <= 4096 and self._dense_infer_ok(x_2d) and \
+                    (not grouped28 or self._dense28(nb)):
+                xn, _ = K.rmsnorm_rows(x_2d, norm_weight, eps, want_rstd=False)
+                y = K.ffn_infer(xn, self.gate_proj.weight, self.up_proj.weight, self._down_weight_t, c.k,
+                                grouped=grouped28, residual=x_2d)
+                return self._restore_output_shape(y, shp)
         if self.config.grouped or x_2d.shape[0] > 4 or x_2d.dtype != torch.bfloat16:
             xf = x_2d.float()
             xn = (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)).to(x_2d.dtype) * norm_weight

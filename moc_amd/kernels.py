@@ -767,6 +767,35 @@ def global_decode_rmsnorm_residual_fits(nb: int, inter: int, k: int, hidden: int
     return 1 <= nb <= 4 and hidden % 256 == 0 and hidden <= 4096 and inter <= 8192 and int(k) <= 4096
 
 
+def decode_block(x, norm_weight, eps: float, gate_weight, up_weight, down_weight_t, k: int, *,
+                 grouped: bool = False, workspace=None) -> torch.Tensor:
+    """x + FFN(RMSNorm(x)) for at most 16 tokens (moc_decode_block_bf16):
+    global Top-K, or with `grouped` the top 2 of every 8 channels."""
+    N.require_device(x, norm_weight, gate_weight, up_weight, down_weight_t)
+    x, nw, wg, wu = _bf16_contig(x, norm_weight, gate_weight, up_weight)
+    wdt, ldw = _down_t_rows(down_weight_t)
+    nb, hidden = x.shape
+    inter = wg.shape[0]
+    if (wg.shape != (inter, hidden) or wu.shape != wg.shape or wdt.shape != wg.shape or nw.shape != (hidden,)
+            or not decode_block_fits(nb, inter, int(k), hidden)):
+        raise ValueError(f"decode_block: unsupported shape nb={nb}, inter={inter}, hidden={hidden}, k={k}")
+    y = torch.empty_like(x)
+    ws_bytes = moc28_decode_workspace_bytes(nb, max(inter, 8), hidden)
+    if workspace is None:
+        workspace = _decode_workspace(x.device, ws_bytes)
+    elif workspace.numel() < ws_bytes:
+        raise ValueError(f"decode_block: workspace of {ws_bytes} bytes required")
+    N.call("moc_decode_block_bf16", x.data_ptr(), nb, hidden, nw.data_ptr(), float(eps), wg.data_ptr(),
+           wu.data_ptr(), inter, wdt.data_ptr(), ldw, int(k), int(grouped), y.data_ptr(), workspace.data_ptr(),
+           ws_bytes, N.stream_of(x))
+    return y
+
+
+def decode_block_fits(nb: int, inter: int, k: int, hidden: int) -> bool:
+    """Shapes moc_decode_block_bf16 takes."""
+    return 1 <= nb <= 16 and hidden % 256 == 0 and hidden <= 4096 and inter <= 8192 and int(k) <= 4096
+
+
 def decode_attention(x, norm_weight, eps: float, qkv_weight, out_weight, cos, sin, pos, k_t, v,
                      scale: float) -> torch.Tensor:
     """x + out_proj(attention(RoPE(qkv_proj(RMSNorm(x))))) of one token x

@@ -98,3 +98,26 @@ def test_28_nan_rows_and_ties():
     ref, mags = _reference(torch.nan_to_num(x), w, 0, True)
     keep = [i for i in range(20) if i != 3]
     _check(y[keep], ref[keep], mags[keep], 64)
+
+
+@pytest.mark.parametrize("nb", [5, 8, 9, 16, 17, 40])
+@pytest.mark.parametrize("grouped", [False, True])
+@pytest.mark.parametrize("hidden,inter", [(256, 704), (1024, 2736), (2048, 5464)])
+def test_layer_with_norm_and_residual(nb, grouped, hidden, inter):
+    """x + FFN(RMSNorm(x)) equals the layer on the row kernel's norm, plus x,
+    bit for bit: the same launches with the residual in the last one."""
+    gen = torch.Generator(device="cuda").manual_seed(nb + hidden)
+    kw = dict(grouped_a=2, grouped_b=8) if grouped else {}
+    m = InferenceMoCSwiGLUFFN(hidden, inter, inter // 4 if grouped else hidden // 2, **kw).to("cuda", BF)
+    x = torch.randn(nb, hidden, generator=gen, device="cuda").to(BF)
+    w = (1 + 0.1 * torch.randn(hidden, generator=gen, device="cuda")).to(BF)
+    xn, _ = K.rmsnorm_rows(x, w, 1e-6)
+    xf = x.float()
+    stock = (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-6)).to(BF) * w
+    # the factor's f32 sum runs in another order: an ulp of f32 decides a
+    # bf16 rounding at most here and there
+    assert ((xn.float() - stock.float()).abs() <= 2.0 ** -7 * stock.float().abs()).all()
+    with torch.no_grad():
+        y = m.fused_decode_residual(x, w, 1e-6)
+        assert torch.equal(y, (x.float() + m(xn).float()).to(BF))
+        assert torch.equal(y[:, None], m.fused_decode_residual(x[:, None], w, 1e-6))
