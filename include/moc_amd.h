@@ -302,6 +302,37 @@ int moc_ffn_backward_bf16(int64_t rows, int64_t d, int64_t inter, int64_t k, con
 int moc_rmsnorm_rows_bf16(const void* x, int64_t ldx, int64_t rows, int64_t d, const void* w, float eps,
                           void* y, int64_t ldy, float* rstd, void* stream);
 
+/* moc_rmsnorm_rows_bf16 / moc_rmsnorm_backward_bf16 of an f32 stream (x, dres,
+ * dx, the norm weight and its gradient f32; y and dy bf16), as in a model with
+ * f32 parameters under bf16 autocast: y = bf16(x r w), rounded once.  Same
+ * workspace size as the bf16 backward. */
+int moc_rmsnorm_rows_f32(const float* x, int64_t ldx, int64_t rows, int64_t d, const float* w, float eps,
+                         void* y, int64_t ldy, float* rstd, void* stream);
+int moc_rmsnorm_backward_f32(const float* x, int64_t ldx, int64_t rows, int64_t d, const float* w,
+                             const float* rstd, const void* dy, int64_t lddy, const float* dres, int64_t ldres,
+                             float* dx, int64_t lddx, float* dw, void* workspace, int64_t workspace_bytes,
+                             void* stream);
+
+/* bf16 copies (round to nearest even) of n <= 8 contiguous f32 matrices
+ * [rows[i], cols[i]] in one launch; dst rows dst_ld[i] apart, 16-byte aligned,
+ * whole chunks of 8 (zeros past cols). */
+int moc_cast_bf16_multi(int n, const void* const* src, const int64_t* rows, const int64_t* cols,
+                        void* const* dst, const int64_t* dst_ld, void* stream);
+
+/* Causal attention with RoPE on q and k (moc/model.py:31-64), forward and
+ * backward: qkv [batch seq, 3 heads head_dim] bf16 (rows ld apart: q, k, v, each
+ * by head), cos, sin [>= seq, head_dim / 2] in table_dtype, pairs (2i, 2i + 1);
+ * head_dim 64 or 128; o, go [batch seq, heads head_dim] bf16; lse, delta [batch,
+ * heads, seq] f32 (lse in log2; delta is scratch of the backward); dqkv laid
+ * out as qkv. */
+int moc_rope_attention_forward_bf16(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim,
+                                    const void* qkv, int64_t ld, const void* cos, const void* sin,
+                                    int table_dtype, float scale, void* o, float* lse, void* stream);
+int moc_rope_attention_backward_bf16(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim,
+                                     const void* qkv, int64_t ld, const void* cos, const void* sin,
+                                     int table_dtype, float scale, const void* o, const float* lse,
+                                     const void* go, float* delta, void* dqkv, void* stream);
+
 /* Workspace bytes of moc_rmsnorm_backward_bf16 (f32 partial rows of dw). */
 int64_t moc_rmsnorm_backward_workspace_size(int64_t rows, int64_t d);
 

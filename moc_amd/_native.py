@@ -76,6 +76,14 @@ SIGNATURES: dict[str, tuple] = {
                                            _int, _vp, _i64, _vp]),
     "moc_decode_block_bf16": (_int, [_vp, _i64, _i64, _vp, ctypes.c_float, _vp, _vp, _i64, _vp, _i64, _i64,
                                      _int, _vp, _vp, _i64, _vp]),
+    "moc_rmsnorm_rows_f32": (_int, [_vp, _i64, _i64, _i64, _vp, ctypes.c_float, _vp, _i64, _vp, _vp]),
+    "moc_rmsnorm_backward_f32": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64,
+                                        _vp, _vp, _i64, _vp]),
+    "moc_cast_bf16_multi": (_int, [_int, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "moc_rope_attention_forward_bf16": (_int, [_i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _int,
+                                               ctypes.c_float, _vp, _vp, _vp]),
+    "moc_rope_attention_backward_bf16": (_int, [_i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _int,
+                                                ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp]),
     "moc_decode_attention_workspace_size": (_i64, [_i64]),
     "moc_decode_attention_bf16": (_int, [_vp, _i64, _i64, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _i64,
                                          _vp, _vp, ctypes.c_float, _vp, _vp, _i64, _vp]),

@@ -198,6 +198,167 @@ __global__ __launch_bounds__(64 * kDwWaves) void rmsnorm_dw_reduce_kernel(const 
   }
 }
 
+// The same for an f32 stream with f32 norm weights whose consumer is a bf16
+// product (a model with f32 parameters under bf16 autocast): y = bf16(x r w),
+// rounded once, where the stock norm stores x r and x r w in f32 and casts;
+// dx = dres + r (dy w) - (r^3 / d) x sum_j(dy_j w_j x_j) in f32 from the bf16
+// dy, dw = sum over rows of dy x r.
+struct F8 {
+  float v[8];
+};
+__device__ __forceinline__ F8 load8(const float* p) {
+  const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+  return {{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
+}
+__device__ __forceinline__ F8 zero8() { return {{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}}; }
+
+template <int NC>
+__global__ __launch_bounds__(64 * kRmsWaves) void rmsnorm_f32_rows_kernel(
+    const float* __restrict__ x, int64_t ldx, int rows, int d, const float* __restrict__ w, float eps,
+    uint16_t* __restrict__ y, int64_t ldy, float* __restrict__ rstd) {
+  const int lane = threadIdx.x & 63;
+  const int nchunk = d >> 3;
+  const int waves = gridDim.x * kRmsWaves;
+  for (int row = blockIdx.x * kRmsWaves + (threadIdx.x >> 6); row < rows; row += waves) {
+    const float* xr = x + static_cast<int64_t>(row) * ldx;
+    F8 xv[NC];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int c = lane + 64 * i;
+      xv[i] = c < nchunk ? load8(xr + 8 * c) : zero8();
+#pragma unroll
+      for (int q = 0; q < 8; ++q) ss = fmaf(xv[i].v[q], xv[i].v[q], ss);
+    }
+    ss = wave_sum(ss);
+    const float r = 1.0f / sqrtf(ss / static_cast<float>(d) + eps);
+    uint16_t* yr = y + static_cast<int64_t>(row) * ldy;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int c = lane + 64 * i;
+      if (c >= nchunk) continue;
+      const F8 wv = load8(w + 8 * c);
+      uint32_t o[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        o[q] = pack2(xv[i].v[2 * q] * r * wv.v[2 * q], xv[i].v[2 * q + 1] * r * wv.v[2 * q + 1]);
+      *reinterpret_cast<uint4*>(yr + 8 * c) = make_uint4(o[0], o[1], o[2], o[3]);
+    }
+    if (lane == 0 && rstd != nullptr) rstd[row] = r;
+  }
+}
+
+template <int NC>
+__global__ __launch_bounds__(64 * kRmsWaves) void rmsnorm_f32_bwd_rows_kernel(
+    const float* __restrict__ x, int64_t ldx, int rows, int d, const float* __restrict__ w,
+    const float* __restrict__ rstd, const uint16_t* __restrict__ dy, int64_t lddy, const float* __restrict__ dres,
+    int64_t ldres, float* __restrict__ dx, int64_t lddx, float* __restrict__ dw_part) {
+  __shared__ float red[kRmsWaves][64 * 8];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int nchunk = d >> 3;
+  F8 wv[NC];
+  float dwa[NC][8];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int c = lane + 64 * i;
+    wv[i] = c < nchunk ? load8(w + 8 * c) : zero8();
+#pragma unroll
+    for (int q = 0; q < 8; ++q) dwa[i][q] = 0.f;
+  }
+  const float inv_d = 1.0f / static_cast<float>(d);
+  const int waves = gridDim.x * kRmsWaves;
+  for (int row = blockIdx.x * kRmsWaves + wave; row < rows; row += waves) {
+    const float* xr = x + static_cast<int64_t>(row) * ldx;
+    const uint16_t* gr = dy + static_cast<int64_t>(row) * lddy;
+    const float r = rstd[row];
+    F8 xv[NC];
+    float gw[NC][8];  // dy w
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int c = lane + 64 * i;
+      const bool ok = c < nchunk;
+      xv[i] = ok ? load8(xr + 8 * c) : zero8();
+      const uint4 gv = ok ? *reinterpret_cast<const uint4*>(gr + 8 * c) : make_uint4(0, 0, 0, 0);
+      const uint32_t ge[4] = {gv.x, gv.y, gv.z, gv.w};
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const float g = (q & 1) ? hi16(ge[q >> 1]) : lo16(ge[q >> 1]);
+        gw[i][q] = g * wv[i].v[q];
+        s = fmaf(gw[i][q], xv[i].v[q], s);
+        dwa[i][q] = fmaf(g, xv[i].v[q] * r, dwa[i][q]);
+      }
+    }
+    s = wave_sum(s);
+    const float c3 = s * r * r * r * inv_d;
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int c = lane + 64 * i;
+      if (c >= nchunk) continue;
+      const F8 rv = dres != nullptr ? load8(dres + static_cast<int64_t>(row) * ldres + 8 * c) : zero8();
+      float o[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) o[q] = rv.v[q] + (r * gw[i][q] - c3 * xv[i].v[q]);
+      float4* p = reinterpret_cast<float4*>(dx + static_cast<int64_t>(row) * lddx + 8 * c);
+      p[0] = make_float4(o[0], o[1], o[2], o[3]);
+      p[1] = make_float4(o[4], o[5], o[6], o[7]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) red[wave][lane * 8 + q] = dwa[i][q];
+    __syncthreads();
+    for (int e = threadIdx.x; e < 64 * 8; e += 64 * kRmsWaves) {
+      const int col = 512 * i + e;
+      if (col < d) {
+        float t = red[0][e];
+#pragma unroll
+        for (int v = 1; v < kRmsWaves; ++v) t += red[v][e];
+        dw_part[static_cast<int64_t>(blockIdx.x) * d + col] = t;
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// f32 -> bf16 copies of up to kCastMax matrices in one launch (the weights of
+// a layer under autocast): workgroups [start[i], start[i + 1]) take matrix i,
+// eight consecutive columns a thread; dst rows 16-byte aligned, pitch dld.
+constexpr int kCastMax = 8;
+struct CastJob {
+  const float* src;
+  uint16_t* dst;
+  int64_t rows, cols, dld;
+};
+struct CastArgs {
+  CastJob job[kCastMax];
+  int start[kCastMax + 1];
+  int n;
+};
+
+__global__ __launch_bounds__(256) void cast_bf16_multi_kernel(CastArgs a) {
+  int i = 0;
+  while (i + 1 < a.n && static_cast<int>(blockIdx.x) >= a.start[i + 1]) ++i;
+  const CastJob& j = a.job[i];
+  const int64_t per = (j.cols + 7) / 8;
+  const int64_t g = static_cast<int64_t>(static_cast<int>(blockIdx.x) - a.start[i]) * 256 + threadIdx.x;
+  if (g >= j.rows * per) return;
+  const int64_t r = g / per, c = (g - r * per) * 8;
+  const float* s = j.src + r * j.cols + c;
+  float v[8];
+  if (c + 8 <= j.cols && (reinterpret_cast<uintptr_t>(s) & 15) == 0) {
+    const F8 f = load8(s);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = f.v[e];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = c + e < j.cols ? s[e] : 0.f;
+  }
+  *reinterpret_cast<uint4*>(j.dst + r * j.dld + c) =
+      make_uint4(pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7]));
+}
+
 int rms_blocks(int64_t rows) {
   return static_cast<int>(std::min<int64_t>((rows + kRmsWaves - 1) / kRmsWaves, kRmsMaxBlocks));
 }
@@ -283,4 +444,85 @@ extern "C" int moc_rmsnorm_backward_bf16(const void* x, int64_t ldx, int64_t row
   if (dw_dtype == MOC_F32) rmsnorm_dw_reduce_kernel<true><<<grid, 64 * kDwWaves, 0, st>>>(part, blocks, (int)d, dw);
   else rmsnorm_dw_reduce_kernel<false><<<grid, 64 * kDwWaves, 0, st>>>(part, blocks, (int)d, dw);
   return check_launch("rmsnorm_dw_reduce_kernel");
+}
+
+extern "C" int moc_rmsnorm_rows_f32(const float* x, int64_t ldx, int64_t rows, int64_t d, const float* w, float eps,
+                                    void* y, int64_t ldy, float* rstd, void* stream) {
+  MOC_REQUIRE(rows >= 0 && rows < (1LL << 31), "moc_rmsnorm_rows_f32: bad row count");
+  MOC_REQUIRE(d >= 8 && d % 8 == 0 && d <= 4096, "moc_rmsnorm_rows_f32: hidden must be a multiple of 8 in [8, 4096]");
+  MOC_REQUIRE(eps >= 0.f, "moc_rmsnorm_rows_f32: eps must be >= 0");
+  if (rows == 0) return MOC_OK;
+  MOC_REQUIRE(x && w && y && aligned16(x) && aligned16(w) && aligned16(y) && ldx % 4 == 0 && ldx >= d && ldy % 8 == 0 &&
+                  ldy >= d,
+              "moc_rmsnorm_rows_f32: x, y and w need 16-byte aligned rows");
+  const int blocks = static_cast<int>(std::min<int64_t>((rows + kRmsWaves - 1) / kRmsWaves, 8 * cu_count()));
+  hipStream_t st = as_stream(stream);
+  const int nc = static_cast<int>((d / 8 + 63) / 64);
+#define MOC_RMS_FWD(NC)                                                                                         \
+  rmsnorm_f32_rows_kernel<NC><<<blocks, 64 * kRmsWaves, 0, st>>>(x, ldx, (int)rows, (int)d, w, eps, (uint16_t*)y, \
+                                                                 ldy, rstd)
+  if (nc <= 1) MOC_RMS_FWD(1);
+  else if (nc <= 2) MOC_RMS_FWD(2);
+  else if (nc <= 4) MOC_RMS_FWD(4);
+  else MOC_RMS_FWD(8);
+#undef MOC_RMS_FWD
+  return check_launch("rmsnorm_f32_rows_kernel");
+}
+
+extern "C" int moc_rmsnorm_backward_f32(const float* x, int64_t ldx, int64_t rows, int64_t d, const float* w,
+                                        const float* rstd, const void* dy, int64_t lddy, const float* dres,
+                                        int64_t ldres, float* dx, int64_t lddx, float* dw, void* workspace,
+                                        int64_t workspace_bytes, void* stream) {
+  MOC_REQUIRE(rows >= 0 && rows < (1LL << 31), "moc_rmsnorm_backward_f32: bad row count");
+  MOC_REQUIRE(d >= 8 && d % 8 == 0 && d <= 4096,
+              "moc_rmsnorm_backward_f32: hidden must be a multiple of 8 in [8, 4096]");
+  MOC_REQUIRE(dw != nullptr && w != nullptr && aligned16(w), "moc_rmsnorm_backward_f32: null or unaligned w/dw");
+  if (rows == 0) return moc_fill_zero(dw, d * 4, stream);
+  MOC_REQUIRE(x && dy && dx && rstd && aligned16(x) && aligned16(dy) && aligned16(dx) && ldx % 4 == 0 && ldx >= d &&
+                  lddy % 8 == 0 && lddy >= d && lddx % 4 == 0 && lddx >= d &&
+                  (dres == nullptr || (aligned16(dres) && ldres % 4 == 0 && ldres >= d)),
+              "moc_rmsnorm_backward_f32: x, dy, dres and dx need 16-byte aligned rows");
+  const int64_t need = moc_rmsnorm_backward_workspace_size(rows, d);
+  MOC_REQUIRE(workspace != nullptr && workspace_bytes >= need && aligned16(workspace),
+              "moc_rmsnorm_backward_f32: workspace of %lld bytes required", (long long)need);
+  const int blocks = rms_blocks(rows);
+  auto* part = static_cast<float*>(workspace);
+  hipStream_t st = as_stream(stream);
+  const int nc = static_cast<int>((d / 8 + 63) / 64);
+#define MOC_RMS_BWD(NC)                                                                                     \
+  rmsnorm_f32_bwd_rows_kernel<NC><<<blocks, 64 * kRmsWaves, 0, st>>>(x, ldx, (int)rows, (int)d, w, rstd,     \
+                                                                     (const uint16_t*)dy, lddy, dres, ldres, \
+                                                                     dx, lddx, part)
+  if (nc <= 1) MOC_RMS_BWD(1);
+  else if (nc <= 2) MOC_RMS_BWD(2);
+  else if (nc <= 4) MOC_RMS_BWD(4);
+  else MOC_RMS_BWD(8);
+#undef MOC_RMS_BWD
+  int rc = check_launch("rmsnorm_f32_bwd_rows_kernel");
+  if (rc != MOC_OK) return rc;
+  rmsnorm_dw_reduce_kernel<true><<<dim3(static_cast<unsigned>((d + 63) / 64)), 64 * kDwWaves, 0, st>>>(part, blocks,
+                                                                                                      (int)d, dw);
+  return check_launch("rmsnorm_dw_reduce_kernel");
+}
+
+extern "C" int moc_cast_bf16_multi(int n, const void* const* src, const int64_t* rows, const int64_t* cols,
+                                   void* const* dst, const int64_t* dst_ld, void* stream) {
+  MOC_REQUIRE(n >= 0 && n <= kCastMax, "moc_cast_bf16_multi: at most %d matrices", kCastMax);
+  CastArgs a{};
+  int64_t at = 0;
+  for (int i = 0; i < n; ++i) {
+    MOC_REQUIRE(rows[i] >= 0 && cols[i] >= 0, "moc_cast_bf16_multi: bad shape");
+    if (rows[i] == 0 || cols[i] == 0) continue;
+    MOC_REQUIRE(src[i] && dst[i] && reinterpret_cast<uintptr_t>(src[i]) % 4 == 0 && aligned16(dst[i]) &&
+                    dst_ld[i] % 8 == 0 && dst_ld[i] >= (cols[i] + 7) / 8 * 8,
+                "moc_cast_bf16_multi: dst needs 16-byte aligned rows of whole chunks of 8");
+    a.job[a.n] = {static_cast<const float*>(src[i]), static_cast<uint16_t*>(dst[i]), rows[i], cols[i], dst_ld[i]};
+    a.start[a.n++] = static_cast<int>(at);
+    at += (rows[i] * ((cols[i] + 7) / 8) + 255) / 256;
+    MOC_REQUIRE(at < (1LL << 31), "moc_cast_bf16_multi: too large");
+  }
+  if (a.n == 0) return MOC_OK;
+  a.start[a.n] = static_cast<int>(at);
+  cast_bf16_multi_kernel<<<dim3(static_cast<unsigned>(at)), 256, 0, as_stream(stream)>>>(a);
+  return check_launch("cast_bf16_multi_kernel");
 }

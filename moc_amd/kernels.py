@@ -477,6 +477,91 @@ def rmsnorm_backward(x2d: torch.Tensor, weight: torch.Tensor, rstd: torch.Tensor
     return dx, dw
 
 
+def rmsnorm_rows_f32(x2d, weight, eps: float):
+    """(y bf16, rstd f32) of an f32 [rows, d] stream with an f32 weight:
+    y = bf16(x / rms(x) * weight), rounded once (moc_rmsnorm_rows_f32)."""
+    N.require_device(x2d, weight)
+    if x2d.dtype != torch.float32 or weight.dtype != torch.float32 or not x2d.is_contiguous():
+        raise ValueError("rmsnorm_rows_f32 takes contiguous f32 rows and an f32 weight")
+    rows, d = x2d.shape
+    w = weight.contiguous()
+    y = _empty((rows, d), torch.bfloat16, x2d.device)
+    rstd = _empty((rows,), torch.float32, x2d.device)
+    N.call("moc_rmsnorm_rows_f32", x2d.data_ptr(), d, rows, d, w.data_ptr(), float(eps), y.data_ptr(), d,
+           rstd.data_ptr(), N.stream_of(x2d))
+    return y, rstd
+
+
+def rmsnorm_backward_f32(x2d, weight, rstd, dy, dres=None):
+    """(dx, dw) f32 of rmsnorm_rows_f32 from the bf16 dy, plus dres (f32)."""
+    N.require_device(x2d, weight, rstd, dy, dres)
+    rows, d = x2d.shape
+    ga = aligned_rows(dy)
+    dx = _empty((rows, d), torch.float32, x2d.device)
+    dw = _empty((d,), torch.float32, x2d.device)
+    nbytes = N.query("moc_rmsnorm_backward_workspace_size", rows, d)
+    ws = _empty((max(nbytes, 256),), torch.uint8, x2d.device)
+    r = None if dres is None else dres.contiguous()
+    N.call("moc_rmsnorm_backward_f32", x2d.data_ptr(), d, rows, d, weight.contiguous().data_ptr(),
+           rstd.data_ptr(), ga.data_ptr(), ga.stride(0) if rows > 1 else round_up(d, 8), N.ptr(r), d,
+           dx.data_ptr(), d, dw.data_ptr(), ws.data_ptr(), ws.numel(), N.stream_of(x2d))
+    return dx, dw
+
+
+def cast_bf16(*mats: torch.Tensor) -> list:
+    """bf16 copies of contiguous f32 device matrices in one launch per eight;
+    rows come 16-byte aligned (a padded view where the columns need it)."""
+    N.require_device(*mats)
+    out = []
+    for m in mats:
+        if m.dtype != torch.float32 or m.dim() != 2 or not m.is_contiguous():
+            raise ValueError("cast_bf16 takes contiguous f32 matrices")
+        c = m.shape[1]
+        out.append(_empty(m.shape, torch.bfloat16, m.device) if c % 8 == 0
+                   else padded_empty(m.shape[0], c, torch.bfloat16, m.device))
+    for i in range(0, len(mats), 8):
+        src, dst = mats[i:i + 8], out[i:i + 8]
+        n = len(src)
+        i64, vp = N.ctypes.c_int64 * n, N.ctypes.c_void_p * n
+        N.call("moc_cast_bf16_multi", n, vp(*[t.data_ptr() for t in src]), i64(*[t.shape[0] for t in src]),
+               i64(*[t.shape[1] for t in src]), vp(*[t.data_ptr() for t in dst]),
+               i64(*[t.stride(0) for t in dst]), N.stream_of(src[0]))
+    return out
+
+
+def rope_attention(qkv, batch: int, seq: int, heads: int, cos, sin, scale: float):
+    """(o, lse): causal attention of qkv [batch seq, 3 heads head_dim] with RoPE
+    on q and k (moc_rope_attention_forward_bf16)."""
+    N.require_device(qkv, cos, sin)
+    t, d3 = qkv.shape
+    head_dim = d3 // (3 * heads)
+    if t != batch * seq or qkv.dtype != torch.bfloat16 or cos.dtype != sin.dtype or \
+            cos.shape[0] < seq or cos.shape[1] != head_dim // 2 or cos.shape != sin.shape or \
+            not (cos.is_contiguous() and sin.is_contiguous()):
+        raise ValueError("rope_attention shape or dtype mismatch")
+    qkv = aligned_rows(qkv)
+    o = _empty((t, heads * head_dim), torch.bfloat16, qkv.device)
+    lse = _empty((batch, heads, seq), torch.float32, qkv.device)
+    N.call("moc_rope_attention_forward_bf16", batch, seq, heads, head_dim, qkv.data_ptr(), qkv.stride(0),
+           cos.data_ptr(), sin.data_ptr(), N.dtype_code(cos.dtype), float(scale), o.data_ptr(), lse.data_ptr(),
+           N.stream_of(qkv))
+    return o, lse
+
+
+def rope_attention_backward(qkv, batch: int, seq: int, heads: int, cos, sin, scale: float, o, lse, go):
+    """dqkv of rope_attention from go, the gradient of o."""
+    N.require_device(qkv, o, lse, go)
+    go = go.contiguous()
+    if go.shape != o.shape or go.dtype != torch.bfloat16 or not (qkv.is_contiguous() and o.is_contiguous()):
+        raise ValueError("rope_attention_backward shape or dtype mismatch")
+    dqkv = torch.empty_like(qkv)
+    delta = torch.empty_like(lse)
+    N.call("moc_rope_attention_backward_bf16", batch, seq, heads, qkv.shape[1] // (3 * heads), qkv.data_ptr(),
+           qkv.stride(0), cos.data_ptr(), sin.data_ptr(), N.dtype_code(cos.dtype), float(scale), o.data_ptr(),
+           lse.data_ptr(), go.data_ptr(), delta.data_ptr(), dqkv.data_ptr(), N.stream_of(qkv))
+    return dqkv
+
+
 def linear(x2d: torch.Tensor, weight: torch.Tensor, *, out: torch.Tensor | None = None,
            out_dtype=None) -> torch.Tensor:
     """x2d @ weight.T for an nn.Linear weight [out_features, in_features]."""

@@ -1,0 +1,161 @@
+"""The decoder block's fused attention half and its kernels (causal attention
+with RoPE, the f32-stream norm, the multi-matrix cast) against 64 bits and the
+stock composition."""
+import math
+
+import pytest
+import torch
+
+import moc_amd.block as B
+from moc_amd import MoCConfig
+from moc_amd import kernels as K
+from moc_amd.model import CausalSelfAttention, RMSNorm, TransformerBlock, rotary_tables
+
+pytestmark = pytest.mark.gpu
+BF, F32, F64 = torch.bfloat16, torch.float32, torch.float64
+
+
+def _rot(x, c, s):
+    a, b = x[..., 0::2], x[..., 1::2]
+    return torch.stack((a * c - b * s, a * s + b * c), -1).flatten(-2)
+
+
+@pytest.mark.parametrize("seq", [1, 2, 31, 33, 64, 65, 127, 129, 200, 256, 300, 513])
+@pytest.mark.parametrize("heads,dim,table", [(3, 64, BF), (2, 64, F32), (2, 128, BF)])
+def test_rope_attention(seq, heads, dim, table):
+    batch = 2
+    g = torch.Generator(device="cuda").manual_seed(seq * heads + dim)
+    t, d = batch * seq, heads * dim
+    qkv = torch.randn(t, 3 * d, generator=g, device="cuda").to(BF)
+    go = torch.randn(t, d, generator=g, device="cuda").to(BF)
+    cos, sin = (x.to("cuda", table) for x in rotary_tables(dim, seq + 3))
+    scale = 1.0 / math.sqrt(dim)
+    o, lse = K.rope_attention(qkv, batch, seq, heads, cos, sin, scale)
+    dqkv = K.rope_attention_backward(qkv, batch, seq, heads, cos, sin, scale, o, lse, go)
+    assert all(torch.equal(a, b) for a, b in zip((o, lse), K.rope_attention(qkv, batch, seq, heads, cos, sin, scale)))
+
+    c, s = cos[:seq].to(F64), sin[:seq].to(F64)
+    q, k, v = qkv.to(F64).view(batch, seq, 3, heads, dim).permute(2, 0, 3, 1, 4)
+    if table == BF:  # bf16 tensor operations: each product and the sum rounded
+        q, k = (_rot(x.to(BF), cos[:seq], sin[:seq]).to(F64) for x in (q, k))
+    else:
+        q, k = (_rot(x.float(), cos[:seq], sin[:seq]).to(BF).to(F64) for x in (q, k))
+    gg = go.to(F64).view(batch, seq, heads, dim).transpose(1, 2)
+    sc = (q @ k.transpose(-1, -2)) * scale + torch.full((seq, seq), -math.inf, device="cuda", dtype=F64).triu(1)
+    p = torch.softmax(sc, -1)
+    ref = p @ v
+    # o: its rounding, and P's to bf16 in the product
+    e8 = 2.0 ** -8
+    ob = o.to(F64).view(batch, seq, heads, dim).transpose(1, 2)
+    assert ((ob - ref).abs() <= e8 * (ref.abs() + 2 * p @ v.abs()) + 1e-5).all()
+    want = torch.logsumexp(sc, -1) / math.log(2.0)
+    assert ((lse.to(F64) - want).abs() <= 1e-5 * (1 + want.abs())).all()
+    # dS = P (dP - delta) scale; delta comes from the rounded o, dS is rounded
+    dp = gg @ v.transpose(-1, -2)
+    delta = (gg * ref).sum(-1, keepdim=True)
+    ds = p * (dp - delta)
+    ds_err = p * (e8 * (gg.abs() * (ref.abs() + 2 * p @ v.abs())).sum(-1, keepdim=True)) + 2 * e8 * ds.abs()
+    grads = {"q": (ds @ k * scale, ds_err @ k.abs() * scale),
+             "k": (ds.transpose(-1, -2) @ q * scale, ds_err.transpose(-1, -2) @ q.abs() * scale),
+             "v": (p.transpose(-1, -2) @ gg, 2 * e8 * p.transpose(-1, -2) @ gg.abs())}
+    got = dict(zip("qkv", dqkv.to(F64).view(batch, seq, 3, heads, dim).permute(2, 0, 3, 1, 4)))
+    for n, (r, err) in grads.items():
+        if n != "v":  # rotated back: each value mixes its pair
+            r = _rot(r, c, -s)
+            err = (err[..., 0::2] + err[..., 1::2]).repeat_interleave(2, -1)
+        bad = (got[n] - r).abs() > e8 * r.abs() + err + 1e-5
+        assert not bad.any(), (n, int(bad.sum()))
+
+
+def _pair(dtype, hidden, heads, seq, seed):
+    torch.manual_seed(seed)
+    cfg = MoCConfig(hidden_size=hidden, intermediate_size=2 * hidden, num_hidden_layers=1,
+                    num_attention_heads=heads, vocab_size=32, max_seq_len=max(seq, 8))
+    norm, attn = RMSNorm(hidden), CausalSelfAttention(cfg)
+    norm.weight.data += 0.1 * torch.randn(hidden)
+    return norm.to("cuda", dtype), attn.to("cuda", dtype)
+
+
+@pytest.mark.parametrize("dtype", [BF, F32])
+@pytest.mark.parametrize("batch,seq,hidden,heads", [(2, 1, 64, 1), (3, 77, 256, 4), (2, 256, 512, 8),
+                                                    (1, 130, 256, 2)])
+def test_attention_half_matches_the_stock_composition(dtype, batch, seq, hidden, heads):
+    norm, attn = _pair(dtype, hidden, heads, seq, 7)
+    ref_n, ref_a = _pair(F64, hidden, heads, seq, 7)
+    for m, r in ((norm, ref_n), (attn, ref_a)):
+        for a, b in zip(m.parameters(), r.parameters()):
+            b.data.copy_(a.data)
+    x = torch.randn(batch, seq, hidden, device="cuda").to(dtype)
+    dh = torch.randn(batch, seq, hidden, device="cuda").to(dtype)
+
+    def run(fn, n, a, xx, gg, cast):
+        xx = xx.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=BF, enabled=cast):
+            if fn is B.attention_half:
+                assert B.attention_half_ok(xx, n, RMSNorm, a, CausalSelfAttention)
+            y = fn(xx, n, a)
+        grads = torch.autograd.grad(y, [xx, n.weight, a.qkv_proj.weight, a.out_proj.weight], gg)
+        return [y - xx, *grads]
+
+    stock = lambda xx, n, a: xx + a(n(xx))  # noqa: E731
+    cast = dtype == F32
+    got = run(B.attention_half, norm, attn, x, dh, cast)
+    old = run(stock, norm, attn, x, dh, cast)
+    exact = run(stock, ref_n, ref_a, x.to(F64), dh.to(F64), False)
+    for g, o, e in zip(got, old, exact):
+        assert g.dtype == o.dtype and g.shape == o.shape
+        err = lambda t: ((t.to(F64) - e).norm() / e.norm().clamp_min(1e-12)).item()  # noqa: E731
+        # no further from 64 bits than the stock composition
+        assert err(g) <= 1.1 * err(o) + 1e-4, (err(g), err(o))
+
+
+def test_block_takes_the_fused_half_and_hooks_keep_the_stock_one():
+    cfg = MoCConfig(hidden_size=256, intermediate_size=512, num_hidden_layers=1, num_attention_heads=4, vocab_size=32)
+    blk = TransformerBlock(cfg, "moc").to("cuda", BF)
+    x = torch.randn(2, 40, 256, device="cuda").to(BF)
+    calls = []
+    blk.attn.register_forward_hook(lambda *a: calls.append(1))
+    y1 = blk(x)
+    assert calls
+    blk.attn._forward_hooks.clear()
+    y2 = blk(x)
+    assert len(calls) == 1
+    assert (y1.float() - y2.float()).norm() <= 2e-2 * y1.float().norm()
+    from torch.utils.checkpoint import checkpoint
+    xs = [x.clone().requires_grad_() for _ in range(2)]
+    blk(xs[0]).sum().backward()
+    g0 = [p.grad.clone() for p in blk.parameters()]
+    blk.zero_grad()
+    checkpoint(blk, xs[1], use_reentrant=False).sum().backward()
+    assert torch.equal(xs[0].grad, xs[1].grad)
+    assert all(torch.equal(a, p.grad) for a, p in zip(g0, blk.parameters()))
+
+
+@pytest.mark.parametrize("rows,d", [(1, 8), (5, 64), (37, 520), (300, 1024), (9, 4096)])
+def test_rmsnorm_f32(rows, d):
+    g = torch.Generator(device="cuda").manual_seed(rows + d)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    x, w, dres, dy = r(rows, d), 1 + 0.1 * r(d), r(rows, d), r(rows, d).to(BF)
+    y, rstd = K.rmsnorm_rows_f32(x, w, 1e-6)
+    xd, wd = x.to(F64).requires_grad_(), w.to(F64).requires_grad_()
+    ref = xd * torch.rsqrt(xd.square().mean(-1, keepdim=True) + 1e-6) * wd
+    assert ((y.to(F64) - ref).abs() <= (2.0 ** -8 + 1e-5) * ref.abs()).all()
+    dx, dw = K.rmsnorm_backward_f32(x, w, rstd, dy, dres)
+    gx, gw = torch.autograd.grad(ref, [xd, wd], dy.to(F64))
+    gx = gx + dres.to(F64)
+    n = xd.detach() * rstd.to(F64)[:, None]
+    # f32 sums: d (rows) terms of the products' magnitudes
+    mag = dres.abs().to(F64) + (dy.to(F64) * wd * rstd.to(F64)[:, None]).abs() * (1 + n.abs())
+    assert ((dx.to(F64) - gx).abs() <= 1e-6 * (d ** 0.5) * mag + 1e-6).all()
+    assert ((dw.to(F64) - gw).abs() <= 1e-5 * (dy.to(F64) * n).abs().sum(0) + 1e-6).all()
+
+
+def test_cast_bf16():
+    g = torch.Generator(device="cuda").manual_seed(3)
+    mats = [torch.randn(r, c, generator=g, device="cuda") for r, c in
+            ((1, 1), (3, 7), (64, 64), (5, 1001), (2048, 5461), (33, 8), (10, 12), (7, 4), (128, 100), (2, 3))]
+    mats[2][0, :4] = torch.tensor([float("nan"), float("inf"), -float("inf"), -0.0])
+    for m, c in zip(mats, K.cast_bf16(*mats)):
+        assert c.stride(0) % 8 == 0 and c.data_ptr() % 16 == 0
+        assert torch.equal(c.contiguous().view(torch.int16), m.to(BF).view(torch.int16))
+
