@@ -393,9 +393,14 @@ def _autocast_dtype(x):
 
 
 def _in_compute_dtype(cdt, *ts):
-    """ts cast to the compute dtype (temporaries; None: unchanged)."""
+    """ts cast to the compute dtype (temporaries; None: unchanged).  f32 to
+    bf16, the usual autocast, is one launch for all of them."""
     if cdt is None:
         return ts
+    if cdt == torch.bfloat16 and all(t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() and t.dim() >= 2
+                                     and t.numel() > 0 for t in ts):
+        mats = [t.detach().reshape(-1, t.shape[-1]) for t in ts]
+        return tuple(c if c.dim() == t.dim() else c.reshape(t.shape) for c, t in zip(K.cast_bf16(*mats), ts))
     return tuple(t if t.dtype == cdt else t.to(cdt) for t in ts)
 
 
@@ -568,10 +573,27 @@ def block_ffn_ok(h, norm_weight, ffn) -> bool:
                (ffn.gate_proj.weight, ffn.up_proj.weight, ffn.down_proj.weight))
 
 
+def block_ffn_f32_ok(h, norm_weight, ffn) -> bool:
+    """True if block_ffn takes this block in its f32-stream form: an f32 model
+    under bf16 autocast, otherwise as block_ffn_ok."""
+    if not FUSE_BLOCK_FFN or not isinstance(ffn, MoCSwiGLUFFN) or ffn.mode not in _SELECTION_OF_MODE:
+        return False
+    d = h.shape[-1]
+    if not h.is_cuda or _autocast_dtype(h) != torch.bfloat16 or d % 8 or d > 4096 or h.numel() == 0:
+        return False
+    return all(t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in
+               (h, norm_weight, ffn.gate_proj.weight, ffn.up_proj.weight, ffn.down_proj.weight))
+
+
 def block_ffn(h, norm_weight, eps: float, ffn) -> torch.Tensor:
     """h + ffn(RMSNorm(h)) with the norm (weight norm_weight, eps) and the
-    residual fused around the MoC FFN `ffn` (block_ffn_ok must hold)."""
+    residual fused around the MoC FFN `ffn` (block_ffn_ok or block_ffn_f32_ok
+    must hold)."""
     selection, gcp = _SELECTION_OF_MODE[ffn.mode]
+    if h.dtype == torch.float32:
+        return _MoCBlockF32Function.apply(h, norm_weight, ffn.gate_proj.weight, ffn.up_proj.weight,
+                                          ffn.down_proj.weight, float(eps), ffn.k, ffn.index_save_dtype,
+                                          ffn.mode.endswith("_triton_aux"), selection, gcp)
     return _MoCBlockFunction.apply(h, norm_weight, ffn.gate_proj.weight, ffn.up_proj.weight,
                                    ffn.down_proj.weight, float(eps), ffn.k, ffn.index_save_dtype,
                                    ffn.mode.endswith("_triton_aux"), selection, gcp)
@@ -638,6 +660,49 @@ class _MoCBlockFunction(torch.autograd.Function):
             del xn
             dh, dnw = K.rmsnorm_backward(h2, norm_w, rstd, dxn.reshape(-1, d), dres=go)
         return (dh.reshape(ctx.h_shape), dnw, dwg, dwu, dwd, None, None, None, None, None, None)
+
+
+class _MoCBlockF32Function(torch.autograd.Function):
+    """The FFN half over an f32 residual stream with f32 parameters under bf16
+    autocast: the norm writes the FFN's bf16 input at once (the stock module
+    stores three f32 tensors and a cast on the way), the weights are cast in
+    one launch per pass, the residual sum and the norm's backward stay f32."""
+
+    @staticmethod
+    def forward(ctx, h, norm_w, gate_w, up_w, down_w, eps, k, index_save_dtype, use_triton_aux, selection, gcp):
+        d = h.shape[-1]
+        inter = gate_w.shape[0]
+        h2 = h.reshape(-1, d)
+        xn, rstd = K.rmsnorm_rows_f32(h2, norm_w, eps)
+        wg, wu, wd = K.cast_bf16(gate_w, up_w, down_w)
+        _check_inputs(xn, wg, wu, wd, use_triton_aux, index_save_dtype)
+        bitmask = index_save_dtype == INDEX_SAVE_BITMASK
+        out, idx, vals, u_s, s_s, z_s, *mask = _forward_common(
+            xn, wg, wu, wd, k, selection, _pack_topk_idx_dtype(index_save_dtype, inter), save_s=not gcp,
+            want_mask=bitmask)
+        sel = _saved_index(idx, mask[0] if mask else None, bitmask)
+        # the parameters, not their casts: the backward casts them again
+        if gcp:
+            ctx.save_for_backward(h2, xn, rstd, norm_w, sel, vals, u_s, gate_w, up_w, down_w)
+        else:
+            ctx.save_for_backward(h2, xn, rstd, norm_w, sel, vals, u_s, s_s, z_s, gate_w, up_w, down_w)
+        ctx.k, ctx.inter, ctx.bitmask, ctx.gcp, ctx.h_shape = idx.shape[-1], inter, bitmask, gcp, h.shape
+        return (h2 + out).reshape(h.shape)
+
+    @staticmethod
+    def backward(ctx, dout):
+        if ctx.gcp:
+            h2, xn, rstd, norm_w, saved, g_s, u_s, gate_w, up_w, down_w = ctx.saved_tensors
+            s_s = z_s = None
+        else:
+            h2, xn, rstd, norm_w, saved, g_s, u_s, s_s, z_s, gate_w, up_w, down_w = ctx.saved_tensors
+        idx = _restore_index(ctx, saved)
+        wg, wu, wd = K.cast_bf16(gate_w, up_w, down_w)
+        d2 = dout.reshape(h2.shape).contiguous()
+        dxn, dwg, dwu, dwd = _backward_common(d2.to(torch.bfloat16), xn, idx, g_s, u_s, s_s, z_s, wg, wu, wd,
+                                              gcp=ctx.gcp, grad_dtype=gate_w.dtype)
+        dh, dnw = K.rmsnorm_backward_f32(h2, norm_w, rstd, dxn, dres=d2)
+        return dh.reshape(ctx.h_shape), dnw, dwg, dwu, dwd, None, None, None, None, None, None
 
 
 def _block_forward_native(h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s):

@@ -159,3 +159,30 @@ def test_cast_bf16():
         assert c.stride(0) % 8 == 0 and c.data_ptr() % 16 == 0
         assert torch.equal(c.contiguous().view(torch.int16), m.to(BF).view(torch.int16))
 
+
+@pytest.mark.parametrize("ffn_type", ["moc", "moc_gcp", "moc_2_8", "moc_post_silu_abs"])
+@pytest.mark.parametrize("inter", [320, 333])
+def test_ffn_half_under_autocast_matches_the_stock_composition(ffn_type, inter):
+    """h + ffn(norm(h)) of an f32 block under autocast: the norm's output, so
+    the FFN's bf16 input, is the stock one but for f32 sums in another order."""
+    import moc_amd.ffn as FF
+    torch.manual_seed(3)
+    cfg = MoCConfig(hidden_size=128, intermediate_size=inter, num_hidden_layers=1, num_attention_heads=2, vocab_size=32)
+    blk = TransformerBlock(cfg, ffn_type).to("cuda")
+    h = torch.randn(3, 50, 128, device="cuda")
+    dy = torch.randn_like(h)
+
+    def run(fused):
+        x = h.clone().requires_grad_()
+        with torch.autocast("cuda", dtype=BF):
+            if fused:
+                assert FF.block_ffn_f32_ok(x, blk.ffn_norm.weight, blk.ffn)
+                y = FF.block_ffn(x, blk.ffn_norm.weight, blk.ffn_norm.eps, blk.ffn)
+            else:
+                y = x + blk.ffn(blk.ffn_norm(x))
+        ps = [blk.ffn_norm.weight, *blk.ffn.parameters()]
+        return [y - x, *torch.autograd.grad(y, [x, *ps], dy)]
+
+    for a, b in zip(run(True), run(False)):
+        assert a.dtype == b.dtype == F32 and a.shape == b.shape
+        assert (a - b).norm() <= 5e-3 * b.norm()
