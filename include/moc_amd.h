@@ -238,6 +238,65 @@ int moc_ffn_infer_bf16(int64_t rows, int64_t d, int64_t inter, int64_t k, int se
                        const void* res, int64_t ldres, void* y, int64_t ldy, void* scratch,
                        int64_t scratch_bytes, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The attention half of a decoder block, h = x + out_proj(attention(RoPE(
+ * qkv_proj(RMSNorm(x))))) (moc/model.py:31-64,83-84), one call per pass, bit for
+ * bit the separate entry points in order.  f32 = 0: x, dh, h, dx, the weights
+ * and their gradients bf16 and cos/sin bf16; f32 = 1: all of these f32 (a model
+ * with f32 parameters under bf16 autocast), the products' operands cast to
+ * bf16.  batch seq >= 2, heads of 64 or 128, hidden up to 4096; contiguous,
+ * 16-byte aligned.  saved: written by the forward, read by the backward
+ * (moc_attention_half_saved_size); y_tmp [tokens, hidden] bf16 (f32 = 1);
+ * scratch: no contents kept; workspace: as moc_gemm_ws uses it. */
+int64_t moc_attention_half_saved_size(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim, int f32);
+int64_t moc_attention_half_scratch_size(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim, int f32);
+int64_t moc_attention_half_workspace_size(int64_t tokens, int64_t d);
+int moc_attention_half_forward(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim, int f32,
+                               const void* x, const void* norm_w, float eps, const void* w_qkv,
+                               const void* w_out, const void* cos, const void* sin, float scale, void* h,
+                               void* saved, int64_t saved_bytes, void* y_tmp, void* workspace,
+                               int64_t workspace_bytes, void* stream);
+int moc_attention_half_backward(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim, int f32,
+                                const void* dh, const void* x, const void* norm_w, const void* w_qkv,
+                                const void* w_out, const void* cos, const void* sin, float scale,
+                                const void* saved, int64_t saved_bytes, void* dx, void* dnorm_w,
+                                void* dw_qkv, void* dw_out, void* scratch, int64_t scratch_bytes,
+                                void* workspace, int64_t workspace_bytes, void* stream);
+
+/* The FFN half h + FFN(RMSNorm(h)) over an f32 stream with f32 weights under
+ * bf16 autocast, one call per pass: moc_cast_bf16_multi of the weights (and of
+ * dout), moc_rmsnorm_rows_f32, the launches of moc_ffn_forward_bf16 /
+ * moc_ffn_backward_bf16, the residual in f32.  Contiguous operands, inter a
+ * multiple of 8; cast: moc_ffn_block_f32_cast_size bytes of scratch; dxn [rows,
+ * d] bf16 scratch; the other arguments and the workspaces as in the bf16 block
+ * entries (moc_ffn_forward_workspace_size, moc_ffn_block_backward_workspace_size). */
+int64_t moc_ffn_block_f32_cast_size(int64_t rows, int64_t d, int64_t inter);
+int moc_ffn_block_forward_f32(int64_t rows, int64_t d, int64_t inter, int64_t k, int selection,
+                              const float* h, const float* norm_w, float eps, void* xn, float* rstd,
+                              const float* wg, const float* wu, const float* wd, void* cast,
+                              int64_t cast_bytes, void* g, void* u, int64_t ld_gu, void* vals, void* idx,
+                              int idx_dtype, void* u_s, void* s_s, void* z_s, float* out, void* workspace,
+                              int64_t workspace_bytes, void* stream);
+int moc_ffn_block_backward_f32(int64_t rows, int64_t d, int64_t inter, int64_t k, const float* dout,
+                               const float* h, const float* norm_w, const float* rstd, const void* xn,
+                               const void* idx, int idx_dtype, const void* g_s, const void* u_s,
+                               const void* s_s, const void* z_s, const float* wg, const float* wu,
+                               const float* wd, void* cast, int64_t cast_bytes, void* zbuf, int64_t ldz,
+                               void* gg, void* gu, int64_t ld_ggu, int stacked, void* dxn, float* dh,
+                               float* dwg, float* dwu, float* dwd, float* dnorm_w, void* workspace,
+                               int64_t workspace_bytes, void* stream);
+
+/* The f32 layer's backward, one call: the launches of the separate entry
+ * points in their order.  Contiguous operands, d and inter multiples of 4;
+ * zbuf, gg, gu [rows, pitch]; s_s and z_s NULL: recomputed (GCP) into s_tmp,
+ * z_tmp [rows, k]. */
+int64_t moc_ffn_backward_f32_workspace_size(int64_t rows, int64_t d, int64_t inter);
+int moc_ffn_backward_f32(int64_t rows, int64_t d, int64_t inter, int64_t k, const float* go,
+                         const float* x, const void* idx, int idx_dtype, const float* g_s,
+                         const float* u_s, const float* s_s, const float* z_s, float* s_tmp, float* z_tmp,
+                         const float* wg, const float* wu, const float* wd, float* zbuf, float* gg,
+                         float* gu, int64_t pitch, float* dx, float* dwg, float* dwu, float* dwd,
+                         void* workspace, int64_t workspace_bytes, void* stream);
+
 /* GEMM workspace bytes of moc_ffn_forward_bf16 (0: none). */
 int64_t moc_ffn_forward_workspace_size(int64_t rows, int64_t d, int64_t inter);
 

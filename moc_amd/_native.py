@@ -76,6 +76,24 @@ SIGNATURES: dict[str, tuple] = {
                                            _int, _vp, _i64, _vp]),
     "moc_decode_block_bf16": (_int, [_vp, _i64, _i64, _vp, ctypes.c_float, _vp, _vp, _i64, _vp, _i64, _i64,
                                      _int, _vp, _vp, _i64, _vp]),
+    "moc_attention_half_saved_size": (_i64, [_i64, _i64, _i64, _i64, _int]),
+    "moc_attention_half_scratch_size": (_i64, [_i64, _i64, _i64, _i64, _int]),
+    "moc_attention_half_workspace_size": (_i64, [_i64, _i64]),
+    "moc_attention_half_forward": (_int, [_i64, _i64, _i64, _i64, _int, _vp, _vp, ctypes.c_float, _vp, _vp, _vp,
+                                          _vp, ctypes.c_float, _vp, _vp, _i64, _vp, _vp, _i64, _vp]),
+    "moc_attention_half_backward": (_int, [_i64, _i64, _i64, _i64, _int, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                                           ctypes.c_float, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64,
+                                           _vp]),
+    "moc_ffn_block_f32_cast_size": (_i64, [_i64, _i64, _i64]),
+    "moc_ffn_block_forward_f32": (_int, [_i64, _i64, _i64, _i64, _int, _vp, _vp, ctypes.c_float, _vp, _vp, _vp,
+                                         _vp, _vp, _vp, _i64, _vp, _vp, _i64, _vp, _vp, _int, _vp, _vp, _vp, _vp,
+                                         _vp, _i64, _vp]),
+    "moc_ffn_block_backward_f32": (_int, [_i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _int, _vp, _vp,
+                                          _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _i64, _int,
+                                          _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
+    "moc_ffn_backward_f32_workspace_size": (_i64, [_i64, _i64, _i64]),
+    "moc_ffn_backward_f32": (_int, [_i64, _i64, _i64, _i64, _vp, _vp, _vp, _int, _vp, _vp, _vp, _vp, _vp, _vp,
+                                    _vp, _vp, _vp, _vp, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
     "moc_rmsnorm_rows_f32": (_int, [_vp, _i64, _i64, _i64, _vp, ctypes.c_float, _vp, _i64, _vp, _vp]),
     "moc_rmsnorm_backward_f32": (_int, [_vp, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _i64,
                                         _vp, _vp, _i64, _vp]),

@@ -12,10 +12,12 @@ attention output, out_proj's output), f32 in between.
 from __future__ import annotations
 
 import math
+from functools import lru_cache
 
 import torch
 import torch.nn as nn
 
+from . import _native as N
 from . import kernels as K
 
 BF16, F32 = torch.bfloat16, torch.float32
@@ -55,6 +57,8 @@ def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:
     if attn.head_dim not in (64, 128) or d != attn.num_heads * attn.head_dim or d > 4096 or x.numel() < 2 * d or \
             x.shape[1] > attn.rope_cos.shape[0] or x.shape[0] > 65535:
         return False
+    if x.is_contiguous() and x.data_ptr() % 16:
+        return False
     return all(t.dtype == dt and t.is_contiguous() and t.device == x.device and t.data_ptr() % 16 == 0
                for t in (norm.weight, qkv.weight, out.weight, attn.rope_cos, attn.rope_sin))
 
@@ -65,44 +69,54 @@ def attention_half(x, norm, attn) -> torch.Tensor:
                                 attn.rope_sin, float(norm.eps), attn.num_heads)
 
 
+@lru_cache(maxsize=256)
+def _sizes(device_index: int, batch: int, seq: int, heads: int, head_dim: int, f32: int):
+    """(saved buffer, backward scratch, GEMM workspace) bytes of a shape."""
+    return (N.query("moc_attention_half_saved_size", batch, seq, heads, head_dim, f32),
+            N.query("moc_attention_half_scratch_size", batch, seq, heads, head_dim, f32),
+            N.query("moc_attention_half_workspace_size", batch * seq, heads * head_dim))
+
+
 class _AttentionHalf(torch.autograd.Function):
+    """One native call per pass; between them one buffer of the forward's
+    results (norm output, q/k/v, attention output, row factors and, under
+    autocast, the weights' casts, which autocast keeps too)."""
+
     @staticmethod
     def forward(ctx, x, norm_w, qkv_w, out_w, cos, sin, eps, heads):
         batch, seq, d = x.shape
-        x2 = x.reshape(-1, d).contiguous()
+        x = x.contiguous()
+        f32 = int(x.dtype == F32)
+        dev = x.device
+        nsaved, _, nws = _sizes(dev.index, batch, seq, heads, d // heads, f32)
+        saved = torch.empty(nsaved, dtype=torch.uint8, device=dev)
+        h = torch.empty_like(x)
+        y = torch.empty((batch * seq, d), dtype=BF16, device=dev) if f32 else None
+        ws = K._gemm_workspace(dev, nws) if nws > 0 else None
         scale = 1.0 / math.sqrt(d // heads)
-        if x.dtype == F32:
-            wq, wo = K.cast_bf16(qkv_w, out_w)
-            xn, rstd = K.rmsnorm_rows_f32(x2, norm_w, eps)
-        else:
-            wq, wo = qkv_w, out_w
-            xn, rstd = K.rmsnorm_rows(x2, norm_w, eps)
-        qkv = K.linear(xn, wq)
-        o, lse = K.rope_attention(qkv, batch, seq, heads, cos, sin, scale)
-        if x.dtype == F32:
-            h = x2 + K.linear(o, wo)
-        else:
-            h = K.gemm(o, wo.t(), residual=x2)
-        # under autocast the casts are kept for the backward, as autocast keeps them
-        ctx.save_for_backward(x2, rstd, norm_w, xn, qkv, o, lse, wq, wo, cos, sin)
-        ctx.shape, ctx.heads, ctx.scale = x.shape, heads, scale
-        ctx.grad_dtype = qkv_w.dtype
-        return h.reshape(x.shape)
+        N.call("moc_attention_half_forward", batch, seq, heads, d // heads, f32, x.data_ptr(), norm_w.data_ptr(),
+               eps, qkv_w.data_ptr(), out_w.data_ptr(), cos.data_ptr(), sin.data_ptr(), scale, h.data_ptr(),
+               saved.data_ptr(), nsaved, N.ptr(y), N.ptr(ws), nws, N.stream_of(x))
+        ctx.save_for_backward(x, norm_w, qkv_w, out_w, cos, sin, saved)
+        ctx.heads, ctx.scale = heads, scale
+        return h
 
     @staticmethod
     def backward(ctx, dh):
-        x2, rstd, norm_w, xn, qkv, o, lse, wq, wo, cos, sin = ctx.saved_tensors
-        batch, seq, d = ctx.shape
-        dh2 = dh.reshape(-1, d).contiguous()
-        go = K.aligned_rows(dh2.to(BF16))
-        gdt = ctx.grad_dtype
-        d_out = K.gemm(go.t(), o, out_dtype=gdt)
-        do = K.gemm(go, wo)
-        dqkv = K.rope_attention_backward(qkv, batch, seq, ctx.heads, cos, sin, ctx.scale, o, lse, do)
-        d_qkv = K.gemm(dqkv.t(), xn, out_dtype=gdt)
-        dxn = K.gemm(dqkv, wq)
-        if x2.dtype == F32:
-            dx, dn = K.rmsnorm_backward_f32(x2, norm_w, rstd, dxn, dres=dh2)
-        else:
-            dx, dn = K.rmsnorm_backward(x2, norm_w, rstd, dxn, dres=go)
-        return dx.reshape(ctx.shape), dn, d_qkv, d_out, None, None, None, None
+        x, norm_w, qkv_w, out_w, cos, sin, saved = ctx.saved_tensors
+        batch, seq, d = x.shape
+        heads = ctx.heads
+        f32 = int(x.dtype == F32)
+        dev = x.device
+        _, nscratch, nws = _sizes(dev.index, batch, seq, heads, d // heads, f32)
+        dh = dh.to(x.dtype).contiguous()
+        if dh.data_ptr() % 16:
+            dh = dh.clone()
+        scratch = torch.empty(nscratch, dtype=torch.uint8, device=dev)
+        ws = K._gemm_workspace(dev, nws) if nws > 0 else None
+        dx, dn, dq, do = (torch.empty_like(t) for t in (x, norm_w, qkv_w, out_w))
+        N.call("moc_attention_half_backward", batch, seq, heads, d // heads, f32, dh.data_ptr(), x.data_ptr(),
+               norm_w.data_ptr(), qkv_w.data_ptr(), out_w.data_ptr(), cos.data_ptr(), sin.data_ptr(), ctx.scale,
+               saved.data_ptr(), saved.numel(), dx.data_ptr(), dn.data_ptr(), dq.data_ptr(), do.data_ptr(),
+               scratch.data_ptr(), nscratch, N.ptr(ws), nws, N.stream_of(x))
+        return dx, dn, dq, do, None, None, None, None

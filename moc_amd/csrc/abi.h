@@ -46,6 +46,10 @@ int launch_gate_up_2of8(const void* x, int64_t nb, int64_t hidden, const void* w
                         int64_t inter, int64_t* idx, uint16_t* sz, hipStream_t st, uint16_t* ap = nullptr,
                         int64_t ld_ap = 0, uint32_t* meta = nullptr, int64_t meta_rows = 0);
 
+// out = x + y over n values (a multiple of 8), x and out f32, y bf16
+// (rmsnorm.hip).
+int add_f32_bf16(const float* x, const void* y, float* out, int64_t n, hipStream_t st);
+
 // MoC 2:8: the dense Z of G's and U's rows (pitch ld, a multiple of 8, 16-byte
 // aligned; inter a multiple of 8) in G's place: z of the top 2 of every 8
 // channels, zeros for the rest (moc28.hip).

@@ -396,3 +396,318 @@ extern "C" int moc_ffn_block_backward_bf16(int64_t rows, int64_t d, int64_t inte
   return moc_rmsnorm_backward_bf16(h, ldh, rows, d, norm_w, rstd, xn, ldxn, dout, ldgo, dh, lddh, dnorm_w,
                                    dnorm_dtype, static_cast<char*>(workspace) + f, workspace_bytes - f, stream);
 }
+
+// ---------------------------------------------------------------------------
+// The attention half of a block, x + out_proj(attention(RMSNorm(x)))
+// (moc/model.py:31-64,83-84), as one call per pass, for a bf16 stream with
+// bf16 weights or an f32 stream with f32 weights (bf16 autocast: the weights
+// are cast here, one launch).  What the backward needs beyond x lives in one
+// caller buffer, laid out here.
+
+namespace {
+struct AttnHalf {
+  int64_t t, d, heads;
+  // saved by the forward
+  int64_t xn, qkv, o, rstd, lse, wq, wo, saved;
+  // scratch of the backward: go (f32 stream), do / dxn, dqkv, delta, norm partials
+  int64_t go, dox, dqkv, delta, rms, scratch;
+};
+AttnHalf attn_half(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim, int f32) {
+  auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
+  AttnHalf a{};
+  a.t = batch * seq;
+  a.d = heads * head_dim;
+  a.heads = heads;
+  int64_t p = 0;
+  auto take = [&](int64_t bytes) {
+    const int64_t at = p;
+    p += up(bytes);
+    return at;
+  };
+  a.xn = take(a.t * a.d * 2);
+  a.qkv = take(a.t * a.d * 6);
+  a.o = take(a.t * a.d * 2);
+  a.rstd = take(a.t * 4);
+  a.lse = take(a.t * heads * 4);
+  a.wq = take(f32 ? a.d * a.d * 6 : 0);
+  a.wo = take(f32 ? a.d * a.d * 2 : 0);
+  a.saved = p;
+  p = 0;
+  a.go = take(f32 ? a.t * a.d * 2 : 0);
+  a.dox = take(a.t * a.d * 2);
+  a.dqkv = take(a.t * a.d * 6);
+  a.delta = take(a.t * heads * 4);
+  a.rms = take(moc_rmsnorm_backward_workspace_size(a.t, a.d));
+  a.scratch = p;
+  return a;
+}
+bool attn_half_shape(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim) {
+  return batch >= 1 && seq >= 1 && batch * seq >= 2 && heads >= 1 && (head_dim == 64 || head_dim == 128) &&
+         heads * head_dim <= 4096 && batch * seq < (1LL << 31);
+}
+}  // namespace
+
+extern "C" int64_t moc_attention_half_saved_size(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim, int f32) {
+  return attn_half_shape(batch, seq, heads, head_dim) ? attn_half(batch, seq, heads, head_dim, f32).saved : 0;
+}
+extern "C" int64_t moc_attention_half_scratch_size(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim,
+                                                   int f32) {
+  return attn_half_shape(batch, seq, heads, head_dim) ? attn_half(batch, seq, heads, head_dim, f32).scratch : 0;
+}
+extern "C" int64_t moc_attention_half_workspace_size(int64_t tokens, int64_t d) {
+  if (tokens <= 0 || d <= 0) return 0;
+  return std::max({gemm_ws(tokens, 3 * d, d, 0), gemm_ws(tokens, d, d, 0), gemm_ws(d, d, tokens, 0),
+                   gemm_ws(3 * d, d, tokens, 0), gemm_ws(tokens, d, 3 * d, 0)});
+}
+
+extern "C" int moc_attention_half_forward(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim, int f32,
+                                          const void* x, const void* norm_w, float eps, const void* w_qkv,
+                                          const void* w_out, const void* cos, const void* sin, float scale, void* h,
+                                          void* saved, int64_t saved_bytes, void* y_tmp, void* workspace,
+                                          int64_t workspace_bytes, void* stream) {
+  MOC_REQUIRE(attn_half_shape(batch, seq, heads, head_dim),
+              "moc_attention_half_forward: two tokens or more, heads of 64 or 128, hidden up to 4096");
+  const AttnHalf a = attn_half(batch, seq, heads, head_dim, f32);
+  const int64_t t = a.t, d = a.d;
+  MOC_REQUIRE(x && norm_w && w_qkv && w_out && h && saved && (!f32 || y_tmp),
+              "moc_attention_half_forward: null pointer");
+  MOC_REQUIRE(moc::aligned16(x) && moc::aligned16(w_qkv) && moc::aligned16(w_out) && moc::aligned16(h) &&
+                  moc::aligned16(saved) && moc::aligned16(y_tmp),
+              "moc_attention_half_forward: operands must be 16-byte aligned");
+  MOC_REQUIRE(saved_bytes >= a.saved, "moc_attention_half_forward: buffer of %lld bytes required", (long long)a.saved);
+  const int64_t need = moc_attention_half_workspace_size(t, d);
+  MOC_REQUIRE(workspace_bytes >= need && (need == 0 || workspace != nullptr),
+              "moc_attention_half_forward: workspace of %lld bytes required", (long long)need);
+  char* b = static_cast<char*>(saved);
+  void *xn = b + a.xn, *qkv = b + a.qkv, *o = b + a.o;
+  float *rstd = reinterpret_cast<float*>(b + a.rstd), *lse = reinterpret_cast<float*>(b + a.lse);
+  const void *wq = w_qkv, *wo = w_out;
+  int rc;
+  if (f32) {
+    const void* src[2] = {w_qkv, w_out};
+    void* dst[2] = {b + a.wq, b + a.wo};
+    const int64_t rows[2] = {3 * d, d}, cols[2] = {d, d};
+    rc = moc_cast_bf16_multi(2, src, rows, cols, dst, cols, stream);
+    if (rc != MOC_OK) return rc;
+    wq = dst[0];
+    wo = dst[1];
+    rc = moc_rmsnorm_rows_f32(static_cast<const float*>(x), d, t, d, static_cast<const float*>(norm_w), eps, xn, d,
+                              rstd, stream);
+  } else {
+    rc = moc_rmsnorm_rows_bf16(x, d, t, d, norm_w, eps, xn, d, rstd, stream);
+  }
+  if (rc != MOC_OK) return rc;
+  rc = moc_gemm_ws(MOC_BF16, t, 3 * d, d, xn, d, 1, wq, 1, d, 0, nullptr, 0, 0, nullptr, 0, 0, qkv, 3 * d, MOC_BF16,
+                   workspace, workspace_bytes, stream);
+  if (rc != MOC_OK) return rc;
+  rc = moc_rope_attention_forward_bf16(batch, seq, heads, head_dim, qkv, 3 * d, cos, sin, f32 ? MOC_F32 : MOC_BF16,
+                                       scale, o, lse, stream);
+  if (rc != MOC_OK) return rc;
+  if (!f32)
+    return moc_gemm_residual_bf16(t, d, d, o, d, 1, wo, 1, d, h, d, x, d, workspace, workspace_bytes, stream);
+  rc = moc_gemm_ws(MOC_BF16, t, d, d, o, d, 1, wo, 1, d, 0, nullptr, 0, 0, nullptr, 0, 0, y_tmp, d, MOC_BF16,
+                   workspace, workspace_bytes, stream);
+  if (rc != MOC_OK) return rc;
+  return moc::add_f32_bf16(static_cast<const float*>(x), y_tmp, static_cast<float*>(h), t * d,
+                           moc::as_stream(stream));
+}
+
+extern "C" int moc_attention_half_backward(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim, int f32,
+                                           const void* dh, const void* x, const void* norm_w, const void* w_qkv,
+                                           const void* w_out, const void* cos, const void* sin, float scale,
+                                           const void* saved, int64_t saved_bytes, void* dx, void* dnorm_w,
+                                           void* dw_qkv, void* dw_out, void* scratch, int64_t scratch_bytes,
+                                           void* workspace, int64_t workspace_bytes, void* stream) {
+  MOC_REQUIRE(attn_half_shape(batch, seq, heads, head_dim),
+              "moc_attention_half_backward: two tokens or more, heads of 64 or 128, hidden up to 4096");
+  const AttnHalf a = attn_half(batch, seq, heads, head_dim, f32);
+  const int64_t t = a.t, d = a.d;
+  MOC_REQUIRE(dh && x && norm_w && w_qkv && w_out && saved && dx && dnorm_w && dw_qkv && dw_out && scratch,
+              "moc_attention_half_backward: null pointer");
+  MOC_REQUIRE(moc::aligned16(dh) && moc::aligned16(x) && moc::aligned16(w_qkv) && moc::aligned16(w_out) &&
+                  moc::aligned16(saved) && moc::aligned16(dx) && moc::aligned16(scratch),
+              "moc_attention_half_backward: operands must be 16-byte aligned");
+  MOC_REQUIRE(saved_bytes >= a.saved && scratch_bytes >= a.scratch,
+              "moc_attention_half_backward: buffers of %lld and %lld bytes required", (long long)a.saved,
+              (long long)a.scratch);
+  const int64_t need = moc_attention_half_workspace_size(t, d);
+  MOC_REQUIRE(workspace_bytes >= need && (need == 0 || workspace != nullptr),
+              "moc_attention_half_backward: workspace of %lld bytes required", (long long)need);
+  const char* b = static_cast<const char*>(saved);
+  char* s = static_cast<char*>(scratch);
+  const void *xn = b + a.xn, *qkv = b + a.qkv, *o = b + a.o;
+  const float *rstd = reinterpret_cast<const float*>(b + a.rstd), *lse = reinterpret_cast<const float*>(b + a.lse);
+  const void *wq = f32 ? b + a.wq : w_qkv, *wo = f32 ? b + a.wo : w_out, *go = dh;
+  void *dox = s + a.dox, *dqkv = s + a.dqkv;
+  const int gdt = f32 ? MOC_F32 : MOC_BF16;
+  int rc;
+  if (f32) {
+    const void* src[1] = {dh};
+    void* dst[1] = {s + a.go};
+    rc = moc_cast_bf16_multi(1, src, &t, &d, dst, &d, stream);
+    if (rc != MOC_OK) return rc;
+    go = dst[0];
+  }
+  // dW_out = go^T o, do = go W_out
+  rc = moc_gemm_ws(MOC_BF16, d, d, t, go, 1, d, o, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dw_out, d, gdt, workspace,
+                   workspace_bytes, stream);
+  if (rc == MOC_OK)
+    rc = moc_gemm_ws(MOC_BF16, t, d, d, go, d, 1, wo, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dox, d, MOC_BF16,
+                     workspace, workspace_bytes, stream);
+  if (rc == MOC_OK)
+    rc = moc_rope_attention_backward_bf16(batch, seq, heads, head_dim, qkv, 3 * d, cos, sin, gdt, scale, o, lse, dox,
+                                          reinterpret_cast<float*>(s + a.delta), dqkv, stream);
+  // dW_qkv = dqkv^T xn, dxn = dqkv W_qkv (in do's place)
+  if (rc == MOC_OK)
+    rc = moc_gemm_ws(MOC_BF16, 3 * d, d, t, dqkv, 1, 3 * d, xn, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dw_qkv, d, gdt,
+                     workspace, workspace_bytes, stream);
+  if (rc == MOC_OK)
+    rc = moc_gemm_ws(MOC_BF16, t, d, 3 * d, dqkv, 3 * d, 1, wq, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dox, d,
+                     MOC_BF16, workspace, workspace_bytes, stream);
+  if (rc != MOC_OK) return rc;
+  void* part = s + a.rms;
+  const int64_t pbytes = a.scratch - a.rms;
+  if (f32)
+    return moc_rmsnorm_backward_f32(static_cast<const float*>(x), d, t, d, static_cast<const float*>(norm_w), rstd,
+                                    dox, d, static_cast<const float*>(dh), d, static_cast<float*>(dx), d,
+                                    static_cast<float*>(dnorm_w), part, pbytes, stream);
+  return moc_rmsnorm_backward_bf16(x, d, t, d, norm_w, rstd, dox, d, dh, d, dx, d, dnorm_w, MOC_BF16, part, pbytes,
+                                   stream);
+}
+
+// ---------------------------------------------------------------------------
+// The FFN half over an f32 stream with f32 weights under bf16 autocast, one
+// call per pass: the weights' casts (and the incoming gradient's) in one
+// launch, the norm writing the FFN's bf16 input, the FFN's launches, the
+// residual sum in f32.  cast: bf16 W_gate, W_up [inter, d], W_down [d, inter]
+// and, in the backward, the gradient [rows, d], one after the other, each
+// 256-byte aligned.
+namespace {
+struct CastF32 {
+  int64_t wg, wu, wd, go, bytes;
+};
+CastF32 cast_f32(int64_t rows, int64_t d, int64_t inter) {
+  auto up = [](int64_t b) { return (b + 255) / 256 * 256; };
+  CastF32 c;
+  c.wg = 0;
+  c.wu = up(inter * d * 2);
+  c.wd = 2 * c.wu;
+  c.go = 3 * c.wu;
+  c.bytes = c.go + up(rows * d * 2);
+  return c;
+}
+}  // namespace
+
+extern "C" int64_t moc_ffn_block_f32_cast_size(int64_t rows, int64_t d, int64_t inter) {
+  return rows > 0 && d > 0 && inter > 0 ? cast_f32(rows, d, inter).bytes : 0;
+}
+
+extern "C" int moc_ffn_block_forward_f32(int64_t rows, int64_t d, int64_t inter, int64_t k, int selection,
+                                         const float* h, const float* norm_w, float eps, void* xn, float* rstd,
+                                         const float* wg, const float* wu, const float* wd, void* cast,
+                                         int64_t cast_bytes, void* g, void* u, int64_t ld_gu, void* vals, void* idx,
+                                         int idx_dtype, void* u_s, void* s_s, void* z_s, float* out, void* workspace,
+                                         int64_t workspace_bytes, void* stream) {
+  MOC_REQUIRE(rows >= 1 && d >= 8 && d % 8 == 0 && inter >= 8 && inter % 8 == 0, "moc_ffn_block_forward_f32: bad shape");
+  MOC_REQUIRE(h && norm_w && xn && rstd && wg && wu && wd && cast && out && moc::aligned16(cast) && moc::aligned16(h) &&
+                  moc::aligned16(out),
+              "moc_ffn_block_forward_f32: null or unaligned operand");
+  const CastF32 c = cast_f32(rows, d, inter);
+  MOC_REQUIRE(cast_bytes >= c.bytes, "moc_ffn_block_forward_f32: cast buffer of %lld bytes required",
+              (long long)c.bytes);
+  char* b = static_cast<char*>(cast);
+  const void* src[3] = {wg, wu, wd};
+  void* dst[3] = {b + c.wg, b + c.wu, b + c.wd};
+  const int64_t r[3] = {inter, inter, d}, cols[3] = {d, d, inter};
+  int rc = moc_cast_bf16_multi(3, src, r, cols, dst, cols, stream);
+  if (rc == MOC_OK) rc = moc_rmsnorm_rows_f32(h, d, rows, d, norm_w, eps, xn, d, rstd, stream);
+  if (rc != MOC_OK) return rc;
+  void* y = b + c.go;  // the FFN's bf16 output
+  rc = ffn_forward(MOC_BF16, "moc_ffn_block_forward_f32", rows, d, inter, k, selection, xn, d, dst[0], d, dst[1], d,
+                   dst[2], inter, g, u, ld_gu, vals, idx, idx_dtype, u_s, s_s, z_s, y, d, workspace, workspace_bytes,
+                   stream);
+  if (rc != MOC_OK) return rc;
+  return moc::add_f32_bf16(h, y, out, rows * d, moc::as_stream(stream));
+}
+
+extern "C" int moc_ffn_block_backward_f32(int64_t rows, int64_t d, int64_t inter, int64_t k, const float* dout,
+                                          const float* h, const float* norm_w, const float* rstd, const void* xn,
+                                          const void* idx, int idx_dtype, const void* g_s, const void* u_s,
+                                          const void* s_s, const void* z_s, const float* wg, const float* wu,
+                                          const float* wd, void* cast, int64_t cast_bytes, void* zbuf, int64_t ldz,
+                                          void* gg, void* gu, int64_t ld_ggu, int stacked, void* dxn, float* dh,
+                                          float* dwg, float* dwu, float* dwd, float* dnorm_w, void* workspace,
+                                          int64_t workspace_bytes, void* stream) {
+  MOC_REQUIRE(rows >= 1 && d >= 8 && d % 8 == 0 && inter >= 8 && inter % 8 == 0,
+              "moc_ffn_block_backward_f32: bad shape");
+  MOC_REQUIRE(dout && h && norm_w && rstd && xn && wg && wu && wd && cast && dxn && dh && dnorm_w &&
+                  moc::aligned16(cast) && moc::aligned16(dout),
+              "moc_ffn_block_backward_f32: null or unaligned operand");
+  const CastF32 c = cast_f32(rows, d, inter);
+  const int64_t need = moc_ffn_block_backward_workspace_size(rows, d, inter, ld_ggu, stacked);
+  MOC_REQUIRE(cast_bytes >= c.bytes && workspace != nullptr && workspace_bytes >= need && moc::aligned16(workspace),
+              "moc_ffn_block_backward_f32: cast buffer of %lld and workspace of %lld bytes required",
+              (long long)c.bytes, (long long)need);
+  char* b = static_cast<char*>(cast);
+  const void* src[4] = {wg, wu, wd, dout};
+  void* dst[4] = {b + c.wg, b + c.wu, b + c.wd, b + c.go};
+  const int64_t r[4] = {inter, inter, d, rows}, cols[4] = {d, d, inter, d};
+  int rc = moc_cast_bf16_multi(4, src, r, cols, dst, cols, stream);
+  if (rc != MOC_OK) return rc;
+  const int64_t f = block_rms_offset(rows, d, inter, ld_ggu, stacked);
+  rc = moc_ffn_backward_bf16(rows, d, inter, k, dst[3], d, xn, d, idx, idx_dtype, g_s, u_s, s_s, z_s, dst[0], d,
+                             dst[1], d, dst[2], inter, zbuf, ldz, gg, gu, ld_ggu, stacked, nullptr, dxn, d, dwg, dwu, d,
+                             dwd, inter, MOC_F32, workspace, f, stream);
+  if (rc != MOC_OK) return rc;
+  return moc_rmsnorm_backward_f32(h, d, rows, d, norm_w, rstd, dxn, d, dout, d, dh, d, dnorm_w,
+                                  static_cast<char*>(workspace) + f, workspace_bytes - f, stream);
+}
+
+// ---------------------------------------------------------------------------
+// The f32 layer's backward (moc/ffn.py:175-259, :423-497) as one call: the
+// launches of the per-kernel path in its order.  s_s and z_s NULL: the GCP
+// form, recomputed into s_tmp and z_tmp [rows, k].
+extern "C" int64_t moc_ffn_backward_f32_workspace_size(int64_t rows, int64_t d, int64_t inter) {
+  if (rows <= 0 || d <= 0 || inter <= 0) return 0;
+  return std::max({gemm_ws(d, inter, rows, 0, MOC_F32), gemm_ws(rows, inter, d, 0, MOC_F32),
+                   gemm_ws(inter, d, rows, 0, MOC_F32), gemm_ws(rows, d, inter, inter, MOC_F32)});
+}
+
+extern "C" int moc_ffn_backward_f32(int64_t rows, int64_t d, int64_t inter, int64_t k, const float* go,
+                                    const float* x, const void* idx, int idx_dtype, const float* g_s,
+                                    const float* u_s, const float* s_s, const float* z_s, float* s_tmp, float* z_tmp,
+                                    const float* wg, const float* wu, const float* wd, float* zbuf, float* gg,
+                                    float* gu, int64_t pitch, float* dx, float* dwg, float* dwu, float* dwd,
+                                    void* workspace, int64_t workspace_bytes, void* stream) {
+  MOC_REQUIRE(rows >= 1 && d >= 4 && d % 4 == 0 && inter >= 4 && inter % 4 == 0 && k >= 1 && k <= inter &&
+                  pitch >= inter && pitch % 4 == 0,
+              "moc_ffn_backward_f32: bad shape");
+  MOC_REQUIRE(go && x && idx && g_s && u_s && wg && wu && wd && zbuf && gg && gu && dx && dwg && dwu && dwd &&
+                  (s_s != nullptr ? z_s != nullptr : (s_tmp != nullptr && z_tmp != nullptr)),
+              "moc_ffn_backward_f32: null operand");
+  const int64_t need = moc_ffn_backward_f32_workspace_size(rows, d, inter);
+  MOC_REQUIRE(workspace_bytes >= need && (need == 0 || workspace != nullptr),
+              "moc_ffn_backward_f32: workspace of %lld bytes required", (long long)need);
+  int rc = MOC_OK;
+  if (s_s == nullptr) {
+    rc = moc_gcp_recompute(MOC_F32, g_s, u_s, rows * k, s_tmp, z_tmp, stream);
+    if (rc != MOC_OK) return rc;
+    s_s = s_tmp;
+    z_s = z_tmp;
+  }
+  auto gemm = [&](int64_t m, int64_t n, int64_t kk, const float* a, int64_t am, int64_t ak, const float* b, int64_t bk,
+                  float* c, int64_t ldc, const float* a2 = nullptr, const float* b2 = nullptr) {
+    return moc_gemm_ws(MOC_F32, m, n, kk, a, am, ak, b, bk, 1, a2 ? kk : 0, a2, a2 ? am : 0, a2 ? ak : 0, b2,
+                       b2 ? bk : 0, b2 ? 1 : 0, c, ldc, MOC_F32, workspace, workspace_bytes, stream);
+  };
+  rc = moc_scatter_sparse_to_dense(MOC_F32, z_s, idx, idx_dtype, rows, k, inter, zbuf, pitch, stream);
+  if (rc == MOC_OK) rc = gemm(d, inter, rows, go, 1, d, zbuf, pitch, dwd, inter);  // dWd = go^T Z
+  if (rc == MOC_OK) rc = gemm(rows, inter, d, go, d, 1, wd, inter, zbuf, pitch);   // gZ = go Wd, in Z's place
+  if (rc == MOC_OK)
+    rc = moc_sparse_backward_aux(MOC_F32, idx, idx_dtype, g_s, u_s, s_s, zbuf, pitch, rows, k, inter, gg, gu, pitch,
+                                 stream);
+  if (rc == MOC_OK) rc = gemm(inter, d, rows, gg, 1, pitch, x, d, dwg, d);  // dWg = gG^T x
+  if (rc == MOC_OK) rc = gemm(inter, d, rows, gu, 1, pitch, x, d, dwu, d);  // dWu = gU^T x
+  if (rc == MOC_OK) rc = gemm(rows, d, inter, gg, pitch, 1, wg, d, dx, d, gu, wu);  // dX = gG Wg + gU Wu
+  return rc;
+}

@@ -322,6 +322,19 @@ __global__ __launch_bounds__(64 * kRmsWaves) void rmsnorm_f32_bwd_rows_kernel(
   }
 }
 
+// out = x + y, x and out f32, y bf16 (the residual stream's sum under
+// autocast): eight values a thread.
+__global__ __launch_bounds__(256) void add_f32_bf16_kernel(const float* __restrict__ x, const uint16_t* __restrict__ y,
+                                                           float* __restrict__ out, int64_t n8) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n8) return;
+  const F8 a = load8(x + 8 * i);
+  const uint4 b = reinterpret_cast<const uint4*>(y)[i];
+  float4* o = reinterpret_cast<float4*>(out + 8 * i);
+  o[0] = make_float4(a.v[0] + lo16(b.x), a.v[1] + hi16(b.x), a.v[2] + lo16(b.y), a.v[3] + hi16(b.y));
+  o[1] = make_float4(a.v[4] + lo16(b.z), a.v[5] + hi16(b.z), a.v[6] + lo16(b.w), a.v[7] + hi16(b.w));
+}
+
 // f32 -> bf16 copies of up to kCastMax matrices in one launch (the weights of
 // a layer under autocast): workgroups [start[i], start[i + 1]) take matrix i,
 // eight consecutive columns a thread; dst rows 16-byte aligned, pitch dld.
@@ -368,6 +381,14 @@ bool rows_ok(const void* p, int64_t ld, int64_t d) {
 }
 
 }  // namespace
+
+int add_f32_bf16(const float* x, const void* y, float* out, int64_t n, hipStream_t st) {
+  MOC_REQUIRE(n % 8 == 0 && aligned16(x) && aligned16(y) && aligned16(out), "add_f32_bf16: whole aligned chunks of 8");
+  if (n == 0) return MOC_OK;
+  add_f32_bf16_kernel<<<dim3(static_cast<unsigned>((n / 8 + 255) / 256)), 256, 0, st>>>(
+      x, static_cast<const uint16_t*>(y), out, n / 8);
+  return check_launch("add_f32_bf16_kernel");
+}
 }  // namespace moc
 
 using namespace moc;

@@ -299,6 +299,10 @@ def _backward_common(grad_out, x, idx, g_s, u_s, s_s, z_s, gate_w, up_w, down_w,
         # one native call for the whole single-stream backward
         return _layer_backward(x, x2, go, idx, g_s, u_s, s_s, z_s, gate_w, up_w, down_w, gcp,
                                grad_dtype or down_w.dtype)
+    if side is None and x.dtype == torch.float32 and (grad_dtype or down_w.dtype) == torch.float32 and \
+            down_w.shape[0] == d and _layer_ok(x2, gate_w, up_w, down_w, dtypes=(torch.float32,)) and \
+            _layer_ok(go, dtypes=(torch.float32,)) and x2.is_contiguous() and go.is_contiguous():
+        return _layer_backward_f32(x, x2, go, idx, g_s, u_s, s_s, z_s, gate_w, up_w, down_w, gcp)
     if gcp and x.dtype == torch.bfloat16 and K.row_pitch(inter, torch.bfloat16) <= 8192:
         # S is not kept: the aux kernel recomputes it from g_s (the same bits)
         s_s, z_full = K.gcp_recompute_scatter(g_s, u_s, idx, inter, want_s=False)
@@ -372,6 +376,29 @@ def _layer_backward(x, x2, go, idx, g_s, u_s, s_s, z_s, gate_w, up_w, down_w, gc
              dx.data_ptr(), d, dwg.data_ptr(), dwu.data_ptr(), d, dwd.data_ptr(), inter,
              N.dtype_code(grad_dtype), N.ptr(ws), nbytes, N.stream_of(x2))
     return dx.reshape(x.shape).to(x.dtype), dwg, dwu, dwd
+
+
+def _layer_backward_f32(x, x2, go, idx, g_s, u_s, s_s, z_s, gate_w, up_w, down_w, gcp: bool):
+    """_backward_common's f32 launches as one native call (same results)."""
+    rows, d = x2.shape
+    inter = gate_w.shape[0]
+    dev = x2.device
+    pitch = K.row_pitch(inter, torch.float32)
+    sel = [t if t is None else t.reshape(rows, -1).contiguous() for t in (idx, g_s, u_s, s_s, z_s)]
+    kk = sel[0].shape[1]
+    tmp = torch.empty((2, rows, kk), dtype=torch.float32, device=dev) if gcp else None
+    buf = torch.empty((3, rows, pitch), dtype=torch.float32, device=dev)
+    dx, dwg, dwu, dwd = (torch.empty_like(t) for t in (x2, gate_w, up_w, down_w))
+    nbytes = _layer_ws_bytes(("bf32", dev.index, rows, d, inter), "moc_ffn_backward_f32_workspace_size", rows, d, inter)
+    ws = K._gemm_workspace(dev, nbytes) if nbytes > 0 else None
+    b0, step = buf.data_ptr(), rows * pitch * 4
+    t0 = tmp.data_ptr() if gcp else None
+    N.call("moc_ffn_backward_f32", rows, d, inter, kk, go.data_ptr(), x2.data_ptr(), sel[0].data_ptr(),
+           N.idx_code(sel[0].dtype), sel[1].data_ptr(), sel[2].data_ptr(), None if gcp else sel[3].data_ptr(),
+           None if gcp else sel[4].data_ptr(), t0, t0 + rows * kk * 4 if gcp else None, gate_w.data_ptr(),
+           up_w.data_ptr(), down_w.data_ptr(), b0, b0 + step, b0 + 2 * step, pitch, dx.data_ptr(), dwg.data_ptr(),
+           dwu.data_ptr(), dwd.data_ptr(), N.ptr(ws), nbytes, N.stream_of(x2))
+    return dx.reshape(x.shape), dwg, dwu, dwd
 
 
 def _stack_weight_grads(dev, inter: int, d: int, pitch: int, dtype) -> bool:
@@ -673,13 +700,20 @@ class _MoCBlockF32Function(torch.autograd.Function):
         d = h.shape[-1]
         inter = gate_w.shape[0]
         h2 = h.reshape(-1, d)
-        xn, rstd = K.rmsnorm_rows_f32(h2, norm_w, eps)
-        wg, wu, wd = K.cast_bf16(gate_w, up_w, down_w)
-        _check_inputs(xn, wg, wu, wd, use_triton_aux, index_save_dtype)
+        _check_inputs(h, gate_w, up_w, down_w, use_triton_aux, index_save_dtype)
         bitmask = index_save_dtype == INDEX_SAVE_BITMASK
-        out, idx, vals, u_s, s_s, z_s, *mask = _forward_common(
-            xn, wg, wu, wd, k, selection, _pack_topk_idx_dtype(index_save_dtype, inter), save_s=not gcp,
-            want_mask=bitmask)
+        idx_dtype = _pack_topk_idx_dtype(index_save_dtype, inter)
+        native = not bitmask and _block_f32_native(h2, gate_w, down_w)
+        if native:
+            out, idx, vals, u_s, s_s, z_s, xn, rstd = _block_forward_f32_native(
+                h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s=not gcp)
+            mask = ()
+        else:
+            xn, rstd = K.rmsnorm_rows_f32(h2, norm_w, eps)
+            wg, wu, wd = K.cast_bf16(gate_w, up_w, down_w)
+            y, idx, vals, u_s, s_s, z_s, *mask = _forward_common(xn, wg, wu, wd, k, selection, idx_dtype,
+                                                                 save_s=not gcp, want_mask=bitmask)
+            out = h2 + y
         sel = _saved_index(idx, mask[0] if mask else None, bitmask)
         # the parameters, not their casts: the backward casts them again
         if gcp:
@@ -687,7 +721,8 @@ class _MoCBlockF32Function(torch.autograd.Function):
         else:
             ctx.save_for_backward(h2, xn, rstd, norm_w, sel, vals, u_s, s_s, z_s, gate_w, up_w, down_w)
         ctx.k, ctx.inter, ctx.bitmask, ctx.gcp, ctx.h_shape = idx.shape[-1], inter, bitmask, gcp, h.shape
-        return (h2 + out).reshape(h.shape)
+        ctx.native = native
+        return out.reshape(h.shape)
 
     @staticmethod
     def backward(ctx, dout):
@@ -697,12 +732,90 @@ class _MoCBlockF32Function(torch.autograd.Function):
         else:
             h2, xn, rstd, norm_w, saved, g_s, u_s, s_s, z_s, gate_w, up_w, down_w = ctx.saved_tensors
         idx = _restore_index(ctx, saved)
-        wg, wu, wd = K.cast_bf16(gate_w, up_w, down_w)
         d2 = dout.reshape(h2.shape).contiguous()
+        if ctx.native and d2.data_ptr() % 16 == 0 and d2.dtype == torch.float32 and (
+                not ctx.gcp or K.row_pitch(ctx.inter, torch.bfloat16) <= 8192):
+            dh, dnw, dwg, dwu, dwd = _block_backward_f32_native(d2, h2, xn, rstd, norm_w, idx, g_s, u_s, s_s, z_s,
+                                                                gate_w, up_w, down_w, ctx.gcp)
+            return dh.reshape(ctx.h_shape), dnw, dwg, dwu, dwd, None, None, None, None, None, None
+        wg, wu, wd = K.cast_bf16(gate_w, up_w, down_w)
         dxn, dwg, dwu, dwd = _backward_common(d2.to(torch.bfloat16), xn, idx, g_s, u_s, s_s, z_s, wg, wu, wd,
                                               gcp=ctx.gcp, grad_dtype=gate_w.dtype)
         dh, dnw = K.rmsnorm_backward_f32(h2, norm_w, rstd, dxn, dres=d2)
         return dh.reshape(ctx.h_shape), dnw, dwg, dwu, dwd, None, None, None, None, None, None
+
+
+def _block_f32_native(h2, gate_w, down_w) -> bool:
+    """The one-call f32-stream entries take this shape (single-stream, two
+    rows or more, whole 16-byte rows of every bf16 operand)."""
+    rows, d = h2.shape
+    inter = gate_w.shape[0]
+    return (USE_NATIVE_LAYER and K._GEMM_PROBE is None and rows >= 2 and inter % 8 == 0 and down_w.shape[0] == d
+            and h2.is_contiguous() and _side_for(h2.device, rows, inter) is None)
+
+
+def _block_forward_f32_native(h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s):
+    """moc_ffn_block_forward_f32: casts, norm, FFN and residual in one call."""
+    rows, d = h2.shape
+    inter = gate_w.shape[0]
+    dev = h2.device
+    bf16 = torch.bfloat16
+    pitch = K.row_pitch(inter, bf16)
+    kk = _moc_2_8_effective_k(inter) if selection == "2of8" else k
+    xn = torch.empty((rows, d), dtype=bf16, device=dev)
+    rstd = torch.empty(rows, dtype=torch.float32, device=dev)
+    gu = torch.empty((2, rows, pitch), dtype=bf16, device=dev)
+    sel = [torch.empty((rows, kk), dtype=bf16, device=dev) for _ in range(4 if save_s else 2)]
+    idx = torch.empty((rows, kk), dtype=idx_dtype, device=dev)
+    out = torch.empty_like(h2)
+    ncast = _layer_ws_bytes(("c", rows, d, inter), "moc_ffn_block_f32_cast_size", rows, d, inter)
+    cast = torch.empty(ncast, dtype=torch.uint8, device=dev)
+    nbytes = _layer_ws_bytes(("f", False, dev.index, rows, d, inter), "moc_ffn_forward_workspace_size",
+                             rows, d, inter)
+    ws = K._gemm_workspace(dev, nbytes) if nbytes > 0 else None
+    vals, u_s, s_s, z_s = (*sel, None, None)[:4]
+    g0 = gu.data_ptr()
+    N.call("moc_ffn_block_forward_f32", rows, d, inter, kk, _SELECTION_CODE[selection], h2.data_ptr(),
+           norm_w.data_ptr(), eps, xn.data_ptr(), rstd.data_ptr(), gate_w.data_ptr(), up_w.data_ptr(),
+           down_w.data_ptr(), cast.data_ptr(), ncast, g0, g0 + rows * pitch * 2, pitch, vals.data_ptr(),
+           idx.data_ptr(), N.idx_code(idx_dtype), u_s.data_ptr(), N.ptr(s_s), N.ptr(z_s), out.data_ptr(), N.ptr(ws),
+           nbytes, N.stream_of(h2))
+    return out, idx, vals, u_s, s_s, z_s, xn, rstd
+
+
+def _block_backward_f32_native(dout, h2, xn, rstd, norm_w, idx, g_s, u_s, s_s, z_s, gate_w, up_w, down_w, gcp):
+    """moc_ffn_block_backward_f32: casts, FFN backward and the norm's backward
+    in one call."""
+    rows, d = h2.shape
+    inter = gate_w.shape[0]
+    dev = h2.device
+    bf16, f32 = torch.bfloat16, torch.float32
+    pitch = K.row_pitch(inter, bf16)
+    sel = [t if t is None else t.contiguous() for t in (idx, g_s, u_s, s_s, z_s)]
+    kk = sel[0].shape[-1]
+    stacked = _stack_weight_grads(dev, inter, d, pitch, bf16)
+    buf = torch.empty((3, rows, pitch), dtype=bf16, device=dev)  # Z, then [gG | gU]
+    dxn = torch.empty((rows, d), dtype=bf16, device=dev)
+    dh, dnw, dwd = torch.empty_like(h2), torch.empty_like(norm_w), torch.empty_like(down_w)
+    if stacked:
+        dw = torch.empty((2 * pitch, d), dtype=f32, device=dev)
+        dwg, dwu = dw[:inter], dw[pitch:pitch + inter]
+    else:
+        dwg, dwu = torch.empty_like(gate_w), torch.empty_like(up_w)
+    ncast = _layer_ws_bytes(("c", rows, d, inter), "moc_ffn_block_f32_cast_size", rows, d, inter)
+    cast = torch.empty(ncast, dtype=torch.uint8, device=dev)
+    nbytes = _layer_ws_bytes(("bb", dev.index, rows, d, inter, stacked), "moc_ffn_block_backward_workspace_size",
+                             rows, d, inter, 2 * pitch, int(stacked))
+    ws = K._gemm_workspace(dev, nbytes)
+    z0 = buf.data_ptr()
+    gg = z0 + rows * pitch * 2
+    N.call("moc_ffn_block_backward_f32", rows, d, inter, kk, dout.data_ptr(), h2.data_ptr(), norm_w.data_ptr(),
+           rstd.data_ptr(), xn.data_ptr(), sel[0].data_ptr(), N.idx_code(sel[0].dtype), sel[1].data_ptr(),
+           sel[2].data_ptr(), None if gcp else sel[3].data_ptr(), None if gcp else sel[4].data_ptr(),
+           gate_w.data_ptr(), up_w.data_ptr(), down_w.data_ptr(), cast.data_ptr(), ncast, z0, pitch, gg,
+           gg + 2 * pitch, 2 * pitch, int(stacked), dxn.data_ptr(), dh.data_ptr(), dwg.data_ptr(), dwu.data_ptr(),
+           dwd.data_ptr(), dnw.data_ptr(), ws.data_ptr(), nbytes, N.stream_of(h2))
+    return dh, dnw, dwg, dwu, dwd
 
 
 def _block_forward_native(h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s):
