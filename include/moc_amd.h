@@ -238,6 +238,21 @@ int moc_ffn_infer_bf16(int64_t rows, int64_t d, int64_t inter, int64_t k, int se
                        const void* res, int64_t ldres, void* y, int64_t ldy, void* scratch,
                        int64_t scratch_bytes, void* workspace, int64_t workspace_bytes, void* stream);
 
+/* Next-token cross entropy of bf16 logits [batch, seq, vocab] (rows ld apart):
+ * position t < seq - 1 against labels[b, t + 1], the mean over the labels that
+ * are not ignore_index (moc/model.py:139-144); vocab a multiple of 8 up to
+ * 65536, at most 2^22 positions.  forward: loss (loss_dtype), and for the backward lse [batch seq] and
+ * inv_count [1]; row_loss [batch seq] is scratch.  A label outside the
+ * vocabulary makes the loss NaN.  backward: dlogits bf16 (rows ldd apart, zeros
+ * where there is no label) from grad_loss, a device scalar of loss_dtype. */
+int moc_next_token_loss_forward(const void* logits, int64_t ld, int64_t batch, int64_t seq, int64_t vocab,
+                                const int64_t* labels, int64_t ignore_index, float* lse, float* row_loss,
+                                void* loss, int loss_dtype, float* inv_count, void* stream);
+int moc_next_token_loss_backward(const void* logits, int64_t ld, int64_t batch, int64_t seq, int64_t vocab,
+                                 const int64_t* labels, int64_t ignore_index, const float* lse,
+                                 const float* inv_count, const void* grad_loss, int loss_dtype,
+                                 void* dlogits, int64_t ldd, void* stream);
+
 /* The attention half of a decoder block, h = x + out_proj(attention(RoPE(
  * qkv_proj(RMSNorm(x))))) (moc/model.py:31-64,83-84), one call per pass, bit for
  * bit the separate entry points in order.  f32 = 0: x, dh, h, dx, the weights

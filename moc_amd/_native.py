@@ -76,6 +76,10 @@ SIGNATURES: dict[str, tuple] = {
                                            _int, _vp, _i64, _vp]),
     "moc_decode_block_bf16": (_int, [_vp, _i64, _i64, _vp, ctypes.c_float, _vp, _vp, _i64, _vp, _i64, _i64,
                                      _int, _vp, _vp, _i64, _vp]),
+    "moc_next_token_loss_forward": (_int, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _vp, _int, _vp,
+                                           _vp]),
+    "moc_next_token_loss_backward": (_int, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _vp, _int, _vp,
+                                            _i64, _vp]),
     "moc_attention_half_saved_size": (_i64, [_i64, _i64, _i64, _i64, _int]),
     "moc_attention_half_scratch_size": (_i64, [_i64, _i64, _i64, _i64, _int]),
     "moc_attention_half_workspace_size": (_i64, [_i64, _i64]),

@@ -4,6 +4,7 @@ over the library's kernels: the norm as a row kernel, the projections on the
 MFMA engine, causal attention with RoPE inside (moc_amd/csrc/attn.hip), the
 residual added in out_proj's epilogue.  The stock composition (about 45
 elementwise launches a step besides the products) stays for everything else.
+And the model's next-token loss (moc_amd/csrc/loss.hip).
 
 bf16 models and f32 models under bf16 autocast; the rounding points are the
 stock ones where it stores bf16 (norm output, q/k/v, rotated q and k, the
@@ -16,6 +17,8 @@ from functools import lru_cache
 
 import torch
 import torch.nn as nn
+import torch.nn.functional as F
+from torch.autograd.function import once_differentiable
 
 from . import _native as N
 from . import kernels as K
@@ -102,6 +105,7 @@ class _AttentionHalf(torch.autograd.Function):
         return h
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, dh):
         x, norm_w, qkv_w, out_w, cos, sin, saved = ctx.saved_tensors
         batch, seq, d = x.shape
@@ -120,3 +124,51 @@ class _AttentionHalf(torch.autograd.Function):
                saved.data_ptr(), saved.numel(), dx.data_ptr(), dn.data_ptr(), dq.data_ptr(), do.data_ptr(),
                scratch.data_ptr(), nscratch, N.ptr(ws), nws, N.stream_of(x))
         return dx, dn, dq, do, None, None, None, None
+
+
+def next_token_loss_ok(logits, labels) -> bool:
+    """True if next_token_loss takes these: bf16 device logits whose stock loss
+    is f32 (autocast) or bf16, int64 labels of their shape."""
+    return (logits.is_cuda and logits.dtype == BF16 and logits.dim() == 3 and logits.shape[1] >= 2
+            and logits.is_contiguous() and logits.data_ptr() % 16 == 0 and logits.numel() > 0
+            and logits.shape[2] % 8 == 0 and logits.shape[2] <= 65536 and logits.shape[0] * logits.shape[1] <= 1 << 22
+            and labels.device == logits.device and labels.dtype == torch.int64
+            and labels.shape == logits.shape[:2])
+
+
+def next_token_loss(logits, labels, ignore_index: int = -100) -> torch.Tensor:
+    """F.cross_entropy(logits[:, :-1], labels[:, 1:], ignore_index) of bf16
+    logits, f32 under autocast (as autocast runs it), else bf16;
+    next_token_loss_ok must hold."""
+    f32 = torch.is_autocast_enabled("cuda")
+    return _NextTokenLoss.apply(logits, labels.contiguous(), ignore_index, F32 if f32 else BF16)
+
+
+class _NextTokenLoss(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, logits, labels, ignore_index, dtype):
+        b, s, v = logits.shape
+        buf = torch.empty(2 * b * s + 1, dtype=F32, device=logits.device)  # lse, row losses, 1 / count
+        loss = torch.empty((), dtype=dtype, device=logits.device)
+        p = buf.data_ptr()
+        N.call("moc_next_token_loss_forward", logits.data_ptr(), v, b, s, v, labels.data_ptr(), ignore_index, p,
+               p + 4 * b * s, loss.data_ptr(), N.dtype_code(dtype), p + 8 * b * s, N.stream_of(logits))
+        ctx.save_for_backward(logits, labels, buf)
+        ctx.ignore_index = ignore_index
+        return loss
+
+    @staticmethod
+    def backward(ctx, g):
+        logits, labels, buf = ctx.saved_tensors
+        if torch.is_grad_enabled():  # a graph of the gradient is wanted: the stock loss has one
+            x = logits[:, :-1].flatten(0, 1)
+            loss = F.cross_entropy(x.float() if g.dtype == F32 else x, labels[:, 1:].flatten(),
+                                   ignore_index=ctx.ignore_index)
+            return torch.autograd.grad(loss, logits, g, create_graph=True)[0], None, None, None
+        b, s, v = logits.shape
+        d = torch.empty_like(logits)
+        g = g.contiguous()
+        p = buf.data_ptr()
+        N.call("moc_next_token_loss_backward", logits.data_ptr(), v, b, s, v, labels.data_ptr(), ctx.ignore_index, p,
+               p + 8 * b * s, g.data_ptr(), N.dtype_code(g.dtype), d.data_ptr(), v, N.stream_of(logits))
+        return d, None, None, None

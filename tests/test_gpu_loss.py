@@ -1,0 +1,96 @@
+"""The next-token loss kernels against 64 bits and the stock composition."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from moc_amd import MoCConfig, build_model
+from moc_amd.block import next_token_loss, next_token_loss_ok
+
+pytestmark = pytest.mark.gpu
+BF, F64 = torch.bfloat16, torch.float64
+
+
+@pytest.mark.parametrize("batch,seq,vocab", [(1, 2, 8), (3, 5, 4096), (2, 33, 4104), (2, 9, 32000), (1, 3, 65536),
+                                             (4, 64, 1000)])
+@pytest.mark.parametrize("autocast", [True, False])
+def test_loss_and_gradient(batch, seq, vocab, autocast):
+    g = torch.Generator(device="cuda").manual_seed(batch * seq + vocab)
+    x = (3 * torch.randn(batch, seq, vocab, generator=g, device="cuda")).to(BF)
+    labels = torch.randint(0, vocab, (batch, seq), generator=g, device="cuda")
+    if seq > 2:
+        labels[0, 1] = -100
+    if batch > 2:
+        labels[1] = -100
+    x.requires_grad_()
+    assert next_token_loss_ok(x, labels)
+    with torch.autocast("cuda", dtype=BF, enabled=autocast):
+        loss = next_token_loss(x, labels)
+        stock = F.cross_entropy(x[:, :-1].flatten(0, 1), labels[:, 1:].flatten(), ignore_index=-100)
+    assert loss.dtype == stock.dtype
+    xd = x.detach().to(F64).requires_grad_()
+    ref = F.cross_entropy(xd[:, :-1].flatten(0, 1), labels[:, 1:].flatten(), ignore_index=-100)
+    # f32: expf, logf and a sum of vocab terms a row, then a 64-bit mean
+    tol = 2e-6 if loss.dtype == torch.float32 else 2.0 ** -8
+    assert abs(loss.item() - ref.item()) <= tol * max(1.0, abs(ref.item()))
+    grad = torch.autograd.grad(loss, x, torch.tensor(0.7, dtype=loss.dtype, device="cuda"))[0]
+    want = torch.autograd.grad(ref, xd, torch.tensor(0.7, dtype=loss.dtype).to("cuda", F64))[0]
+    # its bf16 rounding; exp(x - lse) - 1 at the label cancels f32 values near 1
+    assert ((grad.to(F64) - want).abs() <= 2.0 ** -8 * want.abs() + 2e-6 / (batch * (seq - 1))).all()
+    assert (grad[:, -1] == 0).all()
+
+
+def test_all_ignored_and_bad_labels_are_nan():
+    x = torch.randn(2, 4, 64, device="cuda").to(BF)
+    assert torch.isnan(next_token_loss(x, torch.full((2, 4), -100, device="cuda")))
+    labels = torch.zeros(2, 4, dtype=torch.int64, device="cuda")
+    labels[1, 2] = 64
+    assert torch.isnan(next_token_loss(x, labels))
+
+
+def test_infinite_logits():
+    x = torch.zeros(1, 3, 16, device="cuda").to(BF)
+    x[0, 0, 3] = -float("inf")
+    labels = torch.tensor([[0, 1, 2]], device="cuda")
+    ref = F.cross_entropy(x.float()[:, :-1].flatten(0, 1), labels[:, 1:].flatten())
+    assert abs(next_token_loss(x, labels).item() - ref.item()) < 2e-2
+    x[0, 0, 3] = float("inf")  # inf - inf, as in the stock loss
+    assert torch.isnan(next_token_loss(x, labels))
+
+
+def test_second_derivative():
+    x = torch.randn(2, 4, 64, device="cuda").to(BF).requires_grad_()
+    labels = torch.randint(0, 64, (2, 4), device="cuda")
+    v = torch.randn(2, 4, 64, device="cuda").to(BF)
+
+    def hv(loss):
+        return torch.autograd.grad((torch.autograd.grad(loss, x, create_graph=True)[0] * v).sum(), x)[0]
+
+    with torch.autocast("cuda", dtype=BF):
+        got = hv(next_token_loss(x, labels))
+    xd = x.detach().to(F64).requires_grad_()
+    loss = F.cross_entropy(xd[:, :-1].flatten(0, 1), labels[:, 1:].flatten())
+    gd = torch.autograd.grad(loss, xd, create_graph=True)[0]
+    want = torch.autograd.grad((gd * v.to(F64)).sum(), xd)[0]
+    # bf16 roundings of the first gradient's product with v, of its cotangent
+    # and of the result, each 2^-9 of its value; the cotangent's difference from
+    # its mean cancels part of it
+    assert (got.to(F64) - want).norm() <= 4 * 2.0 ** -9 * want.norm()
+
+
+@pytest.mark.parametrize("dtype", [BF, torch.float32])
+def test_model_uses_it(dtype):
+    torch.manual_seed(1)
+    cfg = MoCConfig(hidden_size=128, intermediate_size=344, num_hidden_layers=2, num_attention_heads=2,
+                    vocab_size=1000, max_seq_len=64)
+    m = build_model(cfg, "moc").to("cuda", dtype)
+    ids = torch.randint(0, 1000, (3, 40), device="cuda")
+    with torch.autocast("cuda", dtype=BF, enabled=dtype == torch.float32):
+        logits, loss = m(ids, labels=ids)
+        want = F.cross_entropy(logits[:, :-1].flatten(0, 1), ids[:, 1:].flatten())
+    assert type(loss.grad_fn).__name__ == "_NextTokenLossBackward"
+    assert loss.dtype == want.dtype
+    got = torch.autograd.grad(loss, m.lm_head.weight, retain_graph=True)[0]
+    ref = torch.autograd.grad(want, m.lm_head.weight)[0]
+    # bf16: the stock gradient exponentiates bf16 log-probabilities (an error
+    # of 2^-9 of their size, about 7 here)
+    assert (got.float() - ref.float()).norm() <= (3e-2 if dtype == BF else 1e-2) * ref.float().norm()
