@@ -4,7 +4,8 @@ over the library's kernels: the norm as a row kernel, the projections on the
 MFMA engine, causal attention with RoPE inside (moc_amd/csrc/attn.hip), the
 residual added in out_proj's epilogue.  The stock composition (about 45
 elementwise launches a step besides the products) stays for everything else.
-And the model's next-token loss (moc_amd/csrc/loss.hip).
+And the model's last steps: final norm with LM head, next-token loss
+(moc_amd/csrc/loss.hip).
 
 bf16 models and f32 models under bf16 autocast; the rounding points are the
 stock ones where it stores bf16 (norm output, q/k/v, rotated q and k, the
@@ -124,6 +125,84 @@ class _AttentionHalf(torch.autograd.Function):
                saved.data_ptr(), saved.numel(), dx.data_ptr(), dn.data_ptr(), dq.data_ptr(), do.data_ptr(),
                scratch.data_ptr(), nscratch, N.ptr(ws), nws, N.stream_of(x))
         return dx, dn, dq, do, None, None, None, None
+
+
+def lm_head_ok(h, norm, norm_type, head, weight) -> bool:
+    """True if lm_head takes the model's last step, weight @ norm(h): plain
+    modules (head: the nn.Linear that holds weight, or None for a tied one) in
+    the stream's dtype, two tokens or more."""
+    dt = stream_dtype(h)
+    if dt is None or type(norm) is not norm_type or h.dim() != 3 or not bare(norm):
+        return False
+    if head is not None and (type(head) is not nn.Linear or head.bias is not None or not bare(head)):
+        return False
+    d = h.shape[-1]
+    if d % 8 or d > 4096 or weight.dim() != 2 or weight.shape[0] % 8 or h.numel() < 2 * d:
+        return False
+    return all(t.dtype == dt and t.is_contiguous() and t.device == h.device and t.data_ptr() % 16 == 0
+               for t in (h, norm.weight, weight)) and norm.weight.shape == (d,) and weight.shape[1] == d
+
+
+def lm_head(h, norm, weight) -> torch.Tensor:
+    """norm(h) @ weight.T as bf16 logits; lm_head_ok must hold."""
+    return _LMHead.apply(h, norm.weight, weight, float(norm.eps))
+
+
+def _own_head_dx(tokens: int, d: int) -> bool:
+    """dX contracts over the vocabulary into few tiles: the library's product
+    leaves most CUs idle, the engine's splits K.  Library and engine, us, of 32000
+    words: 93 / 21 (16 tokens, d 512), 106 / 34 (512, 512), 295 / 128 (4096,
+    512), 327 / 224 (4096, 1024), 427 / 406 (4096, 2048), the last of the range
+    where the engine was ahead."""
+    return tokens * d <= 1 << 23
+
+
+def _own_head_dw(d: int, vocab: int) -> bool:
+    """dW, library and engine, us: 139 / 113 (32000 words, d 512, 4096 tokens),
+    250 / 210 (d 1024), 494 / 421 (d 2048); but 25 / 43 (d 256, 1024 tokens) and
+    25 / 38 (8192 words, d 1024, 1024 tokens), where half of the CUs get no tile."""
+    return d >= 512 and vocab >= 16384
+
+
+class _LMHead(torch.autograd.Function):
+    """The final norm as one row kernel each way (f32 stream: straight to the
+    product's bf16 operand), the forward product by the library (equal to the
+    engine's at d <= 1024: 160 and 153 us at 4096 x 512 x 32000, ahead above:
+    377 and 434 at d 2048), the backward's by shape."""
+
+    @staticmethod
+    def forward(ctx, h, norm_w, weight, eps):
+        d = h.shape[-1]
+        h2 = h.reshape(-1, d)
+        if h.dtype == F32:
+            xn, rstd = K.rmsnorm_rows_f32(h2, norm_w, eps)
+            wb, = K.cast_bf16(weight)
+        else:
+            (xn, rstd), wb = K.rmsnorm_rows(h2, norm_w, eps), weight
+        ctx.save_for_backward(h, norm_w, weight, xn, rstd, wb)
+        ctx.eps = eps
+        return torch.matmul(xn, wb.t()).reshape(*h.shape[:-1], weight.shape[0])
+
+    @staticmethod
+    def backward(ctx, g):
+        h, norm_w, weight, xn, rstd, wb = ctx.saved_tensors
+        if torch.is_grad_enabled():  # a graph of the gradient is wanted: the stock operators have one
+            xf = h.float()
+            y = (xf * torch.rsqrt(torch.mean(xf * xf, dim=-1, keepdim=True) + ctx.eps)).to(h.dtype) * norm_w
+            wanted = [t for t in (h, norm_w, weight) if t.requires_grad]
+            it = iter(torch.autograd.grad(y.to(BF16) @ weight.to(BF16).t(), wanted, g, create_graph=True))
+            return (*(next(it) if t.requires_grad else None for t in (h, norm_w, weight)), None)
+        d, vocab = h.shape[-1], weight.shape[0]
+        h2, g2 = h.reshape(-1, d), g.reshape(-1, vocab)
+        dh = dnw = dw = None
+        if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
+            dxn = K.gemm(g2, wb) if _own_head_dx(h2.shape[0], d) else torch.matmul(g2, wb)
+            dh, dnw = (K.rmsnorm_backward_f32 if h.dtype == F32 else K.rmsnorm_backward)(h2, norm_w, rstd, dxn)
+            dh = dh.reshape(h.shape)
+        if ctx.needs_input_grad[2]:
+            dw = (K.gemm(g2.t(), xn, out_dtype=weight.dtype) if _own_head_dw(d, vocab)
+                  else torch.matmul(g2.t(), xn).to(weight.dtype))
+        return dh, dnw, dw, None
 
 
 def next_token_loss_ok(logits, labels) -> bool:

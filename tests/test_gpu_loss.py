@@ -1,10 +1,12 @@
-"""The next-token loss kernels against 64 bits and the stock composition."""
+"""The model's last steps, final norm with LM head and next-token loss, against
+64 bits and the stock composition."""
 import pytest
 import torch
 import torch.nn.functional as F
 
 from moc_amd import MoCConfig, build_model
-from moc_amd.block import next_token_loss, next_token_loss_ok
+from moc_amd.block import lm_head, lm_head_ok, next_token_loss, next_token_loss_ok
+from moc_amd.model import RMSNorm
 
 pytestmark = pytest.mark.gpu
 BF, F64 = torch.bfloat16, torch.float64
@@ -94,3 +96,73 @@ def test_model_uses_it(dtype):
     # bf16: the stock gradient exponentiates bf16 log-probabilities (an error
     # of 2^-9 of their size, about 7 here)
     assert (got.float() - ref.float()).norm() <= (3e-2 if dtype == BF else 1e-2) * ref.float().norm()
+
+
+def _stock_head(h, norm_w, w, eps):
+    inv = torch.rsqrt((h * h).mean(-1, keepdim=True) + eps)
+    return (h * inv * norm_w) @ w.t()
+
+
+@pytest.mark.parametrize("tokens,d,vocab", [(2, 8, 8), (3, 72, 1000), (70, 512, 16384), (65, 256, 16392),
+                                            (257, 520, 32000), (2100, 4096, 64)])
+@pytest.mark.parametrize("dtype", [BF, torch.float32])
+def test_lm_head(tokens, d, vocab, dtype):
+    g = torch.Generator(device="cuda").manual_seed(tokens + d)
+    h = torch.randn(1, tokens, d, generator=g, device="cuda").to(dtype).requires_grad_()
+    w = (torch.randn(vocab, d, generator=g, device="cuda") / d ** 0.5).to(dtype).requires_grad_()
+    norm = RMSNorm(d).to("cuda", dtype)
+    with torch.no_grad():
+        norm.weight.add_(0.1 * torch.randn(d, generator=g, device="cuda").to(dtype))
+    dy = torch.randn(1, tokens, vocab, generator=g, device="cuda").to(BF)
+    with torch.autocast("cuda", dtype=BF, enabled=dtype == torch.float32):
+        assert lm_head_ok(h, norm, RMSNorm, None, w)
+        y = lm_head(h, norm, w)
+    got = [y, *torch.autograd.grad(y, (h, norm.weight, w), dy)]
+    leaf = [t.detach().to(F64).requires_grad_() for t in (h, norm.weight, w)]
+    yd = _stock_head(*leaf, norm.eps)
+    want = [yd, *torch.autograd.grad(yd, leaf, dy.to(F64))]
+    assert [t.dtype for t in got] == [BF, dtype, dtype, dtype]
+    for a, b in zip(got, want):
+        # bf16 operands of every product (up to two roundings of 2^-9 each way)
+        # and of its result; their errors are independent
+        assert (a.to(F64) - b).norm() <= 4 * 2.0 ** -9 * b.norm(), (a.shape, ((a.to(F64) - b).norm() / b.norm()).item())
+
+
+@pytest.mark.parametrize("dtype", [BF, torch.float32])
+def test_lm_head_second_derivative_and_frozen_weights(dtype):
+    h = torch.randn(1, 5, 64, device="cuda").to(dtype).requires_grad_()
+    w = torch.randn(128, 64, device="cuda").to(dtype).requires_grad_()
+    norm = RMSNorm(64).to("cuda", dtype)
+
+    def grads(f, *to):
+        with torch.autocast("cuda", dtype=BF, enabled=dtype == torch.float32):
+            y = f()
+        return torch.autograd.grad(y.float().sin().sum(), to, create_graph=True)
+
+    def penalty(f):
+        return torch.autograd.grad(grads(f, h)[0].float().square().sum(), (h, w))
+
+    # the same operators, gradients added in another order (bf16 sums)
+    for a, b in zip(penalty(lambda: lm_head(h, norm, w)), penalty(lambda: F.linear(norm(h), w))):
+        assert a.abs().max() > 0 and (a.float() - b.float()).norm() <= 2e-2 * b.float().norm()
+    norm.weight.requires_grad_(False)
+    w.requires_grad_(False)
+    with torch.autocast("cuda", dtype=BF, enabled=dtype == torch.float32):
+        y = lm_head(h, norm, w)
+    y.sum().backward()
+    assert h.grad.abs().max() > 0 and w.grad is None and norm.weight.grad is None
+
+
+@pytest.mark.parametrize("tied", [True, False])
+def test_model_uses_lm_head(tied):
+    torch.manual_seed(2)
+    cfg = MoCConfig(hidden_size=128, intermediate_size=344, num_hidden_layers=1, num_attention_heads=2,
+                    vocab_size=1000, max_seq_len=64, tie_word_embeddings=tied)
+    m = build_model(cfg, "moc").to("cuda", BF)
+    ids = torch.randint(0, 1000, (2, 33), device="cuda")
+    assert type(m(ids).grad_fn).__name__ == "_LMHeadBackward"
+    seen = []
+    hook = m.norm.register_forward_hook(lambda *a: seen.append(1))
+    m(ids)
+    hook.remove()
+    assert seen == [1]
