@@ -314,7 +314,12 @@ __global__ __launch_bounds__(kAtThreads, HD == 64 ? 2 : 1) void attn_fwd_kernel(
 }
 
 // ----------------------------------------------------------------- backward
-// dQ: the wave's queries against every key tile they see; also delta.
+// dQ: the wave's queries against every key tile they see; also delta.  A
+// kernel of its own for each side, recomputing the scores, keeps every sum
+// inside one wave: no atomics and no cross-workgroup partials.  Bound by the
+// latency of a workgroup's two to four tiles.  4096 tokens of 256, 16 heads of
+// 64: dQ 28 us, dK/dV 44 us, forward 20 us; the library's backward is 104 us,
+// its forward 50, the RoPE launches around them not counted.
 template <int HD, bool TF32>
 __global__ __launch_bounds__(kAtThreads) void attn_bwd_q_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(1024))) char lk[kAtTile * HD * 2];
@@ -392,7 +397,8 @@ __global__ __launch_bounds__(kAtThreads) void attn_bwd_q_kernel(AttnArgs a) {
   if (q < a.seq) store_own<HD, true, TF32>(a, acc, a.scale, a.dqkv + (tok0 + q) * a.ld + head * HD, q, lane);
 }
 
-// dK and dV: the wave's keys against every query tile that sees them.
+// dK and dV: the wave's keys against every query tile that sees them (two
+// products more than dQ, and the recomputed scores).
 template <int HD, bool TF32>
 __global__ __launch_bounds__(kAtThreads) void attn_bwd_kv_kernel(AttnArgs a) {
   __shared__ __attribute__((aligned(1024))) char lq[kAtTile * HD * 2];
@@ -486,7 +492,8 @@ __global__ __launch_bounds__(kAtThreads) void attn_bwd_kv_kernel(AttnArgs a) {
 }
 
 // 128 keys a tile for sequences of 129 to 256 in heads of 64 (two tiles where
-// 64 would take four; 4096 tokens of 256, 16 heads: 20.6 us either way), else 64.
+// 64 would take four; 4096 tokens of 256, 16 heads: 20.3 us, tiles of 64 20.6;
+// the reason is the rounding, above), else 64.
 template <int HD, bool TF32>
 void launch_fwd(const AttnArgs& a, dim3 grid, hipStream_t st) {
   if constexpr (HD == 64) {

@@ -442,7 +442,7 @@ __global__ __launch_bounds__(256) void pack28_kernel(const uint16_t* __restrict_
 
 // One thread per (row, group of 8 channels): two 16-byte loads, the top-2
 // tournament, one 16-byte store over G (bound by the 6 bytes a channel that
-// pass through it).
+// pass through it; 4.0 us at 48 x 5464, where the launch is most of it).
 __global__ __launch_bounds__(256) void select28_dense_kernel(uint4* __restrict__ g, const uint4* __restrict__ u,
                                                              int64_t ld8, int groups, int64_t total) {
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
