@@ -243,7 +243,7 @@ int moc_ffn_infer_bf16(int64_t rows, int64_t d, int64_t inter, int64_t k, int se
  * are not ignore_index (moc/model.py:139-144); vocab a multiple of 8 up to
  * 65536, at most 2^22 positions.  forward: loss (loss_dtype), and for the backward lse [batch seq] and
  * inv_count [1]; row_loss [batch seq] is scratch.  A label outside the
- * vocabulary makes the loss NaN.  backward: dlogits bf16 (rows ldd apart, zeros
+ * vocabulary makes the loss and its row's lse and gradient NaN.  backward: dlogits bf16 (rows ldd apart, zeros
  * where there is no label) from grad_loss, a device scalar of loss_dtype. */
 int moc_next_token_loss_forward(const void* logits, int64_t ld, int64_t batch, int64_t seq, int64_t vocab,
                                 const int64_t* labels, int64_t ignore_index, float* lse, float* row_loss,

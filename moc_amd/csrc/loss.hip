@@ -50,7 +50,8 @@ __device__ __forceinline__ int64_t label_of(const int64_t* __restrict__ labels, 
 
 // One workgroup per row: the row in registers (NC chunks a thread), its maximum,
 // the sum of exponentials; lse[r] and loss[r] (0 where ignored; NaN for a
-// label outside the vocabulary).
+// label outside the vocabulary, which the stock loss refuses: the loss and that
+// row's gradient are then NaN).
 template <int NC>
 __global__ __launch_bounds__(kCeThreads) void ce_forward_kernel(const uint16_t* __restrict__ x, int64_t ld, int vocab,
                                                                 int seq, const int64_t* __restrict__ labels,
@@ -96,8 +97,9 @@ __global__ __launch_bounds__(kCeThreads) void ce_forward_kernel(const uint16_t* 
   sum = block_reduce<false>(sum, red);
   if (tid == 0) {
     const float l = mx + logf(sum);
-    lse[r] = l;
-    loss[r] = label >= 0 && label < vocab ? l - bf16_to_f32(row[label]) : NAN;
+    const bool known = label >= 0 && label < vocab;
+    lse[r] = known ? l : NAN;
+    loss[r] = known ? l - bf16_to_f32(row[label]) : NAN;
   }
 }
 

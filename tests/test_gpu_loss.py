@@ -49,6 +49,18 @@ def test_all_ignored_and_bad_labels_are_nan():
     assert torch.isnan(next_token_loss(x, labels))
 
 
+def test_bad_label_gradient_is_nan():
+    """A label outside the vocabulary: the gradient of its position is NaN, not
+    that of a row without a label; the other rows keep theirs."""
+    x = torch.randn(2, 4, 64, device="cuda").to(BF).requires_grad_()
+    labels = torch.zeros(2, 4, dtype=torch.int64, device="cuda")
+    labels[1, 2], labels[0, 1] = 64, -1
+    grad, = torch.autograd.grad(next_token_loss(x, labels), x)
+    bad = torch.zeros(2, 4, dtype=torch.bool, device="cuda")
+    bad[1, 1] = bad[0, 0] = True
+    assert torch.isnan(grad[bad]).all() and torch.isfinite(grad[~bad]).all()
+
+
 def test_infinite_logits():
     x = torch.zeros(1, 3, 16, device="cuda").to(BF)
     x[0, 0, 3] = -float("inf")
