@@ -193,7 +193,8 @@ class _LMHead(torch.autograd.Function):
             it = iter(torch.autograd.grad(y.to(BF16) @ weight.to(BF16).t(), wanted, g, create_graph=True))
             return (*(next(it) if t.requires_grad else None for t in (h, norm_w, weight)), None)
         d, vocab = h.shape[-1], weight.shape[0]
-        h2, g2 = h.reshape(-1, d), g.reshape(-1, vocab)
+        # contiguous: an expanded gradient has rows 0 apart, which no GEMM operand has
+        h2, g2 = h.reshape(-1, d), g.contiguous().reshape(-1, vocab)
         dh = dnw = dw = None
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
             dxn = K.gemm(g2, wb) if _own_head_dx(h2.shape[0], d) else torch.matmul(g2, wb)

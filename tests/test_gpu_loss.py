@@ -165,6 +165,22 @@ def test_lm_head_second_derivative_and_frozen_weights(dtype):
     assert h.grad.abs().max() > 0 and w.grad is None and norm.weight.grad is None
 
 
+@pytest.mark.parametrize("tokens,d,vocab", [(5, 64, 128), (4, 512, 16384)])
+@pytest.mark.parametrize("rows", [True, False])
+def test_lm_head_expanded_gradient(tokens, d, vocab, rows):
+    """A sum over the tokens (or over everything) sends an expanded gradient
+    back, rows 0 elements apart: the gradients of its contiguous copy."""
+    h = torch.randn(1, tokens, d, device="cuda").to(BF).requires_grad_()
+    w = torch.randn(vocab, d, device="cuda").to(BF).requires_grad_()
+    norm = RMSNorm(d).to("cuda", BF)
+    dy = torch.randn(vocab if rows else 1, device="cuda").to(BF).expand(1, tokens, vocab)
+    assert dy.stride(1) == 0
+    y = lm_head(h, norm, w)
+    got = torch.autograd.grad(y, (h, norm.weight, w), dy, retain_graph=True)
+    want = torch.autograd.grad(y, (h, norm.weight, w), dy.contiguous())
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("tied", [True, False])
 def test_model_uses_lm_head(tied):
     torch.manual_seed(2)
