@@ -289,9 +289,12 @@ class InferenceMoCSwiGLUFFN(nn.Module):
         nb, c = x_2d.shape[0], self.config
         if nb > 4 and (grouped28 or not c.grouped) and x_2d.is_cuda and x_2d.dtype == norm_weight.dtype == torch.bfloat16 \
                 and self.gate_proj.weight.dtype == torch.bfloat16 \
+                and norm_weight.shape == (c.hidden_size,) and norm_weight.is_contiguous() \
+                and norm_weight.data_ptr() % 16 == 0 and (not x_2d.is_contiguous() or x_2d.data_ptr() % 16 == 0) \
                 and not (torch.is_grad_enabled() and (x.requires_grad or norm_weight.requires_grad)):
             # more tokens: the norm as a row kernel in front of the layer's
-            # kernels, the residual added in the last of them
+            # kernels, the residual added in the last of them (x or a norm
+            # weight off the 16-byte grid, a view into a buffer, goes below)
             ensure_native_ops_ready()
             self._ensure_down_weight_t()
             x_2d = x_2d.contiguous()

@@ -121,3 +121,20 @@ def test_layer_with_norm_and_residual(nb, grouped, hidden, inter):
         y = m.fused_decode_residual(x, w, 1e-6)
         assert torch.equal(y, (x.float() + m(xn).float()).to(BF))
         assert torch.equal(y[:, None], m.fused_decode_residual(x[:, None], w, 1e-6))
+
+
+@pytest.mark.parametrize("nb", [5, 16, 40])
+@pytest.mark.parametrize("grouped", [False, True])
+def test_layer_with_norm_takes_unaligned_views(nb, grouped):
+    """x or the norm weight as a view off the 16-byte grid: the result of the
+    aligned copies, up to the norm's own roundings."""
+    kw = dict(grouped_a=2, grouped_b=8) if grouped else {}
+    m = InferenceMoCSwiGLUFFN(256, 704, 176 if grouped else 128, **kw).to("cuda", BF)
+    off = lambda t: torch.cat((t.new_zeros(1), t.flatten()))[1:].view(t.shape)  # noqa: E731
+    x, w = torch.randn(nb, 256, device="cuda").to(BF), torch.ones(256, device="cuda").to(BF)
+    with torch.no_grad():
+        assert off(x).data_ptr() % 16 and off(w).data_ptr() % 16
+        for y in (m.fused_decode_residual(off(x), w, 1e-6), m.fused_decode_residual(x, off(w), 1e-6)):
+            xf = x.float()
+            xn = (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-6)).to(BF) * w
+            assert torch.equal(y, x + m(xn))
