@@ -165,9 +165,9 @@ def _plain(*modules) -> bool:
 
 def _one_token_native(x: torch.Tensor, *weights) -> bool:
     """One bf16 token of a gradient-free pass outside autocast, with
-    contiguous, aligned bf16 weights on its device."""
+    contiguous, aligned bf16 weights on its device (the token aligned too)."""
     return (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[:2] == (1, 1) and not torch.is_grad_enabled()
-            and not torch.is_autocast_enabled("cuda")
+            and not torch.is_autocast_enabled("cuda") and x.data_ptr() % 16 == 0
             and all(w.dtype == torch.bfloat16 and w.device == x.device and w.is_contiguous()
                     and w.data_ptr() % 16 == 0 for w in weights))
 

@@ -118,3 +118,17 @@ def test_hooks_keep_the_stock_path():
     m.layers[0].attn.out_proj.register_forward_hook(lambda *a: seen.append(1))
     make_step(m, "eager")(torch.zeros(1, 1, dtype=torch.int64, device="cuda"), 0)
     assert seen
+
+
+def test_unaligned_token_keeps_the_stock_path():
+    cfg = DecodeConfig(hidden=256, intermediate=704, heads=4, layers=1, vocab=100, k=128, max_seq=8)
+    m = DecoderModel("global_moc", cfg).to("cuda", BF).init_weights(6)
+    m.allocate_cache()
+    layer, pos = m.layers[0], torch.tensor(0, device="cuda")
+    x = torch.randn(1, 1, 256, device="cuda").to(BF)
+    off = torch.cat((x.new_zeros(1), x.flatten()))[1:].view(x.shape)
+    with torch.no_grad():
+        assert layer._attn_native(x) and not layer._attn_native(off)
+        got = layer.forward_step(off, pos)
+        layer.fuse_attn = False
+        assert torch.equal(got, layer.forward_step(x, pos))
