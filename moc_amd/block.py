@@ -20,6 +20,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 from torch.autograd.function import once_differentiable
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import _native as N
 from . import kernels as K
@@ -41,9 +42,10 @@ def stream_dtype(x):
 
 
 def bare(*modules) -> bool:
-    """No hooks on the modules that a fused half does not call."""
-    return not any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
-                   for m in modules)
+    """No hooks on the modules that a fused half does not call, their own or
+    those registered for every module."""
+    return not _has_any_global_hook() and not any(
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
 
 
 def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:

@@ -34,6 +34,7 @@ from typing import Callable
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from .. import kernels as K
 from .inference_ffn import InferenceMoCSwiGLUFFN
@@ -153,8 +154,11 @@ class StaticKVAttention(nn.Module):
 
 
 def _plain(*modules) -> bool:
-    """No forward hooks, and the linears plain bias-free nn.Linear: what a
-    fused step computes from the weights alone."""
+    """No forward hooks (the modules' own or those registered for every
+    module), and the linears plain bias-free nn.Linear: what a fused step
+    computes from the weights alone."""
+    if _has_any_global_hook():
+        return False
     for m in modules:
         if m._forward_hooks or m._forward_pre_hooks:
             return False

@@ -203,3 +203,17 @@ def test_product_never_imports_oracle():
     for path in (ROOT / "moc_amd").rglob("*.py"):
         text = path.read_text()
         assert not re.search(r"^\s*(from|import)\s+oracle", text, flags=re.M), path
+
+
+@pytest.mark.parametrize("register", ["register_module_forward_hook", "register_module_forward_pre_hook"])
+def test_hooks_for_every_module_keep_the_stock_composition(register):
+    from moc_amd.block import bare
+    from moc_amd.inference.decode_model import _plain
+    lin = torch.nn.Linear(8, 8, bias=False)
+    assert bare(lin) and _plain(lin)
+    handle = getattr(torch.nn.modules.module, register)(lambda *a: None)
+    try:
+        assert not bare(lin) and not _plain(lin)
+    finally:
+        handle.remove()
+    assert bare(lin) and _plain(lin)
