@@ -1871,6 +1871,35 @@ F32Split plan_f32(int64_t M, int64_t N, int64_t K, int64_t K2) {
   return p;
 }
 
+// Split-K plan of a bf16 GEMM: a product whose 256x256 tiles fill at most a
+// third of the CUs runs each tile as `ksplit` (>= 3) workgroups over
+// consecutive ranges of at least 4 K tiles.  ldw: row pitch of the f32
+// partials.
+struct SplitPlan {
+  int ksplit = 1;
+  int kper = 0;
+  int64_t ldw = 0;
+  int64_t bytes = 0;
+};
+
+SplitPlan plan_split(int64_t M, int64_t N, int nk) {
+  SplitPlan p;
+  p.kper = nk;
+  const int64_t tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
+  const int cus = cu_count();
+  if (tiles <= 0 || 3 * tiles > cus) return p;
+  int ks = static_cast<int>(std::min<int64_t>(cus / tiles, nk / 4));
+  if (ks < 2) return p;
+  const int kper = (nk + ks - 1) / ks;
+  ks = (nk + kper - 1) / kper;
+  if (ks < 2) return p;
+  p.ksplit = ks;
+  p.kper = kper;
+  p.ldw = (N + 3) & ~3LL;
+  p.bytes = kFixCounterBytes + static_cast<int64_t>(ks) * M * p.ldw * 4;  // partials after the counters
+  return p;
+}
+
 // The small-tile plan of a product [M, N] (with n2 > 0: of the pair [M, N],
 // [M, n2] side by side, never split over K), bm = 0 where the 256-wide tiles
 // are as fast or faster.  Measured on both sides (bf16, cold weights):
@@ -1885,9 +1914,18 @@ F32Split plan_f32(int64_t M, int64_t N, int64_t K, int64_t K2) {
 //       8192 x 768 x 2048     32.0         128 x 128        33.7
 //       2048 x 2048 x 10912   95.3         128 x 128, in 2  99.5
 //       4096 x 2736 x 1024    27.6         128 x 128        33.7
+//       1280 x 3398 x 5000    60.9, 3 parts  128 x 128, in 2  79.3
+//       1619 x 1728 x 7546    56.9, 5 parts  128 x 128, in 4  67.8
+//       1280 x 2605 x 6200    56.8, 4 parts  128 x 128, in 2  53.8
+//   pair 1619 x 3773 x 1728   74.6         128 x 64         78.5
+//   pair 1779 x 3547 x 1728   75.5         128 x 128        71.9
 // so a product takes small tiles while its 256x256 tiles are at most 0.35 of
 // the CUs (a pair: fewer than the CUs) and hold at most 24 K tiles per CU
-// together.  Among the small tiles the least predicted time wins: a K tile
+// together (a pair: 21), unless plan_split fills nearly all CUs and is
+// predicted far ahead: kper K tiles of 1.4 us, 5.5 us of prologue and
+// reduction and its partials' bytes (within 8 % of 12 such shapes).  The line
+// is 1.42 times that, where the two sides measure equal (the small tiles'
+// prediction is up to a third high where K is long).  Among the small tiles the least predicted time wins: a K tile
 // takes t1 us with one workgroup on a CU and t2 with two, each workgroup t0
 // more, a K split one reduction launch and its partials' bytes; the model
 // is within 10 % of the table above and of 40 shapes around it.
@@ -1904,7 +1942,7 @@ MidPlan plan_mid(int64_t M, int64_t N, int nk, int64_t n2, int64_t ws_bytes) {
   auto tiles = [](int64_t m, int64_t n, int bm, int bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
   const int64_t big = tiles(M, N, kBM, kBN) + (n2 > 0 ? tiles(M, n2, kBM, kBN) : 0);
   if (M < 1 || N < 1 || nk < 1 || big * nk > 24 * cus) return p;
-  if (n2 > 0 ? big >= cus : 20 * big > 7 * cus) return p;
+  if (n2 > 0 ? big >= cus || big * nk > 21 * cus : 20 * big > 7 * cus) return p;
   const int64_t ldw = (N + 3) & ~3LL;
   const double part_us = 2.0 * M * ldw * 4 / kPartRate;
   double best = 0;
@@ -1932,35 +1970,13 @@ MidPlan plan_mid(int64_t M, int64_t N, int nk, int64_t n2, int64_t ws_bytes) {
       }
     }
   }
-  return p;
-}
-
-// Split-K plan of a bf16 GEMM: a product whose 256x256 tiles fill at most a
-// third of the CUs runs each tile as `ksplit` (>= 3) workgroups over
-// consecutive ranges of at least 4 K tiles.  ldw: row pitch of the f32
-// partials.
-struct SplitPlan {
-  int ksplit = 1;
-  int kper = 0;
-  int64_t ldw = 0;
-  int64_t bytes = 0;
-};
-
-SplitPlan plan_split(int64_t M, int64_t N, int nk) {
-  SplitPlan p;
-  p.kper = nk;
-  const int64_t tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
-  const int cus = cu_count();
-  if (tiles <= 0 || 3 * tiles > cus) return p;
-  int ks = static_cast<int>(std::min<int64_t>(cus / tiles, nk / 4));
-  if (ks < 2) return p;
-  const int kper = (nk + ks - 1) / ks;
-  ks = (nk + kper - 1) / kper;
-  if (ks < 2) return p;
-  p.ksplit = ks;
-  p.kper = kper;
-  p.ldw = (N + 3) & ~3LL;
-  p.bytes = kFixCounterBytes + static_cast<int64_t>(ks) * M * p.ldw * 4;  // partials after the counters
+  if (n2 == 0) {
+    constexpr double kMargin = 1.42, kTile = 1.4, kEnds = 5.5;
+    const SplitPlan sp = plan_split(M, N, nk);
+    if (sp.ksplit >= 3 && sp.bytes <= ws_bytes &&
+        p.us > kMargin * (sp.kper * kTile + kEnds + sp.ksplit * part_us))
+      return MidPlan();
+  }
   return p;
 }
 

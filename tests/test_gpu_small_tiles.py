@@ -34,6 +34,8 @@ SHAPES = [
     # chunks; long K (split); the largest products the rule gives small tiles
     (17, 64, 64), (64, 65, 72), (65, 129, 130), (129, 127, 1000), (200, 1000, 517), (1, 8, 8),
     (48, 2048, 5461), (333, 300, 4097), (1000, 1024, 2736), (1024, 2736, 1000), (2048, 2048, 5456),
+    # 70 and 49 tiles of 256 with a long K: back on three and five K parts
+    (1280, 3398, 5000), (1619, 1728, 7546),
 ]
 
 
