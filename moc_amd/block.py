@@ -51,7 +51,8 @@ def bare(*modules) -> bool:
 def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:
     """True if attention_half takes this block: plain modules of the model's
     own types in the stream's dtype, heads of 64 or 128, hidden up to 4096, two
-    tokens or more (a gradient product over one token has no aligned operand)."""
+    tokens or more (a gradient product over one token has no aligned operand).
+    Every shape is compared: the kernels take their sizes from x alone."""
     if not FUSE_BLOCK_ATTENTION or type(norm) is not norm_type or type(attn) is not attn_type or x.dim() != 3:
         return False
     dt = stream_dtype(x)
@@ -61,7 +62,12 @@ def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:
         return False
     d = x.shape[-1]
     if attn.head_dim not in (64, 128) or d != attn.num_heads * attn.head_dim or d > 4096 or x.numel() < 2 * d or \
-            x.shape[1] > attn.rope_cos.shape[0] or x.shape[0] > 65535:
+            x.shape[0] > 65535:
+        return False
+    cos = attn.rope_cos
+    if norm.weight.shape != (d,) or qkv.weight.shape != (3 * d, d) or out.weight.shape != (d, d) or \
+            cos.dim() != 2 or cos.shape[0] < x.shape[1] or cos.shape[1] != attn.head_dim // 2 or \
+            attn.rope_sin.shape != cos.shape:
         return False
     if x.is_contiguous() and x.data_ptr() % 16:
         return False
