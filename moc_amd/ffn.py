@@ -78,6 +78,13 @@ class StandardSwiGLUFFN(nn.Module):
         return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
 
 
+def _weights_fit(d: int, gate_w, up_w, down_w) -> bool:
+    """Weights [inter, d], [inter, d] and [any, inter]: the kernels take d and
+    inter from x and gate_w, the rest through bare pointers."""
+    return (gate_w.dim() == 2 and gate_w.shape[1] == d and up_w.shape == gate_w.shape
+            and down_w.dim() == 2 and down_w.shape[1] == gate_w.shape[0])
+
+
 def _check_inputs(x, gate_w, up_w, down_w, strict_aux: bool, index_save_dtype):
     if strict_aux and not (index_save_dtype == torch.int16 or index_save_dtype == INDEX_SAVE_BITMASK):
         raise ValueError("MoC fused helper kernels require compact saved indices.")
@@ -88,6 +95,9 @@ def _check_inputs(x, gate_w, up_w, down_w, strict_aux: bool, index_save_dtype):
         raise ValueError(
             f"MoC HIP kernels need one compute dtype, got x={x.dtype}, weights="
             f"{gate_w.dtype}/{up_w.dtype}/{down_w.dtype}")
+    if not _weights_fit(x.shape[-1], gate_w, up_w, down_w):
+        raise ValueError(f"MoC FFN shapes do not fit: x {tuple(x.shape)}, gate {tuple(gate_w.shape)}, "
+                         f"up {tuple(up_w.shape)}, down {tuple(down_w.shape)}")
 
 
 _SIDE_STREAMS: dict = {}
@@ -583,10 +593,18 @@ _SELECTION_OF_MODE = {"moc": ("topk", False), "moc_triton_aux": ("topk", False),
                       "moc_post_silu_abs_triton_aux": ("post_silu_abs", False)}
 
 
+def _block_fits(h, norm_weight, ffn) -> bool:
+    """Norm and FFN weights of the shapes that h + ffn(norm(h)) needs."""
+    d = h.shape[-1]
+    wd = ffn.down_proj.weight
+    return (norm_weight.shape == (d,) and wd.shape[0] == d
+            and _weights_fit(d, ffn.gate_proj.weight, ffn.up_proj.weight, wd))
+
+
 def block_ffn_ok(h, norm_weight, ffn) -> bool:
     """True if block_ffn takes this block: a MoC FFN, bf16 activations,
     norm weight and FFN weights on the device, no autocast, hidden a
-    multiple of 8 up to 4096."""
+    multiple of 8 up to 4096, weights that fit each other and h."""
     if not FUSE_BLOCK_FFN or not isinstance(ffn, MoCSwiGLUFFN) or ffn.mode not in _SELECTION_OF_MODE:
         return False
     if not h.is_cuda or h.dtype != torch.bfloat16 or norm_weight.dtype != torch.bfloat16:
@@ -596,8 +614,9 @@ def block_ffn_ok(h, norm_weight, ffn) -> bool:
     d = h.shape[-1]
     if d % 8 or d > 4096:
         return False
-    return all(w.dtype == torch.bfloat16 and w.is_cuda for w in
-               (ffn.gate_proj.weight, ffn.up_proj.weight, ffn.down_proj.weight))
+    return _block_fits(h, norm_weight, ffn) and all(
+        w.dtype == torch.bfloat16 and w.is_cuda for w in
+        (ffn.gate_proj.weight, ffn.up_proj.weight, ffn.down_proj.weight))
 
 
 def block_ffn_f32_ok(h, norm_weight, ffn) -> bool:
@@ -608,8 +627,9 @@ def block_ffn_f32_ok(h, norm_weight, ffn) -> bool:
     d = h.shape[-1]
     if not h.is_cuda or _autocast_dtype(h) != torch.bfloat16 or d % 8 or d > 4096 or h.numel() == 0:
         return False
-    return all(t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in
-               (h, norm_weight, ffn.gate_proj.weight, ffn.up_proj.weight, ffn.down_proj.weight))
+    return _block_fits(h, norm_weight, ffn) and all(
+        t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in
+        (h, norm_weight, ffn.gate_proj.weight, ffn.up_proj.weight, ffn.down_proj.weight))
 
 
 def block_ffn(h, norm_weight, eps: float, ffn) -> torch.Tensor:

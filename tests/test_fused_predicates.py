@@ -8,6 +8,7 @@ import torch.nn as nn
 
 from moc_amd import MoCConfig
 from moc_amd.block import attention_half_ok
+from moc_amd.ffn import block_ffn_f32_ok, block_ffn_ok
 from moc_amd.model import CausalSelfAttention, RMSNorm, TransformerBlock
 
 BF = torch.bfloat16
@@ -59,3 +60,58 @@ def test_attention_half_takes_only_its_shapes(on_device, change):
 def test_attention_half_takes_longer_tables(on_device):
     blk = _block()
     assert _attn_ok(blk, torch.zeros(2, 32, 256, dtype=BF)) and not _attn_ok(blk, torch.zeros(2, 33, 256, dtype=BF))
+
+
+@pytest.fixture
+def autocast():
+    """bf16 autocast for the device type, which torch.autocast refuses to enter without one."""
+    was = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
+    torch.set_autocast_enabled("cuda", True)
+    torch.set_autocast_dtype("cuda", BF)
+    yield
+    torch.set_autocast_enabled("cuda", was[0])
+    torch.set_autocast_dtype("cuda", was[1])
+
+
+FFN = {
+    "narrow norm": lambda b, dt: setattr(b, "ffn_norm", RMSNorm(128).to(dt)),
+    "broadcast norm": lambda b, dt: setattr(b, "ffn_norm", RMSNorm(1).to(dt)),
+    "gate_proj of another input": lambda b, dt: setattr(b.ffn, "gate_proj", nn.Linear(128, 512, bias=False).to(dt)),
+    "up_proj of another input": lambda b, dt: setattr(b.ffn, "up_proj", nn.Linear(128, 512, bias=False).to(dt)),
+    "narrow up_proj": lambda b, dt: setattr(b.ffn, "up_proj", nn.Linear(256, 504, bias=False).to(dt)),
+    "narrow down_proj": lambda b, dt: setattr(b.ffn, "down_proj", nn.Linear(512, 128, bias=False).to(dt)),
+    "down_proj of another input": lambda b, dt: setattr(b.ffn, "down_proj", nn.Linear(504, 256, bias=False).to(dt)),
+}
+
+
+def _ffn_halves(blk, h):
+    return block_ffn_ok(h, blk.ffn_norm.weight, blk.ffn), block_ffn_f32_ok(h, blk.ffn_norm.weight, blk.ffn)
+
+
+@pytest.mark.parametrize("change", list(FFN))
+def test_bf16_ffn_half_takes_only_its_shapes(on_device, change):
+    blk, h = _block(), torch.zeros(2, 16, 256, dtype=BF)
+    assert _ffn_halves(blk, h) == (True, False)
+    FFN[change](blk, BF)
+    assert _ffn_halves(blk, h) == (False, False)
+
+
+@pytest.mark.parametrize("change", list(FFN))
+def test_f32_ffn_half_takes_only_its_shapes(on_device, autocast, change):
+    blk, h = _block(torch.float32), torch.zeros(2, 16, 256)
+    assert _ffn_halves(blk, h) == (False, True)
+    FFN[change](blk, torch.float32)
+    assert _ffn_halves(blk, h) == (False, False)
+
+
+@pytest.mark.parametrize("change", [c for c in FFN if "norm" not in c and c != "narrow down_proj"])
+def test_ffn_layer_refuses_weights_that_do_not_fit(on_device, change):
+    blk = _block()
+    FFN[change](blk, BF)
+    with pytest.raises(ValueError, match="shapes"):
+        blk.ffn(torch.zeros(2, 16, 256, dtype=BF))
+
+
+def test_ffn_layer_refuses_another_hidden_size(on_device):
+    with pytest.raises(ValueError, match="shapes"):
+        _block().ffn(torch.zeros(2, 16, 128, dtype=BF))
