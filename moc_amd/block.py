@@ -41,11 +41,30 @@ def stream_dtype(x):
     return BF16 if x.dtype == BF16 else None
 
 
+# The methods that the fused halves compute themselves.
+_STOCK = {nn.Linear.forward}
+
+
+def stock_method(name: str = "forward"):
+    """Class decorator: a fused half may stand in for this method of the class."""
+    def mark(cls):
+        _STOCK.add(getattr(cls, name))
+        return cls
+    return mark
+
+
+def runs_stock(m: nn.Module, name: str = "forward") -> bool:
+    """Calling m.<name> runs a method a fused half knows: none of the
+    instance's own, of a subclass's, or put in the class's place."""
+    return name not in m.__dict__ and getattr(type(m), name) in _STOCK
+
+
 def bare(*modules) -> bool:
-    """No hooks on the modules that a fused half does not call, their own or
-    those registered for every module."""
+    """The modules that a fused half does not call have the forward it computes
+    and no hooks, their own or those registered for every module."""
     return not _has_any_global_hook() and not any(
-        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks for m in modules)
+        m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks or not runs_stock(m)
+        for m in modules)
 
 
 def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:

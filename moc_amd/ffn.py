@@ -26,6 +26,7 @@ import torch.nn.functional as F
 
 from . import _native as N
 from . import kernels as K
+from .block import runs_stock, stock_method
 
 _MODES = (
     "moc",
@@ -531,6 +532,7 @@ class _MoCGCPFunction(torch.autograd.Function):
     backward = staticmethod(_moc_backward)
 
 
+@stock_method()
 class MoCSwiGLUFFN(nn.Module):
     """MoC SwiGLU FFN with selectable backward strategy (moc/ffn.py:500-581).
 
@@ -605,7 +607,8 @@ def block_ffn_ok(h, norm_weight, ffn) -> bool:
     """True if block_ffn takes this block: a MoC FFN, bf16 activations,
     norm weight and FFN weights on the device, no autocast, hidden a
     multiple of 8 up to 4096, weights that fit each other and h."""
-    if not FUSE_BLOCK_FFN or not isinstance(ffn, MoCSwiGLUFFN) or ffn.mode not in _SELECTION_OF_MODE:
+    if not FUSE_BLOCK_FFN or not isinstance(ffn, MoCSwiGLUFFN) or not runs_stock(ffn) or \
+            ffn.mode not in _SELECTION_OF_MODE:
         return False
     if not h.is_cuda or h.dtype != torch.bfloat16 or norm_weight.dtype != torch.bfloat16:
         return False
@@ -622,7 +625,8 @@ def block_ffn_ok(h, norm_weight, ffn) -> bool:
 def block_ffn_f32_ok(h, norm_weight, ffn) -> bool:
     """True if block_ffn takes this block in its f32-stream form: an f32 model
     under bf16 autocast, otherwise as block_ffn_ok."""
-    if not FUSE_BLOCK_FFN or not isinstance(ffn, MoCSwiGLUFFN) or ffn.mode not in _SELECTION_OF_MODE:
+    if not FUSE_BLOCK_FFN or not isinstance(ffn, MoCSwiGLUFFN) or not runs_stock(ffn) or \
+            ffn.mode not in _SELECTION_OF_MODE:
         return False
     d = h.shape[-1]
     if not h.is_cuda or _autocast_dtype(h) != torch.bfloat16 or d % 8 or d > 4096 or h.numel() == 0:

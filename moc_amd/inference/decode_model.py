@@ -37,6 +37,7 @@ import torch.nn as nn
 from torch.nn.modules.module import _has_any_global_hook
 
 from .. import kernels as K
+from ..block import runs_stock, stock_method
 from .inference_ffn import InferenceMoCSwiGLUFFN
 
 HIDDEN = 2048
@@ -67,6 +68,7 @@ class DecodeConfig:
     max_seq: int = PROMPT_LEN + GEN_LEN
 
 
+@stock_method()
 class RMSNorm(nn.Module):
     """x / rms(x) in f32, cast back, times the weight (benchmark_decode.py:101-109)."""
 
@@ -94,6 +96,7 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
     return torch.stack((a * cos - b * sin, a * sin + b * cos), dim=-1).flatten(-2)
 
 
+@stock_method("forward_step")
 class StaticKVAttention(nn.Module):
     def __init__(self, hidden: int, heads: int, max_seq: int):
         super().__init__()
@@ -155,14 +158,17 @@ class StaticKVAttention(nn.Module):
 
 def _plain(*modules) -> bool:
     """No forward hooks (the modules' own or those registered for every
-    module), and the linears plain bias-free nn.Linear: what a fused step
-    computes from the weights alone."""
+    module), nothing in place of the method that a fused step computes, and
+    norm and attention of this file, else plain bias-free nn.Linear: what a
+    fused step computes from the weights alone."""
     if _has_any_global_hook():
         return False
     for m in modules:
         if m._forward_hooks or m._forward_pre_hooks:
             return False
-        if isinstance(m, nn.Linear) and (type(m) is not nn.Linear or m.bias is not None):
+        if not runs_stock(m, "forward_step" if type(m) is StaticKVAttention else "forward"):
+            return False
+        if type(m) not in (RMSNorm, StaticKVAttention) and (type(m) is not nn.Linear or m.bias is not None):
             return False
     return True
 
@@ -273,10 +279,14 @@ class DecoderModel(nn.Module):
         for layer in self.layers:
             x = layer.forward_step(x, pos)
         n, head = self.final_norm, self.lm_head
-        if (self.fuse_head and type(n) is RMSNorm and _plain(n, head) and self.cfg.hidden % 8 == 0
-                and self.cfg.hidden <= 4096 and _one_token_native(x, n.weight, head.weight)):
+        if self._head_native(x):
             return K.gemv_rmsnorm(x.reshape(1, -1), n.weight, n.eps, head.weight)[0][None]
         return head(n(x))
+
+    def _head_native(self, x: torch.Tensor) -> bool:
+        n, head = self.final_norm, self.lm_head
+        return (self.fuse_head and type(n) is RMSNorm and _plain(n, head) and self.cfg.hidden % 8 == 0
+                and self.cfg.hidden <= 4096 and _one_token_native(x, n.weight, head.weight))
 
 
 def make_step(model: DecoderModel, scope: str) -> Callable[[torch.Tensor, int], torch.Tensor]:

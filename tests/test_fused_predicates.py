@@ -7,8 +7,9 @@ import torch
 import torch.nn as nn
 
 from moc_amd import MoCConfig
-from moc_amd.block import attention_half_ok
+from moc_amd.block import attention_half_ok, lm_head_ok
 from moc_amd.ffn import block_ffn_f32_ok, block_ffn_ok
+from moc_amd.inference.decode_model import DecodeConfig, DecoderModel
 from moc_amd.model import CausalSelfAttention, RMSNorm, TransformerBlock
 
 BF = torch.bfloat16
@@ -115,3 +116,109 @@ def test_ffn_layer_refuses_weights_that_do_not_fit(on_device, change):
 def test_ffn_layer_refuses_another_hidden_size(on_device):
     with pytest.raises(ValueError, match="shapes"):
         _block().ffn(torch.zeros(2, 16, 128, dtype=BF))
+
+
+def _swap_instance(m, name="forward"):
+    """As wrapping tools do it: the instance gets a function of its own."""
+    inner = getattr(m, name)
+    setattr(m, name, lambda *a, **k: inner(*a, **k))
+
+
+def _swap_class(monkeypatch, cls, name="forward"):
+    inner = getattr(cls, name)
+    monkeypatch.setattr(cls, name, lambda *a, **k: inner(*a, **k))
+
+
+@pytest.mark.parametrize("part", ["attn_norm", "attn", "attn.qkv_proj", "attn.out_proj"])
+@pytest.mark.parametrize("where", ["instance", "class"])
+def test_attention_half_leaves_a_replaced_forward_alone(on_device, monkeypatch, part, where):
+    blk, x = _block(), torch.zeros(2, 16, 256, dtype=BF)
+    m = blk.get_submodule(part)
+    _swap_instance(m) if where == "instance" else _swap_class(monkeypatch, type(m))
+    assert not _attn_ok(blk, x)
+
+
+@pytest.mark.parametrize("part", ["norm", "lm_head"])
+@pytest.mark.parametrize("where", ["instance", "class", "subclass"])
+def test_lm_head_leaves_a_replaced_forward_alone(on_device, monkeypatch, part, where):
+    model = nn.Module()
+    model.norm, model.lm_head = RMSNorm(64).to(BF), _linear(64, 128)
+    h = torch.zeros(1, 4, 64, dtype=BF)
+    ok = lambda: lm_head_ok(h, model.norm, RMSNorm, model.lm_head, model.lm_head.weight)  # noqa: E731
+    assert ok()
+    m = getattr(model, part)
+    if where == "instance":
+        _swap_instance(m)
+    elif where == "class":
+        _swap_class(monkeypatch, type(m))
+    else:
+        m.__class__ = type("Own", (type(m),), {"forward": lambda self, t: t})
+    assert not ok()
+
+
+@pytest.mark.parametrize("dtype", [BF, torch.float32])
+@pytest.mark.parametrize("where", ["instance", "class", "subclass"])
+def test_ffn_half_leaves_a_replaced_ffn_forward_alone(on_device, monkeypatch, request, dtype, where):
+    if dtype == torch.float32:
+        request.getfixturevalue("autocast")
+    blk, h = _block(dtype), torch.zeros(2, 16, 256, dtype=dtype)
+    assert any(_ffn_halves(blk, h))
+    if where == "instance":
+        _swap_instance(blk.ffn)
+    elif where == "class":
+        _swap_class(monkeypatch, type(blk.ffn))
+    else:
+        blk.ffn.__class__ = type("Own", (type(blk.ffn),), {"forward": lambda self, t: t})
+    assert not any(_ffn_halves(blk, h))
+
+
+def test_ffn_half_takes_a_subclass_without_a_forward_of_its_own(on_device):
+    blk, h = _block(), torch.zeros(2, 16, 256, dtype=BF)
+    blk.ffn.__class__ = type("Named", (type(blk.ffn),), {})
+    assert _ffn_halves(blk, h) == (True, False)
+
+
+def _decoder():
+    cfg = DecodeConfig(hidden=256, intermediate=704, heads=4, layers=1, vocab=64, k=128, max_seq=8)
+    m = DecoderModel("global_moc", cfg).to(BF)
+    m.allocate_cache()
+    return m
+
+
+@pytest.mark.parametrize("part,name", [("attn_norm", "forward"), ("attn", "forward_step"), ("attn.qkv_proj", "forward"),
+                                       ("attn.out_proj", "forward")])
+@pytest.mark.parametrize("where", ["instance", "class", "other"])
+def test_decode_attention_leaves_a_replaced_forward_alone(on_device, monkeypatch, part, name, where):
+    layer, x = _decoder().layers[0], torch.zeros(1, 1, 256, dtype=BF)
+    with torch.no_grad():
+        assert layer._attn_native(x)
+        m = layer.get_submodule(part)
+        if where == "instance":
+            _swap_instance(m, name)
+        elif where == "class":
+            _swap_class(monkeypatch, type(m), name)
+        elif isinstance(m, nn.Linear):  # a module of another kind that happens to hold a weight
+            other = nn.Module()
+            other.weight = m.weight
+            setattr(layer.attn, part.split(".")[1], other)
+        else:
+            m.__class__ = type("Own", (type(m),), {})
+        assert not layer._attn_native(x)
+
+
+@pytest.mark.parametrize("part", ["final_norm", "lm_head"])
+@pytest.mark.parametrize("where", ["instance", "class", "other"])
+def test_decode_head_leaves_a_replaced_forward_alone(on_device, monkeypatch, part, where):
+    model, x = _decoder(), torch.zeros(1, 1, 256, dtype=BF)
+    with torch.no_grad():
+        assert model._head_native(x)
+        m = getattr(model, part)
+        if where == "instance":
+            _swap_instance(m)
+        elif where == "class":
+            _swap_class(monkeypatch, type(m))
+        elif part == "lm_head":
+            model.lm_head = nn.Sequential(m)
+        else:
+            m.__class__ = type("Own", (type(m),), {})
+        assert not model._head_native(x)
