@@ -6,7 +6,7 @@ import pytest
 import torch
 import torch.nn as nn
 
-from moc_amd import MoCConfig
+from moc_amd import MoCConfig, build_model
 from moc_amd.block import attention_half_ok, lm_head_ok
 from moc_amd.ffn import block_ffn_f32_ok, block_ffn_ok
 from moc_amd.inference.decode_model import DecodeConfig, DecoderModel
@@ -222,3 +222,14 @@ def test_decode_head_leaves_a_replaced_forward_alone(on_device, monkeypatch, par
         else:
             m.__class__ = type("Own", (type(m),), {})
         assert not model._head_native(x)
+
+
+def test_model_takes_a_head_of_another_kind():
+    """A head without a weight of its own (a wrapper around the linear) is called."""
+    torch.manual_seed(0)
+    cfg = MoCConfig(hidden_size=64, intermediate_size=128, num_hidden_layers=0, num_attention_heads=4, vocab_size=32)
+    model = build_model(cfg, "moc")
+    ids = torch.randint(0, 32, (2, 8))
+    want = model(ids)
+    model.lm_head = nn.Sequential(model.lm_head)
+    assert torch.equal(model(ids), want)
