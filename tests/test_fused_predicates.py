@@ -5,6 +5,7 @@ its input, so a module of another shape has to keep the stock composition."""
 import pytest
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import register_module_forward_hook
 
 from moc_amd import MoCConfig, build_model
 from moc_amd.block import attention_half_ok, lm_head_ok
@@ -233,3 +234,50 @@ def test_model_takes_a_head_of_another_kind():
     want = model(ids)
     model.lm_head = nn.Sequential(model.lm_head)
     assert torch.equal(model(ids), want)
+
+
+def _hook(module, kind):
+    """A forward hook on the module, or one for every module; (calls, handle)."""
+    seen = []
+    if kind == "own":
+        return seen, module.register_forward_hook(lambda m, *a: seen.append(m))
+    return seen, register_module_forward_hook(lambda m, *a: seen.append(m))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [BF, torch.float32])
+@pytest.mark.parametrize("part", ["ffn_norm", "ffn"])
+@pytest.mark.parametrize("kind", ["own", "every"])
+def test_ffn_half_calls_hooked_modules(dtype, part, kind):
+    blk = _block(dtype).cuda()
+    x = torch.randn(2, 16, 256, device="cuda").to(dtype)
+    m = blk.get_submodule(part)
+    with torch.autocast("cuda", dtype=BF, enabled=dtype == torch.float32):
+        want = blk(x)
+        seen, handle = _hook(m, kind)
+        try:
+            got = blk(x)
+        finally:
+            handle.remove()
+        assert sum(s is m for s in seen) == 1
+        # the stock composition: bf16 roundings of the norm's and the FFN's output
+        # where the fused half has none, in a stream of unit scale
+        assert (got.float() - want.float()).norm() <= 2e-2 * want.float().norm()
+        blk(x)
+    assert sum(s is m for s in seen) == 1
+
+
+@pytest.mark.gpu
+def test_ffn_half_calls_a_norm_of_another_type():
+    class Doubled(RMSNorm):
+        def forward(self, t):
+            return 2 * super().forward(t)
+
+    blk = _block().cuda()
+    x = torch.randn(2, 16, 256, device="cuda").to(BF)
+    blk.ffn_norm.__class__ = Doubled
+    with torch.no_grad():
+        got = blk(x)
+        h = x + blk.attn(blk.attn_norm(x))
+        want = h + blk.ffn(2 * RMSNorm.forward(blk.ffn_norm, h))
+    assert (got.float() - want.float()).norm() <= 2e-2 * want.float().norm()
