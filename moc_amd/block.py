@@ -208,7 +208,7 @@ class _LMHead(torch.autograd.Function):
             (xn, rstd), wb = K.rmsnorm_rows(h2, norm_w, eps), weight
         ctx.save_for_backward(h, norm_w, weight, xn, rstd, wb)
         ctx.eps = eps
-        return torch.matmul(xn, wb.t()).reshape(*h.shape[:-1], weight.shape[0])
+        return K.unaliased(torch.matmul(xn, wb.t()), (*h.shape[:-1], weight.shape[0]))
 
     @staticmethod
     def backward(ctx, g):

@@ -62,6 +62,13 @@ def cu_count(device_index: int) -> int:
     return n
 
 
+def unaliased(t: torch.Tensor, shape) -> torch.Tensor:
+    """t, made by the caller and used nowhere else, in another shape and no
+    view of t: what a custom Function returns.  Autograd lets no result of a
+    Function that is a view be written in place."""
+    return torch.ops.aten._unsafe_view(t, shape)
+
+
 def gemm_tiles(m: int, n: int) -> int:
     """Workgroups (256x256 output tiles) of a bf16 GEMM with an [m, n] output."""
     return ((m + 255) // 256) * ((n + 255) // 256)

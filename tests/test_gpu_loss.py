@@ -194,3 +194,22 @@ def test_model_uses_lm_head(tied):
     m(ids)
     hook.remove()
     assert seen == [1]
+
+
+@pytest.mark.parametrize("dtype", [BF, torch.float32])
+def test_logits_take_writes_in_place(dtype):
+    """Masking or scaling the logits in place, with gradients on: F.linear's result allows it."""
+    torch.manual_seed(4)
+    cfg = MoCConfig(hidden_size=128, intermediate_size=344, num_hidden_layers=1, num_attention_heads=2,
+                    vocab_size=1000, max_seq_len=64)
+    m = build_model(cfg, "moc").to("cuda", dtype)
+    ids = torch.randint(0, 1000, (2, 9), device="cuda")
+    with torch.autocast("cuda", dtype=BF, enabled=dtype == torch.float32):
+        got, want = m(ids), m(ids).clone()
+        assert type(got.grad_fn).__name__ == "_LMHeadBackward"
+        for y in (got, want):
+            y[..., 7] = -1.0
+            y.div_(2.0)
+    grads = [torch.autograd.grad(y, m.lm_head.weight, torch.ones_like(y))[0] for y in (got, want)]
+    assert torch.equal(got, want) and torch.equal(*grads)
+    assert (grads[0][7] == 0).all()
