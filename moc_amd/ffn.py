@@ -200,7 +200,7 @@ def _layer_forward(x, x2, gate_w, up_w, down_w, k, selection: str, idx_dtype, sa
              u_s.data_ptr(), N.ptr(s_s), N.ptr(z_s), out.data_ptr(), d_out, N.ptr(ws), nbytes,
              N.stream_of(x2))
     shp = (*x.shape[:-1], kk)
-    return (out.reshape(*x.shape[:-1], d_out), idx.reshape(shp), vals.reshape(shp), u_s.reshape(shp),
+    return (K.unaliased(out, (*x.shape[:-1], d_out)), idx.reshape(shp), vals.reshape(shp), u_s.reshape(shp),
             None if s_s is None else s_s.reshape(shp), None if z_s is None else z_s.reshape(shp))
 
 
@@ -260,7 +260,7 @@ def _forward_common(x, gate_w, up_w, down_w, k, selection: str, idx_dtype, save_
     del z_full
     kk = idx.shape[-1]
     shp = (*x.shape[:-1], kk)
-    res = (out.reshape(*x.shape[:-1], down_w.shape[0]), idx.reshape(shp), vals.reshape(shp),
+    res = (K.unaliased(out, (*x.shape[:-1], down_w.shape[0])), idx.reshape(shp), vals.reshape(shp),
            u_s.reshape(shp), None if s_s is None else s_s.reshape(shp),
            None if z_s is None else z_s.reshape(shp))
     if not want_mask:
@@ -689,7 +689,7 @@ class _MoCBlockFunction(torch.autograd.Function):
         ctx.gcp = gcp
         ctx.eps = eps
         ctx.h_shape = h.shape
-        return out.reshape(h.shape)
+        return K.unaliased(out, h.shape)
 
     @staticmethod
     def backward(ctx, dout):
@@ -746,7 +746,7 @@ class _MoCBlockF32Function(torch.autograd.Function):
             ctx.save_for_backward(h2, xn, rstd, norm_w, sel, vals, u_s, s_s, z_s, gate_w, up_w, down_w)
         ctx.k, ctx.inter, ctx.bitmask, ctx.gcp, ctx.h_shape = idx.shape[-1], inter, bitmask, gcp, h.shape
         ctx.native = native
-        return out.reshape(h.shape)
+        return K.unaliased(out, h.shape)
 
     @staticmethod
     def backward(ctx, dout):

@@ -62,11 +62,14 @@ def cu_count(device_index: int) -> int:
     return n
 
 
+_unsafe_view = torch.ops.aten._unsafe_view.default
+
+
 def unaliased(t: torch.Tensor, shape) -> torch.Tensor:
     """t, made by the caller and used nowhere else, in another shape and no
     view of t: what a custom Function returns.  Autograd lets no result of a
     Function that is a view be written in place."""
-    return torch.ops.aten._unsafe_view(t, shape)
+    return _unsafe_view(t, shape)
 
 
 def gemm_tiles(m: int, n: int) -> int:

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 import moc_amd.block as B
-from moc_amd import MoCConfig
+from moc_amd import MoCConfig, build_ffn
 from moc_amd import kernels as K
 from moc_amd.model import CausalSelfAttention, RMSNorm, TransformerBlock, rotary_tables
 
@@ -216,3 +216,33 @@ def test_one_call_passes_equal_the_separate_launches(mode, dtype, tokens):
             assert (a - b).norm() <= 1e-5 * b.norm() + (2e-3 * b.norm() if a.shape == h.shape else 0)
         else:
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype,tokens,inter", [(BF, 80, 512), (F32, 80, 512), (F32, 80, 333), (BF, 80, 333),
+                                                (BF, 1, 512), (F32, 1, 512)])
+def test_block_output_takes_writes_in_place(dtype, tokens, inter):
+    """A forward hook that adds to the stream in place, as h + ffn(norm(h)) allows."""
+    torch.manual_seed(5)
+    cfg = MoCConfig(hidden_size=256, intermediate_size=inter, num_hidden_layers=1, num_attention_heads=4,
+                    vocab_size=32)
+    blk = TransformerBlock(cfg, "moc").to("cuda", dtype)
+    x = torch.randn(1, tokens, 256, device="cuda").to(dtype).requires_grad_()
+    with torch.autocast("cuda", dtype=BF, enabled=dtype == F32):
+        want = blk(x)
+        hook = blk.register_forward_hook(lambda m, a, y: y.add_(1.0))
+        got = blk(x)
+        hook.remove()
+    assert torch.equal(got, want + 1)
+    assert all(torch.equal(*g) for g in zip(*(torch.autograd.grad(y, [x, *blk.parameters()], y.detach().sign())
+                                              for y in (got, want + 1))))
+
+
+@pytest.mark.parametrize("dtype", [BF, F32])
+def test_ffn_output_takes_writes_in_place(dtype):
+    ffn = build_ffn(256, 512, "moc", k=128).to("cuda", dtype)
+    x = torch.randn(2, 40, 256, device="cuda").to(dtype).requires_grad_()
+    want = ffn(x)
+    got = ffn(x)
+    got.mul_(2.0)
+    assert torch.equal(got, 2 * want)
+    assert torch.equal(torch.autograd.grad(got.sum(), x)[0], torch.autograd.grad((2 * want).sum(), x)[0])
