@@ -219,7 +219,7 @@ def test_one_call_passes_equal_the_separate_launches(mode, dtype, tokens):
 
 
 @pytest.mark.parametrize("dtype,tokens,inter", [(BF, 80, 512), (F32, 80, 512), (F32, 80, 333), (BF, 80, 333),
-                                                (BF, 1, 512), (F32, 1, 512)])
+                                                (BF, 2, 512), (F32, 2, 512)])
 def test_block_output_takes_writes_in_place(dtype, tokens, inter):
     """A forward hook that adds to the stream in place, as h + ffn(norm(h)) allows."""
     torch.manual_seed(5)
