@@ -243,11 +243,17 @@ int moc_ffn_infer_bf16(int64_t rows, int64_t d, int64_t inter, int64_t k, int se
  * are not ignore_index (moc/model.py:139-144); vocab a multiple of 8 up to
  * 65536, at most 2^22 positions.  forward: loss (loss_dtype), and for the backward lse [batch seq] and
  * inv_count [1]; row_loss [batch seq] is scratch.  A label outside the
- * vocabulary makes the loss and its row's lse and gradient NaN.  backward: dlogits bf16 (rows ldd apart, zeros
+ * vocabulary makes the loss and its row's lse and gradient NaN.  _keep: also a
+ * copy of the logits (rows ldk apart; NULL: none), for a backward that has to
+ * see them as they were.  backward: dlogits bf16 (rows ldd apart, zeros
  * where there is no label) from grad_loss, a device scalar of loss_dtype. */
 int moc_next_token_loss_forward(const void* logits, int64_t ld, int64_t batch, int64_t seq, int64_t vocab,
                                 const int64_t* labels, int64_t ignore_index, float* lse, float* row_loss,
                                 void* loss, int loss_dtype, float* inv_count, void* stream);
+int moc_next_token_loss_forward_keep(const void* logits, int64_t ld, int64_t batch, int64_t seq, int64_t vocab,
+                                     const int64_t* labels, int64_t ignore_index, float* lse, float* row_loss,
+                                     void* loss, int loss_dtype, float* inv_count, void* keep, int64_t ldk,
+                                     void* stream);
 int moc_next_token_loss_backward(const void* logits, int64_t ld, int64_t batch, int64_t seq, int64_t vocab,
                                  const int64_t* labels, int64_t ignore_index, const float* lse,
                                  const float* inv_count, const void* grad_loss, int loss_dtype,

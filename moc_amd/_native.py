@@ -78,6 +78,8 @@ SIGNATURES: dict[str, tuple] = {
                                      _int, _vp, _vp, _i64, _vp]),
     "moc_next_token_loss_forward": (_int, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _vp, _int, _vp,
                                            _vp]),
+    "moc_next_token_loss_forward_keep": (_int, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _vp, _int, _vp,
+                                                _vp, _i64, _vp]),
     "moc_next_token_loss_backward": (_int, [_vp, _i64, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _vp, _int, _vp,
                                             _i64, _vp]),
     "moc_attention_half_saved_size": (_i64, [_i64, _i64, _i64, _i64, _int]),

@@ -248,34 +248,43 @@ def next_token_loss(logits, labels, ignore_index: int = -100) -> torch.Tensor:
     logits, f32 under autocast (as autocast runs it), else bf16;
     next_token_loss_ok must hold."""
     f32 = torch.is_autocast_enabled("cuda")
-    return _NextTokenLoss.apply(logits, labels.contiguous(), ignore_index, F32 if f32 else BF16)
+    return _NextTokenLoss.apply(logits, labels.contiguous(), ignore_index, F32 if f32 else BF16)[0]
 
 
 class _NextTokenLoss(torch.autograd.Function):
+    """(loss, the logits as it saw them, which nobody else holds): the backward
+    reads the second, so a caller may write its logits in place before it."""
+
     @staticmethod
     def forward(ctx, logits, labels, ignore_index, dtype):
         b, s, v = logits.shape
         buf = torch.empty(2 * b * s + 1, dtype=F32, device=logits.device)  # lse, row losses, 1 / count
         loss = torch.empty((), dtype=dtype, device=logits.device)
+        seen = torch.empty_like(logits) if ctx.needs_input_grad[0] else None
         p = buf.data_ptr()
-        N.call("moc_next_token_loss_forward", logits.data_ptr(), v, b, s, v, labels.data_ptr(), ignore_index, p,
-               p + 4 * b * s, loss.data_ptr(), N.dtype_code(dtype), p + 8 * b * s, N.stream_of(logits))
-        ctx.save_for_backward(logits, labels, buf)
+        N.call("moc_next_token_loss_forward_keep", logits.data_ptr(), v, b, s, v, labels.data_ptr(), ignore_index, p,
+               p + 4 * b * s, loss.data_ptr(), N.dtype_code(dtype), p + 8 * b * s, N.ptr(seen), v,
+               N.stream_of(logits))
+        ctx.save_for_backward(seen, labels, buf)
         ctx.ignore_index = ignore_index
-        return loss
+        ctx.set_materialize_grads(False)
+        return loss, seen
 
     @staticmethod
-    def backward(ctx, g):
-        logits, labels, buf = ctx.saved_tensors
+    def backward(ctx, g, g_seen):
+        if g is None:  # the second pass of a second derivative: d seen / d logits
+            return g_seen, None, None, None
+        seen, labels, buf = ctx.saved_tensors
         if torch.is_grad_enabled():  # a graph of the gradient is wanted: the stock loss has one
-            x = logits[:, :-1].flatten(0, 1)
+            x = seen[:, :-1].flatten(0, 1)
             loss = F.cross_entropy(x.float() if g.dtype == F32 else x, labels[:, 1:].flatten(),
                                    ignore_index=ctx.ignore_index)
-            return torch.autograd.grad(loss, logits, g, create_graph=True)[0], None, None, None
-        b, s, v = logits.shape
-        d = torch.empty_like(logits)
-        g = g.contiguous()
-        p = buf.data_ptr()
-        N.call("moc_next_token_loss_backward", logits.data_ptr(), v, b, s, v, labels.data_ptr(), ctx.ignore_index, p,
-               p + 8 * b * s, g.data_ptr(), N.dtype_code(g.dtype), d.data_ptr(), v, N.stream_of(logits))
-        return d, None, None, None
+            d = torch.autograd.grad(loss, seen, g, create_graph=True)[0]
+        else:
+            b, s, v = seen.shape
+            d = torch.empty_like(seen)
+            g = g.contiguous()
+            p = buf.data_ptr()
+            N.call("moc_next_token_loss_backward", seen.data_ptr(), v, b, s, v, labels.data_ptr(), ctx.ignore_index,
+                   p, p + 8 * b * s, g.data_ptr(), N.dtype_code(g.dtype), d.data_ptr(), v, N.stream_of(seen))
+        return d if g_seen is None else d + g_seen, None, None, None

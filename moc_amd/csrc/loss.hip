@@ -6,8 +6,10 @@
 // and writes f32 log-probabilities, their gradient, its bf16 cast and the
 // gradient of the shift: about ten passes over [tokens, vocab].  Here the
 // forward reads the logits once where they are and keeps one f32 per token
-// (the log of the sum of exponentials); the backward reads them once and
-// writes the gradient once, zeros at the positions without a label included.
+// (the log of the sum of exponentials) and, for a backward, their copy (a caller
+// may change its logits in place before it; the stock loss keeps its own
+// log-probabilities); the backward reads them once and writes the gradient
+// once, zeros at the positions without a label included.
 // Bound: HBM traffic (4096 x 32000: 262 MB forward, 524 MB backward): 70 us
 // (3.7 TB/s) and 88 us (6.0 TB/s, part of the logits still in the last-level
 // cache) there, against 190 + 123 and 123 + 161 + 166 us of the stock launches.
@@ -51,31 +53,40 @@ __device__ __forceinline__ int64_t label_of(const int64_t* __restrict__ labels, 
 // One workgroup per row: the row in registers (NC chunks a thread), its maximum,
 // the sum of exponentials; lse[r] and loss[r] (0 where ignored; NaN for a
 // label outside the vocabulary, which the stock loss refuses: the loss and that
-// row's gradient are then NaN).
+// row's gradient are then NaN).  keep (may be null): every row's copy.
 template <int NC>
 __global__ __launch_bounds__(kCeThreads) void ce_forward_kernel(const uint16_t* __restrict__ x, int64_t ld, int vocab,
                                                                 int seq, const int64_t* __restrict__ labels,
                                                                 int64_t ignore, float* __restrict__ lse,
-                                                                float* __restrict__ loss) {
+                                                                float* __restrict__ loss,
+                                                                uint16_t* __restrict__ keep, int64_t ldk) {
   __shared__ float red[kCeThreads / 64];
   const int64_t r = blockIdx.x;
   const int tid = threadIdx.x;
   const int64_t label = label_of(labels, r, seq, ignore);
+  const uint16_t* row = x + r * ld;
+  const int n8 = vocab / 8;
   if (label == ignore) {  // uniform over the workgroup
+    if (keep != nullptr)
+      for (int c = tid; c < n8; c += kCeThreads)
+        reinterpret_cast<uint4*>(keep + r * ldk)[c] = reinterpret_cast<const uint4*>(row)[c];
     if (tid == 0) {
       lse[r] = 0.f;
       loss[r] = 0.f;
     }
     return;
   }
-  const uint16_t* row = x + r * ld;
-  const int n8 = vocab / 8;
   uint4 v[NC];
   // all loads in flight before the first is used (95 -> 70 us at 4096 x 32000):
   // past the end a thread reads the last chunk again, which leaves the maximum
   // and is not summed
 #pragma unroll
   for (int i = 0; i < NC; ++i) v[i] = reinterpret_cast<const uint4*>(row)[min(tid + kCeThreads * i, n8 - 1)];
+  if (keep != nullptr) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (tid + kCeThreads * i < n8) reinterpret_cast<uint4*>(keep + r * ldk)[tid + kCeThreads * i] = v[i];
+  }
   float mx = -INFINITY;
 #pragma unroll
   for (int i = 0; i < NC; ++i) {
@@ -190,20 +201,24 @@ int ce_check(const char* name, const void* x, int64_t ld, int64_t batch, int64_t
 
 using namespace moc;
 
-extern "C" int moc_next_token_loss_forward(const void* logits, int64_t ld, int64_t batch, int64_t seq, int64_t vocab,
-                                           const int64_t* labels, int64_t ignore_index, float* lse, float* row_loss,
-                                           void* loss, int loss_dtype, float* inv_count, void* stream) {
+extern "C" int moc_next_token_loss_forward_keep(const void* logits, int64_t ld, int64_t batch, int64_t seq,
+                                                int64_t vocab, const int64_t* labels, int64_t ignore_index, float* lse,
+                                                float* row_loss, void* loss, int loss_dtype, float* inv_count,
+                                                void* keep, int64_t ldk, void* stream) {
   int rc = ce_check("moc_next_token_loss_forward", logits, ld, batch, seq, vocab, labels);
   if (rc != MOC_OK) return rc;
   MOC_REQUIRE(lse && row_loss && loss && inv_count && (loss_dtype == MOC_BF16 || loss_dtype == MOC_F32),
               "moc_next_token_loss_forward: null output or bad loss dtype");
+  MOC_REQUIRE(keep == nullptr || (aligned16(keep) && ldk % 8 == 0 && ldk >= vocab),
+              "moc_next_token_loss_forward: the copy needs 16-byte aligned rows");
   hipStream_t st = as_stream(stream);
   const int64_t rows = batch * seq;
   const dim3 grid(static_cast<unsigned>(rows));
   const int nc = static_cast<int>((vocab / 8 + kCeThreads - 1) / kCeThreads);
 #define MOC_CE(N)                                                                                             \
   ce_forward_kernel<N><<<grid, kCeThreads, 0, st>>>(static_cast<const uint16_t*>(logits), ld, (int)vocab, (int)seq, \
-                                                    labels, ignore_index, lse, row_loss)
+                                                    labels, ignore_index, lse, row_loss,                       \
+                                                    static_cast<uint16_t*>(keep), ldk)
   if (nc <= 2) MOC_CE(2);
   else if (nc <= 4) MOC_CE(4);
   else if (nc <= 8) MOC_CE(8);
@@ -216,6 +231,13 @@ extern "C" int moc_next_token_loss_forward(const void* logits, int64_t ld, int64
   else
     ce_mean_kernel<false><<<1, 1024, 0, st>>>(row_loss, rows, (int)seq, labels, ignore_index, loss, inv_count);
   return check_launch("ce_mean_kernel");
+}
+
+extern "C" int moc_next_token_loss_forward(const void* logits, int64_t ld, int64_t batch, int64_t seq, int64_t vocab,
+                                           const int64_t* labels, int64_t ignore_index, float* lse, float* row_loss,
+                                           void* loss, int loss_dtype, float* inv_count, void* stream) {
+  return moc_next_token_loss_forward_keep(logits, ld, batch, seq, vocab, labels, ignore_index, lse, row_loss, loss,
+                                          loss_dtype, inv_count, nullptr, 0, stream);
 }
 
 extern "C" int moc_next_token_loss_backward(const void* logits, int64_t ld, int64_t batch, int64_t seq, int64_t vocab,

@@ -41,6 +41,41 @@ def test_loss_and_gradient(batch, seq, vocab, autocast):
     assert (grad[:, -1] == 0).all()
 
 
+@pytest.mark.parametrize("autocast", [True, False])
+@pytest.mark.parametrize("batch,seq,vocab", [(1, 2, 8), (3, 5, 4104), (2, 9, 32000), (1, 3, 65536)])
+def test_logits_may_change_between_loss_and_backward(batch, seq, vocab, autocast):
+    """The gradient is that of the logits the loss saw, as with the stock loss,
+    which keeps its own log-probabilities."""
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    leaf = torch.randn(batch, seq, vocab, generator=g, device="cuda").to(BF).requires_grad_()
+    labels = torch.randint(0, vocab, (batch, seq), generator=g, device="cuda")
+    labels[0, 1] = -100
+    if seq * batch == 2:
+        labels[0, 1] = 3
+    x, y = leaf * 3, leaf * 3
+    with torch.autocast("cuda", dtype=BF, enabled=autocast):
+        a, b = next_token_loss(x, labels), next_token_loss(y, labels)
+    with torch.no_grad():
+        x.div_(0.7)
+        x[..., 0] = -float("inf")
+    want, = torch.autograd.grad(b, leaf)
+    for _ in range(2):
+        got, = torch.autograd.grad(a, leaf, retain_graph=True)
+        assert torch.equal(got, want)
+
+
+def test_loss_without_gradient_keeps_no_copy():
+    x = torch.randn(4, 64, 32000, device="cuda").to(BF)
+    labels = torch.randint(0, 32000, (4, 64), device="cuda")
+    with torch.no_grad():
+        next_token_loss(x, labels)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        base = torch.cuda.memory_allocated()
+        next_token_loss(x, labels)
+    assert torch.cuda.max_memory_allocated() - base < x.numel()
+
+
 def test_all_ignored_and_bad_labels_are_nan():
     x = torch.randn(2, 4, 64, device="cuda").to(BF)
     assert torch.isnan(next_token_loss(x, torch.full((2, 4), -100, device="cuda")))
