@@ -10,9 +10,10 @@
 // may change its logits in place before it; the stock loss keeps its own
 // log-probabilities); the backward reads them once and writes the gradient
 // once, zeros at the positions without a label included.
-// Bound: HBM traffic (4096 x 32000: 262 MB forward, 524 MB backward): 70 us
-// (3.7 TB/s) and 88 us (6.0 TB/s, part of the logits still in the last-level
-// cache) there, against 190 + 123 and 123 + 161 + 166 us of the stock launches.
+// Bound: HBM traffic (4096 x 32000: 262 MB forward, as much again for the copy,
+// 524 MB backward): 68 us (3.8 TB/s), 110 with the copy, and 88 us (6.0 TB/s,
+// part of the logits still in the last-level cache) there, against 190 + 123 and
+// 123 + 161 + 166 us of the stock launches.
 #include "abi.h"
 #include "common.h"
 
