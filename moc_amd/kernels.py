@@ -764,7 +764,11 @@ def global_after_gate(x, gate_scores, up_weight, down_weight_t, k: int, *, works
         vals, idx, _ = topk_rows(g, int(k), idx_dtype=torch.int32)
         u = linear(x, wu, out=padded_empty(nb, inter, torch.bfloat16, x.device))
         z = sparse_forward_aux(vals, idx, u, inter, want_s=False, want_z=False)[3]
-        yy = gemm(z, wdt, residual=None if residual is None else residual.reshape(nb, hidden))
+        r = None if residual is None else residual.reshape(nb, hidden)
+        if r is None or r.dtype == torch.bfloat16:
+            yy = gemm(z, wdt, residual=r)
+        else:  # the sum in the type that residual and layer promote to
+            yy = r + gemm(z, wdt)
         if idx_out is not None:
             idx_out.copy_(idx)
         if out is None:

@@ -138,3 +138,19 @@ def test_layer_with_norm_takes_unaligned_views(nb, grouped):
             xf = x.float()
             xn = (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-6)).to(BF) * w
             assert torch.equal(y, x + m(xn))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.float16, BF])
+def test_after_gate_adds_a_residual_of_any_type(dtype):
+    """More than 16 tokens: residual + the layer, in the sum's own type."""
+    x, w = _case(20, 64, 200, 11)
+    wdt = K.down_weight_t_for_decode(w[2])
+    g = K.linear(x, w[0])
+    res = torch.randn(20, 64, device="cuda").to(dtype)
+    plain = K.global_after_gate(x, g, w[1], wdt, 50)
+    got = K.global_after_gate(x, g, w[1], wdt, 50, residual=res)
+    want = res + plain
+    assert got.dtype == want.dtype and torch.equal(got, want)
+    out = torch.empty(20, 64, dtype=BF, device="cuda")
+    assert K.global_after_gate(x, g, w[1], wdt, 50, residual=res, out=out) is out
+    assert torch.equal(out, want.to(BF))
