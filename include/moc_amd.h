@@ -267,7 +267,9 @@ int moc_next_token_loss_backward(const void* logits, int64_t ld, int64_t batch, 
  * bf16.  batch seq >= 2, heads of 64 or 128, hidden up to 4096; contiguous,
  * 16-byte aligned.  saved: written by the forward, read by the backward
  * (moc_attention_half_saved_size); y_tmp [tokens, hidden] bf16 (f32 = 1);
- * scratch: no contents kept; workspace: as moc_gemm_ws uses it. */
+ * scratch: no contents kept; workspace: as moc_gemm_ws uses it.  backward: a
+ * NULL dw_qkv, dw_out, or dx with dnorm_w (both or neither) leaves its products
+ * out. */
 int64_t moc_attention_half_saved_size(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim, int f32);
 int64_t moc_attention_half_scratch_size(int64_t batch, int64_t seq, int64_t heads, int64_t head_dim, int f32);
 int64_t moc_attention_half_workspace_size(int64_t tokens, int64_t d);

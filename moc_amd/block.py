@@ -146,10 +146,12 @@ class _AttentionHalf(torch.autograd.Function):
             dh = dh.clone()
         scratch = torch.empty(nscratch, dtype=torch.uint8, device=dev)
         ws = K._gemm_workspace(dev, nws) if nws > 0 else None
-        dx, dn, dq, do = (torch.empty_like(t) for t in (x, norm_w, qkv_w, out_w))
+        stream, norm, qkv, out = ctx.needs_input_grad[:4]  # dx and dn come from one kernel
+        dx, dn, dq, do = (torch.empty_like(t) if need else None for t, need in (
+            (x, stream or norm), (norm_w, stream or norm), (qkv_w, qkv), (out_w, out)))
         N.call("moc_attention_half_backward", batch, seq, heads, d // heads, f32, dh.data_ptr(), x.data_ptr(),
                norm_w.data_ptr(), qkv_w.data_ptr(), out_w.data_ptr(), cos.data_ptr(), sin.data_ptr(), ctx.scale,
-               saved.data_ptr(), saved.numel(), dx.data_ptr(), dn.data_ptr(), dq.data_ptr(), do.data_ptr(),
+               saved.data_ptr(), saved.numel(), N.ptr(dx), N.ptr(dn), N.ptr(dq), N.ptr(do),
                scratch.data_ptr(), nscratch, N.ptr(ws), nws, N.stream_of(x))
         return dx, dn, dq, do, None, None, None, None
 

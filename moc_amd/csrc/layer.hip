@@ -522,8 +522,9 @@ extern "C" int moc_attention_half_backward(int64_t batch, int64_t seq, int64_t h
               "moc_attention_half_backward: two tokens or more, heads of 64 or 128, hidden up to 4096");
   const AttnHalf a = attn_half(batch, seq, heads, head_dim, f32);
   const int64_t t = a.t, d = a.d;
-  MOC_REQUIRE(dh && x && norm_w && w_qkv && w_out && saved && dx && dnorm_w && dw_qkv && dw_out && scratch,
+  MOC_REQUIRE(dh && x && norm_w && w_qkv && w_out && saved && scratch && (dx != nullptr) == (dnorm_w != nullptr),
               "moc_attention_half_backward: null pointer");
+  if (dx == nullptr && dw_qkv == nullptr && dw_out == nullptr) return MOC_OK;
   MOC_REQUIRE(moc::aligned16(dh) && moc::aligned16(x) && moc::aligned16(w_qkv) && moc::aligned16(w_out) &&
                   moc::aligned16(saved) && moc::aligned16(dx) && moc::aligned16(scratch),
               "moc_attention_half_backward: operands must be 16-byte aligned");
@@ -548,22 +549,26 @@ extern "C" int moc_attention_half_backward(int64_t batch, int64_t seq, int64_t h
     if (rc != MOC_OK) return rc;
     go = dst[0];
   }
-  // dW_out = go^T o, do = go W_out
-  rc = moc_gemm_ws(MOC_BF16, d, d, t, go, 1, d, o, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dw_out, d, gdt, workspace,
-                   workspace_bytes, stream);
-  if (rc == MOC_OK)
-    rc = moc_gemm_ws(MOC_BF16, t, d, d, go, d, 1, wo, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dox, d, MOC_BF16,
-                     workspace, workspace_bytes, stream);
+  // dW_out = go^T o
+  if (dw_out != nullptr) {
+    rc = moc_gemm_ws(MOC_BF16, d, d, t, go, 1, d, o, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dw_out, d, gdt, workspace,
+                     workspace_bytes, stream);
+    if (rc != MOC_OK) return rc;
+  }
+  if (dx == nullptr && dw_qkv == nullptr) return MOC_OK;
+  // do = go W_out
+  rc = moc_gemm_ws(MOC_BF16, t, d, d, go, d, 1, wo, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dox, d, MOC_BF16,
+                   workspace, workspace_bytes, stream);
   if (rc == MOC_OK)
     rc = moc_rope_attention_backward_bf16(batch, seq, heads, head_dim, qkv, 3 * d, cos, sin, gdt, scale, o, lse, dox,
                                           reinterpret_cast<float*>(s + a.delta), dqkv, stream);
   // dW_qkv = dqkv^T xn, dxn = dqkv W_qkv (in do's place)
-  if (rc == MOC_OK)
+  if (rc == MOC_OK && dw_qkv != nullptr)
     rc = moc_gemm_ws(MOC_BF16, 3 * d, d, t, dqkv, 1, 3 * d, xn, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dw_qkv, d, gdt,
                      workspace, workspace_bytes, stream);
-  if (rc == MOC_OK)
-    rc = moc_gemm_ws(MOC_BF16, t, d, 3 * d, dqkv, 3 * d, 1, wq, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dox, d,
-                     MOC_BF16, workspace, workspace_bytes, stream);
+  if (rc != MOC_OK || dx == nullptr) return rc;
+  rc = moc_gemm_ws(MOC_BF16, t, d, 3 * d, dqkv, 3 * d, 1, wq, d, 1, 0, nullptr, 0, 0, nullptr, 0, 0, dox, d,
+                   MOC_BF16, workspace, workspace_bytes, stream);
   if (rc != MOC_OK) return rc;
   void* part = s + a.rms;
   const int64_t pbytes = a.scratch - a.rms;

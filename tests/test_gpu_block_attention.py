@@ -246,3 +246,35 @@ def test_ffn_output_takes_writes_in_place(dtype):
     got.mul_(2.0)
     assert torch.equal(got, 2 * want)
     assert torch.equal(torch.autograd.grad(got.sum(), x)[0], torch.autograd.grad((2 * want).sum(), x)[0])
+
+
+@pytest.mark.parametrize("dtype", [BF, F32])
+@pytest.mark.parametrize("wanted", [("x",), ("qkv",), ("out",), ("norm",), ("x", "out"), ("norm", "qkv"), ("qkv", "out"),
+                                    ("x", "norm", "qkv", "out")])
+def test_attention_half_leaves_frozen_operands_out(dtype, wanted):
+    """Only what needs a gradient gets one, the same bits as with all of them,
+    and the products of the others are not computed."""
+    norm, attn = _pair(dtype, 256, 4, 40, 3)
+    x = torch.randn(2, 40, 256, device="cuda").to(dtype).requires_grad_()
+    dh = torch.randn(2, 40, 256, device="cuda").to(dtype)
+    leaf = {"x": x, "norm": norm.weight, "qkv": attn.qkv_proj.weight, "out": attn.out_proj.weight}
+
+    def grads(names):
+        for n, t in leaf.items():
+            t.requires_grad_(n in names)
+        with torch.autocast("cuda", dtype=BF, enabled=dtype == F32):
+            y = B.attention_half(x, norm, attn)
+        seen, call = [], B.N.call
+        B.N.call = lambda name, *a: seen.append((name, a)) or call(name, *a)
+        try:
+            return dict(zip(names, torch.autograd.grad(y, [leaf[n] for n in names], dh))), seen[-1]
+        finally:
+            B.N.call = call
+
+    every, _ = grads(tuple(leaf))
+    some, (name, args) = grads(wanted)
+    assert name == "moc_attention_half_backward"
+    assert all(torch.equal(some[n], every[n]) for n in wanted)
+    dx, dn, dq, do = args[15:19]
+    assert ("qkv" in wanted) == (dq is not None) and ("out" in wanted) == (do is not None)
+    assert (dx is None) == (dn is None) == (not {"x", "norm"} & set(wanted))
