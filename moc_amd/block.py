@@ -19,7 +19,6 @@ from functools import lru_cache
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
-from torch.autograd.function import once_differentiable
 from torch.nn.modules.module import _has_any_global_hook
 
 from . import _native as N
@@ -67,6 +66,22 @@ def bare(*modules) -> bool:
         for m in modules)
 
 
+def graph_grads(half, inputs, needs, grad):
+    """The gradients of half(*inputs) with a graph of their own, for a backward
+    that is to be differentiated: half is written in f32 tensor operations, which
+    have derivatives of every order (autocast off), inputs are the Function's."""
+    wanted = [t for t, need in zip(inputs, needs) if need]
+    with torch.autocast("cuda", enabled=False):
+        out = half(*inputs)
+        grads = iter(torch.autograd.grad(out, wanted, grad.to(out.dtype), create_graph=True))
+    return [next(grads) if need else None for need in needs]
+
+
+def rms_norm_f32(x, w, eps: float):
+    """x / rms(x) * w of an f32 x."""
+    return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + eps) * w.float()
+
+
 def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:
     """True if attention_half takes this block: plain modules of the model's
     own types in the stream's dtype, heads of 64 or 128, hidden up to 4096, two
@@ -108,6 +123,19 @@ def _sizes(device_index: int, batch: int, seq: int, heads: int, head_dim: int, f
             N.query("moc_attention_half_workspace_size", batch * seq, heads * head_dim))
 
 
+def _attention_f32(x, norm_w, qkv_w, out_w, cos, sin, eps: float, heads: int):
+    """x + out_proj(attention(norm(x))) in f32 tensor operations."""
+    b, n, d = x.shape
+    q, k, v = F.linear(rms_norm_f32(x.float(), norm_w, eps), qkv_w.float()).view(b, n, 3, heads, d // heads).permute(
+        2, 0, 3, 1, 4)
+    c, s = cos[:n].float(), sin[:n].float()
+    q, k = (torch.stack((t[..., 0::2] * c - t[..., 1::2] * s, t[..., 0::2] * s + t[..., 1::2] * c), -1).flatten(-2)
+            for t in (q, k))
+    later = torch.ones(n, n, dtype=torch.bool, device=x.device).triu(1)
+    p = torch.softmax((q @ k.transpose(-1, -2) / math.sqrt(d // heads)).masked_fill(later, -math.inf), -1)
+    return x + F.linear((p @ v).permute(0, 2, 1, 3).reshape(b, n, d), out_w.float())
+
+
 class _AttentionHalf(torch.autograd.Function):
     """One native call per pass; between them one buffer of the forward's
     results (norm output, q/k/v, attention output, row factors and, under
@@ -116,7 +144,7 @@ class _AttentionHalf(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, norm_w, qkv_w, out_w, cos, sin, eps, heads):
         batch, seq, d = x.shape
-        x = x.contiguous()
+        given, x = x, x.contiguous()
         f32 = int(x.dtype == F32)
         dev = x.device
         nsaved, _, nws = _sizes(dev.index, batch, seq, heads, d // heads, f32)
@@ -128,14 +156,17 @@ class _AttentionHalf(torch.autograd.Function):
         N.call("moc_attention_half_forward", batch, seq, heads, d // heads, f32, x.data_ptr(), norm_w.data_ptr(),
                eps, qkv_w.data_ptr(), out_w.data_ptr(), cos.data_ptr(), sin.data_ptr(), scale, h.data_ptr(),
                saved.data_ptr(), nsaved, N.ptr(y), N.ptr(ws), nws, N.stream_of(x))
-        ctx.save_for_backward(x, norm_w, qkv_w, out_w, cos, sin, saved)
-        ctx.heads, ctx.scale = heads, scale
+        ctx.save_for_backward(given, norm_w, qkv_w, out_w, cos, sin, saved)
+        ctx.heads, ctx.scale, ctx.eps = heads, scale, eps
         return h
 
     @staticmethod
-    @once_differentiable
     def backward(ctx, dh):
         x, norm_w, qkv_w, out_w, cos, sin, saved = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return (*graph_grads(lambda *t: _attention_f32(*t, cos, sin, ctx.eps, ctx.heads),
+                                 (x, norm_w, qkv_w, out_w), ctx.needs_input_grad[:4], dh), None, None, None, None)
+        x = x.contiguous()
         batch, seq, d = x.shape
         heads = ctx.heads
         f32 = int(x.dtype == F32)

@@ -26,7 +26,7 @@ import torch.nn.functional as F
 
 from . import _native as N
 from . import kernels as K
-from .block import runs_stock, stock_method
+from .block import graph_grads, rms_norm_f32, runs_stock, stock_method
 
 _MODES = (
     "moc",
@@ -656,6 +656,18 @@ def _block_native(h2, wg, wu, wd) -> bool:
         _layer_ok(h2, wg, wu, wd)
 
 
+def _block_graph_grads(ctx, inputs, idx, dout):
+    """The gradients of h + FFN(RMSNorm(h)) with a graph, the selection as saved
+    (a constant)."""
+    def half(h, norm_w, gate_w, up_w, down_w):
+        xn = rms_norm_f32(h.float(), norm_w, ctx.eps)
+        g, u = F.linear(xn, gate_w.float()), F.linear(xn, up_w.float())
+        mask = torch.zeros(g.shape, device=g.device).scatter_(-1, idx.reshape(*g.shape[:-1], -1).long(), 1.0)
+        return h + F.linear(F.silu(g) * u * mask, down_w.float())
+
+    return (*graph_grads(half, inputs, ctx.needs_input_grad[:5], dout), *[None] * 6)
+
+
 class _MoCBlockFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, h, norm_w, gate_w, up_w, down_w, eps, k, index_save_dtype, use_triton_aux, selection,
@@ -679,10 +691,11 @@ class _MoCBlockFunction(torch.autograd.Function):
             mask = mk[0] if mk else None
             del xn
         sel = _saved_index(idx, mask, bitmask)
+        # h itself: a backward that is to be differentiated needs its graph
         if gcp:
-            ctx.save_for_backward(h2, rstd, norm_w, sel, vals, u_s, gate_w, up_w, down_w)
+            ctx.save_for_backward(h, rstd, norm_w, sel, vals, u_s, gate_w, up_w, down_w)
         else:
-            ctx.save_for_backward(h2, rstd, norm_w, sel, vals, u_s, s_s, z_s, gate_w, up_w, down_w)
+            ctx.save_for_backward(h, rstd, norm_w, sel, vals, u_s, s_s, z_s, gate_w, up_w, down_w)
         ctx.k = idx.shape[-1]
         ctx.inter = inter
         ctx.bitmask = bitmask
@@ -694,12 +707,15 @@ class _MoCBlockFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         if ctx.gcp:
-            h2, rstd, norm_w, saved, g_s, u_s, wg, wu, wd = ctx.saved_tensors
+            h, rstd, norm_w, saved, g_s, u_s, wg, wu, wd = ctx.saved_tensors
             s_s = z_s = None
         else:
-            h2, rstd, norm_w, saved, g_s, u_s, s_s, z_s, wg, wu, wd = ctx.saved_tensors
+            h, rstd, norm_w, saved, g_s, u_s, s_s, z_s, wg, wu, wd = ctx.saved_tensors
         idx = _restore_index(ctx, saved)
-        d = h2.shape[1]
+        if torch.is_grad_enabled():
+            return _block_graph_grads(ctx, (h, norm_w, wg, wu, wd), idx, dout)
+        d = h.shape[-1]
+        h2 = K.aligned_rows(h.reshape(-1, d))
         go = K.aligned_rows(dout.reshape(-1, d).to(h2.dtype))
         if _block_native(h2, wg, wu, wd) and _layer_ok(go) and \
                 (not ctx.gcp or K.row_pitch(ctx.inter, h2.dtype) <= 8192):
@@ -741,21 +757,24 @@ class _MoCBlockF32Function(torch.autograd.Function):
         sel = _saved_index(idx, mask[0] if mask else None, bitmask)
         # the parameters, not their casts: the backward casts them again
         if gcp:
-            ctx.save_for_backward(h2, xn, rstd, norm_w, sel, vals, u_s, gate_w, up_w, down_w)
+            ctx.save_for_backward(h, xn, rstd, norm_w, sel, vals, u_s, gate_w, up_w, down_w)
         else:
-            ctx.save_for_backward(h2, xn, rstd, norm_w, sel, vals, u_s, s_s, z_s, gate_w, up_w, down_w)
+            ctx.save_for_backward(h, xn, rstd, norm_w, sel, vals, u_s, s_s, z_s, gate_w, up_w, down_w)
         ctx.k, ctx.inter, ctx.bitmask, ctx.gcp, ctx.h_shape = idx.shape[-1], inter, bitmask, gcp, h.shape
-        ctx.native = native
+        ctx.native, ctx.eps = native, eps
         return K.unaliased(out, h.shape)
 
     @staticmethod
     def backward(ctx, dout):
         if ctx.gcp:
-            h2, xn, rstd, norm_w, saved, g_s, u_s, gate_w, up_w, down_w = ctx.saved_tensors
+            h, xn, rstd, norm_w, saved, g_s, u_s, gate_w, up_w, down_w = ctx.saved_tensors
             s_s = z_s = None
         else:
-            h2, xn, rstd, norm_w, saved, g_s, u_s, s_s, z_s, gate_w, up_w, down_w = ctx.saved_tensors
+            h, xn, rstd, norm_w, saved, g_s, u_s, s_s, z_s, gate_w, up_w, down_w = ctx.saved_tensors
         idx = _restore_index(ctx, saved)
+        if torch.is_grad_enabled():
+            return _block_graph_grads(ctx, (h, norm_w, gate_w, up_w, down_w), idx, dout)
+        h2 = h.reshape(-1, h.shape[-1])
         d2 = dout.reshape(h2.shape).contiguous()
         if ctx.native and d2.data_ptr() % 16 == 0 and d2.dtype == torch.float32 and (
                 not ctx.gcp or K.row_pitch(ctx.inter, torch.bfloat16) <= 8192):

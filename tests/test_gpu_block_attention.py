@@ -278,3 +278,72 @@ def test_attention_half_leaves_frozen_operands_out(dtype, wanted):
     dx, dn, dq, do = args[15:19]
     assert ("qkv" in wanted) == (dq is not None) and ("out" in wanted) == (do is not None)
     assert (dx is None) == (dn is None) == (not {"x", "norm"} & set(wanted))
+
+
+def _dense_block64(x, blk, heads):
+    """The block in 64 bits with every channel selected."""
+    def norm(t, m):
+        return t * torch.rsqrt(t.square().mean(-1, keepdim=True) + m.eps) * p[m.weight]
+
+    p = {q: q.detach().to(F64).requires_grad_() for q in blk.parameters()}
+    a, f = blk.attn, blk.ffn
+    n, d = x.shape[1:]
+    q, k, v = (norm(x, blk.attn_norm) @ p[a.qkv_proj.weight].t()).view(-1, n, 3, heads, d // heads).permute(2, 0, 3, 1, 4)
+    c, s = a.rope_cos[:n].to(F64), a.rope_sin[:n].to(F64)
+    q, k = _rot(q, c, s), _rot(k, c, s)
+    sc = q @ k.transpose(-1, -2) / math.sqrt(d // heads) + torch.full((n, n), -math.inf, device="cuda", dtype=F64).triu(1)
+    h = x + (torch.softmax(sc, -1) @ v).permute(0, 2, 1, 3).reshape(x.shape) @ p[a.out_proj.weight].t()
+    t = norm(h, blk.ffn_norm)
+    g, u, w = (p[m.weight] for m in (f.gate_proj, f.up_proj, f.down_proj))
+    return h + (torch.nn.functional.silu(t @ g.t()) * (t @ u.t())) @ w.t(), list(p.values())
+
+
+@pytest.mark.parametrize("mode", ["moc", "moc_gcp"])
+@pytest.mark.parametrize("dtype,seq,inter", [(BF, 20, 344), (F32, 20, 344), (BF, 20, 333), (F32, 20, 333)])
+def test_block_second_derivative(mode, dtype, seq, inter):
+    """A gradient penalty through a whole block, every channel selected so that
+    rounding moves no selection, against 64 bits."""
+    torch.manual_seed(6)
+    cfg = MoCConfig(hidden_size=128, intermediate_size=inter, num_hidden_layers=1, num_attention_heads=2,
+                    vocab_size=32, k=inter)
+    blk = TransformerBlock(cfg, mode).to("cuda", dtype)
+    x = torch.randn(2, seq, 128, device="cuda").to(dtype).requires_grad_()
+    dy = torch.randn(2, seq, 128, device="cuda").to(dtype)
+
+    def penalty(y, xx, ps, dd):
+        gx, = torch.autograd.grad(y, xx, dd, create_graph=True)
+        return torch.autograd.grad(gx.to(F64).square().sum(), [xx, *ps])
+
+    with torch.autocast("cuda", dtype=BF, enabled=dtype == F32):
+        y = blk(x)
+    got = penalty(y, x, list(blk.parameters()), dy)
+    xd = x.detach().to(F64).requires_grad_()
+    yd, ps = _dense_block64(xd, blk, 2)
+    want = penalty(yd, xd, ps, dy.to(F64))
+    for a, b, q in zip(got, want, [x, *blk.parameters()]):
+        assert a.dtype == q.dtype
+        # operands and stream of bf16 (2^-9 each): the forward's values, the
+        # stream between the halves and, for a bf16 block, each cotangent that
+        # passes it are rounded once or twice
+        assert (a.to(F64) - b).norm() <= 8 * 2.0 ** -9 * b.norm(), ((a.to(F64) - b).norm() / b.norm()).item()
+
+
+@pytest.mark.parametrize("mode", ["moc", "moc_2_8", "moc_post_silu_abs"])
+def test_block_second_derivative_of_a_selection(mode):
+    """Selected channels only: zero where no token selects a channel."""
+    torch.manual_seed(7)
+    cfg = MoCConfig(hidden_size=128, intermediate_size=344, num_hidden_layers=1, num_attention_heads=2,
+                    vocab_size=32, k=3)
+    blk = TransformerBlock(cfg, mode).to("cuda", BF)
+    x = torch.randn(1, 2, 128, device="cuda").to(BF).requires_grad_()
+    y = blk(x)
+    to = [x, blk.ffn.gate_proj.weight, *blk.parameters()]
+    first = torch.autograd.grad(y, to, torch.ones_like(y), create_graph=True)
+    plain = torch.autograd.grad(blk(x), to, torch.ones_like(y))
+    for a, b in zip(first, plain):
+        assert a.grad_fn is not None and (a.float() - b.float()).norm() <= 2e-2 * b.float().norm()
+    unused = (plain[1] == 0).all(1)
+    dg, = torch.autograd.grad(first[0].float().square().sum(), blk.ffn.gate_proj.weight)
+    assert dg.abs().max() > 0
+    if mode != "moc_2_8":
+        assert unused.any() and (dg[unused] == 0).all()
