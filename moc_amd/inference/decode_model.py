@@ -215,7 +215,16 @@ class DecoderLayer(nn.Module):
                 and _plain(a, n, a.qkv_proj, a.out_proj) and a.k_t is not None and a.k_t.shape[0] == 1
                 and _one_token_native(x, n.weight, a.qkv_proj.weight, a.out_proj.weight, a.rope_cos, a.rope_sin,
                                       a.k_t, a.v)
-                and K.decode_attention_fits(a.hidden, a.heads, a.max_seq))
+                and self._attn_shapes(x.shape[-1]) and K.decode_attention_fits(a.hidden, a.heads, a.max_seq))
+
+    def _attn_shapes(self, h: int) -> bool:
+        """Weights, tables and caches are those of K.decode_attention (another
+        module's may broadcast, which the kernels do not)."""
+        a, hd, s = self.attn, self.attn.head_dim, self.attn.max_seq
+        return (h == a.hidden == a.heads * hd and self.attn_norm.weight.shape == (h,)
+                and a.qkv_proj.weight.shape == (3 * h, h) and a.out_proj.weight.shape == (h, h)
+                and a.rope_cos.shape == a.rope_sin.shape == (s, hd // 2)
+                and a.k_t.shape == (1, a.heads, hd, s) and a.v.shape == (1, a.heads, s, hd))
 
     def forward_step(self, x: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
         if self._attn_native(x):
@@ -286,7 +295,8 @@ class DecoderModel(nn.Module):
     def _head_native(self, x: torch.Tensor) -> bool:
         n, head = self.final_norm, self.lm_head
         return (self.fuse_head and type(n) is RMSNorm and _plain(n, head) and self.cfg.hidden % 8 == 0
-                and self.cfg.hidden <= 4096 and _one_token_native(x, n.weight, head.weight))
+                and self.cfg.hidden <= 4096 and _one_token_native(x, n.weight, head.weight)
+                and n.weight.shape == x.shape[-1:] and head.weight.shape[1:] == x.shape[-1:])
 
 
 def make_step(model: DecoderModel, scope: str) -> Callable[[torch.Tensor, int], torch.Tensor]:

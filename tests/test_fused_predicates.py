@@ -11,6 +11,7 @@ from moc_amd import MoCConfig, build_model
 from moc_amd.block import attention_half_ok, lm_head_ok
 from moc_amd.ffn import block_ffn_f32_ok, block_ffn_ok
 from moc_amd.inference.decode_model import DecodeConfig, DecoderModel
+from moc_amd.inference.decode_model import RMSNorm as DecodeNorm
 from moc_amd.model import CausalSelfAttention, RMSNorm, TransformerBlock
 
 BF = torch.bfloat16
@@ -281,3 +282,31 @@ def test_ffn_half_calls_a_norm_of_another_type():
         h = x + blk.attn(blk.attn_norm(x))
         want = h + blk.ffn(2 * RMSNorm.forward(blk.ffn_norm, h))
     assert (got.float() - want.float()).norm() <= 2e-2 * want.float().norm()
+
+
+@pytest.mark.parametrize("change", [
+    lambda la: setattr(la, "attn_norm", DecodeNorm(1).to(BF)),
+    lambda la: [setattr(la.attn, n, torch.cat([getattr(la.attn, n)] * 2)) for n in ("rope_cos", "rope_sin")],
+    lambda la: setattr(la.attn, "out_proj", _linear(256, 128)),
+    lambda la: setattr(la.attn, "qkv_proj", _linear(256, 512)),
+    lambda la: setattr(la.attn, "v", la.attn.v[:, :, :4].clone()),
+    lambda la: setattr(la.attn, "k_t", la.attn.k_t[:, :2].clone()),
+], ids=["broadcast norm", "longer tables", "narrow out_proj", "narrow qkv_proj", "short v", "fewer heads"])
+def test_decode_attention_takes_only_its_shapes(on_device, change):
+    layer, x = _decoder().layers[0], torch.zeros(1, 1, 256, dtype=BF)
+    with torch.no_grad():
+        assert layer._attn_native(x)
+        change(layer)
+        assert not layer._attn_native(x)
+
+
+@pytest.mark.parametrize("change", [
+    lambda m: setattr(m, "final_norm", DecodeNorm(1).to(BF)),
+    lambda m: setattr(m, "lm_head", _linear(128, 64)),
+], ids=["broadcast norm", "head of another input"])
+def test_decode_head_takes_only_its_shapes(on_device, change):
+    model, x = _decoder(), torch.zeros(1, 1, 256, dtype=BF)
+    with torch.no_grad():
+        assert model._head_native(x)
+        change(model)
+        assert not model._head_native(x)
