@@ -82,11 +82,27 @@ def rms_norm_f32(x, w, eps: float):
     return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + eps) * w.float()
 
 
+# Longest sequence of the fused half; from there on the stock composition over
+# the library's attention is as fast or faster.  Stock time over fused, forward +
+# backward, 4096 tokens a pass (the last column one sequence of 8192):
+#   hidden, heads of        256    1024   4096   8192
+#   bf16 1024, 64           3.72   2.37   1.17   0.98
+#   bf16 1024, 128          3.50   1.98   1.18   0.78
+#   bf16 2048, 64           2.14   1.67   1.03   0.96
+#   bf16 2048, 128          1.99   1.56   1.00   0.76
+#   f32  1024, 64           3.83   2.70   1.40   1.17
+#   f32  2048, 128             -   1.71   1.12   0.84
+# (forward alone 0.97 to 2.0 at 4096, 0.65 to 1.4 at 8192; one sequence of 2 to
+# 2048 positions 1.3 to 8.5).
+MAX_SEQ = 4096
+
+
 def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:
     """True if attention_half takes this block: plain modules of the model's
-    own types in the stream's dtype, heads of 64 or 128, hidden up to 4096, two
-    tokens or more (a gradient product over one token has no aligned operand).
-    Every shape is compared: the kernels take their sizes from x alone."""
+    own types in the stream's dtype, heads of 64 or 128, hidden up to 4096, up
+    to MAX_SEQ positions, two tokens or more (a gradient product over one token
+    has no aligned operand).  Every shape is compared: the kernels take their
+    sizes from x alone."""
     if not FUSE_BLOCK_ATTENTION or type(norm) is not norm_type or type(attn) is not attn_type or x.dim() != 3:
         return False
     dt = stream_dtype(x)
@@ -96,7 +112,7 @@ def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:
         return False
     d = x.shape[-1]
     if attn.head_dim not in (64, 128) or d != attn.num_heads * attn.head_dim or d > 4096 or x.numel() < 2 * d or \
-            x.shape[0] > 65535:
+            x.shape[0] > 65535 or x.shape[1] > MAX_SEQ:
         return False
     cos = attn.rope_cos
     if norm.weight.shape != (d,) or qkv.weight.shape != (3 * d, d) or out.weight.shape != (d, d) or \

@@ -310,3 +310,11 @@ def test_decode_head_takes_only_its_shapes(on_device, change):
         assert model._head_native(x)
         change(model)
         assert not model._head_native(x)
+
+
+def test_attention_half_leaves_long_sequences_to_the_library(on_device):
+    cfg = MoCConfig(hidden_size=256, intermediate_size=512, num_hidden_layers=1, num_attention_heads=4,
+                    vocab_size=32, max_seq_len=8192)
+    blk = TransformerBlock(cfg, "moc").to(BF)
+    assert _attn_ok(blk, torch.zeros(1, 4096, 256, dtype=BF))
+    assert not _attn_ok(blk, torch.zeros(1, 4097, 256, dtype=BF))
