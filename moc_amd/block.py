@@ -227,17 +227,25 @@ def lm_head(h, norm, weight) -> torch.Tensor:
 def _own_head_dx(tokens: int, d: int) -> bool:
     """dX contracts over the vocabulary into few tiles: the library's product
     leaves most CUs idle, the engine's splits K.  Library and engine, us, of 32000
-    words: 93 / 21 (16 tokens, d 512), 106 / 34 (512, 512), 295 / 128 (4096,
-    512), 327 / 224 (4096, 1024), 427 / 406 (4096, 2048), the last of the range
-    where the engine was ahead."""
+    words: 93 / 44 (16 tokens, d 512), 104 / 32 (512, 512), 289 / 127 (4096,
+    512), 325 / 227 (4096, 1024), 427 / 406 (4096, 2048), the last of the range
+    where the engine was ahead.  1000 to 128256 words: the engine at most 4 %
+    behind anywhere in it (8192 words, d 1024, 8192 tokens: 117 / 121)."""
     return tokens * d <= 1 << 23
 
 
 def _own_head_dw(d: int, vocab: int) -> bool:
-    """dW, library and engine, us: 139 / 113 (32000 words, d 512, 4096 tokens),
-    250 / 210 (d 1024), 494 / 421 (d 2048); but 25 / 43 (d 256, 1024 tokens) and
-    25 / 38 (8192 words, d 1024, 1024 tokens), where half of the CUs get no tile."""
-    return d >= 512 and vocab >= 16384
+    """dW on the engine where its 256-wide tiles fill their rounds of 256 CUs:
+    0.8 of one round, 0.7 of several.  Library and engine, us, 4096 tokens: 131 /
+    108 (32000 words, d 512: 250 tiles), 109 / 108 (26624: 208), 249 / 210 (32000,
+    d 1024: 500), 178 / 171 (16384, d 1536: 384); but 68 / 75 (16384, d 512: 128;
+    23 / 37 at 1024 tokens), 90 / 98 (24576: 192), 124 / 169 (24576, d 640: 288).
+    Narrower or with fewer words the engine is ahead or behind by the token count
+    (32000 words, d 256, 512 tokens 20 / 18; 8192, d 1024, 8192 tokens 137 / 123)
+    and the library keeps them."""
+    tiles = -(-d // 256) * -(-vocab // 256)
+    rounds = -(-tiles // 256)
+    return d >= 512 and vocab >= 16384 and tiles >= (0.8 if rounds == 1 else 0.7) * 256 * rounds
 
 
 class _LMHead(torch.autograd.Function):

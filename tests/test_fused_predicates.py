@@ -8,7 +8,7 @@ import torch.nn as nn
 from torch.nn.modules.module import register_module_forward_hook
 
 from moc_amd import MoCConfig, build_model
-from moc_amd.block import attention_half_ok, lm_head_ok
+from moc_amd.block import _own_head_dw, attention_half_ok, lm_head_ok
 from moc_amd.ffn import block_ffn_f32_ok, block_ffn_ok
 from moc_amd.inference.decode_model import DecodeConfig, DecoderModel
 from moc_amd.inference.decode_model import RMSNorm as DecodeNorm
@@ -318,3 +318,13 @@ def test_attention_half_leaves_long_sequences_to_the_library(on_device):
     blk = TransformerBlock(cfg, "moc").to(BF)
     assert _attn_ok(blk, torch.zeros(1, 4096, 256, dtype=BF))
     assert not _attn_ok(blk, torch.zeros(1, 4097, 256, dtype=BF))
+
+
+@pytest.mark.parametrize("d,vocab,own", [(512, 16384, False), (512, 24576, False), (512, 26624, True), (512, 32000, True),
+                                         (576, 16384, False), (640, 20480, True), (640, 24576, False),
+                                         (768, 24576, False), (768, 32000, True), (1024, 16384, True),
+                                         (1536, 16384, True), (2048, 32000, True), (256, 32000, False),
+                                         (1024, 8192, False)])
+def test_head_weight_gradient_takes_the_engine_where_its_rounds_fill(d, vocab, own):
+    """Each side is the faster one measured (_own_head_dw)."""
+    assert _own_head_dw(d, vocab) == own
