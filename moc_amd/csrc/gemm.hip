@@ -43,6 +43,7 @@
 //
 // f32 operands use a plain FMA kernel (parity path for f32 models).
 #include <algorithm>
+#include <cmath>
 
 #include "abi.h"
 #include "common.h"
@@ -1901,8 +1902,9 @@ SplitPlan plan_split(int64_t M, int64_t N, int nk) {
 }
 
 // The small-tile plan of a product [M, N] (with n2 > 0: of the pair [M, N],
-// [M, n2] side by side, never split over K), bm = 0 where the 256-wide tiles
-// are as fast or faster.  Measured on both sides (bf16, cold weights):
+// [M, n2] side by side, never split over K), bm = 0 where its 256x256 tiles
+// fill too many CUs: more than 0.35 of them (a pair: all), or more than 24 K
+// tiles per CU together (a pair: 21).  Measured on both sides (bf16):
 //   M x N x K              256-wide plans      small tiles
 //   pair   48 x 5461 x 2048   39.1 us      64 x 64          15.6 us
 //   pair  200 x 5461 x 2048   52.1         128 x 64         25.2
@@ -1914,29 +1916,30 @@ SplitPlan plan_split(int64_t M, int64_t N, int nk) {
 //       8192 x 768 x 2048     32.0         128 x 128        33.7
 //       2048 x 2048 x 10912   95.3         128 x 128, in 2  99.5
 //       4096 x 2736 x 1024    27.6         128 x 128        33.7
-//       1280 x 3398 x 5000    60.9, 3 parts  128 x 128, in 2  79.3
-//       1619 x 1728 x 7546    56.9, 5 parts  128 x 128, in 4  67.8
-//       1280 x 2605 x 6200    56.8, 4 parts  128 x 128, in 2  53.8
 //   pair 1619 x 3773 x 1728   74.6         128 x 64         78.5
 //   pair 1779 x 3547 x 1728   75.5         128 x 128        71.9
-// so a product takes small tiles while its 256x256 tiles are at most 0.35 of
-// the CUs (a pair: fewer than the CUs) and hold at most 24 K tiles per CU
-// together (a pair: 21), unless plan_split fills nearly all CUs and is
-// predicted far ahead: kper K tiles of 1.4 us, 5.5 us of prologue and
-// reduction and its partials' bytes (within 8 % of 12 such shapes).  The line
-// is 1.42 times that, where the two sides measure equal (the small tiles'
-// prediction is up to a third high where K is long).  Among the small tiles the least predicted time wins: a K tile
-// takes t1 us with one workgroup on a CU and t2 with two, each workgroup t0
-// more, a K split one reduction launch and its partials' bytes; the model
-// is within 10 % of the table above and of 40 shapes around it.
+// Among the small tiles the least cost wins: a K tile takes t1 with one
+// workgroup on a CU and t2 with two, each workgroup t0 more, a K split one
+// reduction launch and its partials' bytes.
+//
+// What the chosen plan is predicted to take (us), which decides against the
+// other plans of a single product (wide_us), has constants of its own, fitted
+// to the device times of the 408 products and pairs of such a sweep that took
+// small tiles (17 to 12000 rows, 4 to 164 K tiles): within 20 %, 6 % in the
+// mean.  The costs above are up to half high where K is long (1280 x 2605 x
+// 6200: 70 against 54 us) and a third low for the shortest.
 MidPlan plan_mid(int64_t M, int64_t N, int nk, int64_t n2, int64_t ws_bytes) {
   struct Tile {
     int bm, bn;
-    double t1, t2, t0;
+    double t1, t2, t0;  // cost
+    double m1, m2, m0;  // the same, measured
   };
-  constexpr Tile kTiles[] = {{64, 64, 0.37, 0.50, 2.5}, {64, 128, 0.45, 0.71, 3.0}, {128, 64, 0.48, 0.70, 3.0},
-                             {128, 128, 0.72, 1.16, 3.0}};
+  constexpr Tile kTiles[] = {{64, 64, 0.37, 0.50, 2.5, 0.338, 0.508, 3.3},
+                             {64, 128, 0.45, 0.71, 3.0, 0.414, 0.615, 4.5},
+                             {128, 64, 0.48, 0.70, 3.0, 0.402, 0.566, 4.8},
+                             {128, 128, 0.72, 1.16, 3.0, 0.494, 0.772, 6.0}};
   constexpr double kReduce = 3.0, kPartRate = 7.4e6;  // us, bytes a us
+  constexpr double kMReduce = 1.5, kMPart = 0.27, kMPartRate = 6.8e6;  // measured: a launch, each part, its bytes
   MidPlan p;
   const int cus = cu_count();
   auto tiles = [](int64_t m, int64_t n, int bm, int bn) { return ((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
@@ -1944,7 +1947,7 @@ MidPlan plan_mid(int64_t M, int64_t N, int nk, int64_t n2, int64_t ws_bytes) {
   if (M < 1 || N < 1 || nk < 1 || big * nk > 24 * cus) return p;
   if (n2 > 0 ? big >= cus || big * nk > 21 * cus : 20 * big > 7 * cus) return p;
   const int64_t ldw = (N + 3) & ~3LL;
-  const double part_us = 2.0 * M * ldw * 4 / kPartRate;
+  const double part = 2.0 * M * ldw * 4;  // bytes of one part, written and read
   double best = 0;
   for (const Tile& t : kTiles) {
     const int n = static_cast<int>(tiles(M, N, t.bm, t.bn) + (n2 > 0 ? tiles(M, n2, t.bm, t.bn) : 0));
@@ -1955,9 +1958,12 @@ MidPlan plan_mid(int64_t M, int64_t N, int nk, int64_t n2, int64_t ws_bytes) {
       const int64_t bytes = ks > 1 ? kFixCounterBytes + ks * M * ldw * 4 : 0;
       if (bytes > ws_bytes) break;
       const int full = n * ks / (2 * cus), rem = n * ks - full * 2 * cus;
-      const double two = kper * t.t2 + t.t0, one = kper * t.t1 + t.t0;
-      double cost = full * two + (rem == 0 ? 0.0 : rem <= cus ? one : two);
-      if (ks > 1) cost += kReduce + ks * part_us;
+      auto rounds = [&](double t1, double t2, double t0) {
+        const double two = kper * t2 + t0, one = kper * t1 + t0;
+        return full * two + (rem == 0 ? 0.0 : rem <= cus ? one : two);
+      };
+      double cost = rounds(t.t1, t.t2, t.t0);
+      if (ks > 1) cost += kReduce + ks * part / kPartRate;
       if (p.bm == 0 || cost < best) {
         best = cost;
         p.bm = t.bm;
@@ -1966,16 +1972,9 @@ MidPlan plan_mid(int64_t M, int64_t N, int nk, int64_t n2, int64_t ws_bytes) {
         p.kper = kper;
         p.ldw = ldw;
         p.bytes = bytes;
-        p.us = best;
+        p.us = rounds(t.m1, t.m2, t.m0) + (ks > 1 ? kMReduce + ks * (kMPart + part / kMPartRate) : 0.0);
       }
     }
-  }
-  if (n2 == 0) {
-    constexpr double kMargin = 1.42, kTile = 1.4, kEnds = 5.5;
-    const SplitPlan sp = plan_split(M, N, nk);
-    if (sp.ksplit >= 3 && sp.bytes <= ws_bytes &&
-        p.us > kMargin * (sp.kper * kTile + kEnds + sp.ksplit * part_us))
-      return MidPlan();
   }
   return p;
 }
@@ -1996,6 +1995,7 @@ MidPlan plan_mid(int64_t M, int64_t N, int nk, int64_t n2, int64_t ws_bytes) {
 struct FixPlan {
   int full = 0, tail = 0, split = 0;
   int64_t bytes = 0;
+  int64_t cost = 0;  // K-tile times
 };
 
 FixPlan plan_fix_tiles(int64_t tiles, int nk) {
@@ -2016,6 +2016,7 @@ FixPlan plan_fix_tiles(int64_t tiles, int nk) {
   if (best_s == 0) return f;
   f.tail = static_cast<int>(tiles);
   f.split = static_cast<int>(best_s);
+  f.cost = best;
   f.bytes = kFixCounterBytes + tiles * 2 * kPartBytes;
   return f;
 }
@@ -2037,6 +2038,45 @@ FixPlan plan_fix_short(int64_t M, int64_t N, int nk) {
   const int64_t tiles256 = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
   if (3 * tiles256 > cu_count() || nk > kShortFixMaxKTiles) return FixPlan();
   return plan_fix_tiles(((M + 127) / 128) * ((N + kBN - 1) / kBN), nk);
+}
+
+// 128-row tiles when 256 x 256 tiles would fill more than a quarter but at
+// most half of the CUs and K is short (the 130m layer's D: 96 tiles, 32 K
+// tiles): twice the tiles run whole, where 256 x 256 tiles need a two-part
+// K split whose f32 partial tile (256 KB) passes through one CU per tile
+// (45 -> 40 us).  A 128-row tile runs its K tiles at ~0.7 of the 256-row
+// tile's rate per FLOP (half the MFMA work per phase, more than half the
+// fragment reads), so for long K the split wins (the 130m dX, 64 K tiles:
+// 72 us split against 78 us).
+bool short_whole_ok(int64_t M, int64_t N, int nk) {
+  const int64_t tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN), cus = cu_count();
+  return 4 * tiles > cus && 2 * tiles <= cus && nk <= kShortMaxKTiles;
+}
+
+// Predicted time of the plan that a product takes without small tiles, us, for
+// the comparison with MidPlan::us; HUGE_VAL where none was measured ahead.
+// a_kc: A's rows are K-contiguous, as the 128-row tiles need; two: a sum of two
+// products.  Fitted to device times: 75 whole products on 128-row tiles (4 % in
+// the mean), 49 on them in two K parts (8 %) and 179 K splits (9 %); the last two
+// have to be predicted 10 and 5 % ahead, which is where the choice went wrong
+// least over the 345 products timed on both sides.  On both sides, us:
+//   7086 x 704 x 1699   25.5 (128 rows)     28.7 (128 x 128)
+//   2048 x 2560 x 2560  34.5 (128 rows)     38.2 (128 x 128)
+//   9216 x 328 x 1376   21.3 (128 rows)     18.5 (128 x 64)
+//   3346 x 1216 x 2824  40.2 (128, 2 parts) 45.4 (64 x 64)
+//   3604 x 712 x 5544   45.6 (5 parts)      53.6 (128 x 128, in 4)
+//   1280 x 3398 x 5000  60.8 (3 parts)      79.3 (128 x 128, in 2)
+//   1280 x 2605 x 6200  56.2 (4 parts)      52.9 (128 x 128, in 2)
+double wide_us(int64_t M, int64_t N, int nk, bool two, bool a_kc, int64_t ws_bytes) {
+  if (a_kc && short_whole_ok(M, N, nk)) return 5.8 + 0.74 * nk + (two ? 2 : 0);
+  if (a_kc) {
+    const FixPlan f = plan_fix_short(M, N, nk);
+    if (f.tail > 0 && f.bytes <= ws_bytes) return (11.6 + 0.73 * f.cost) / 0.9;
+  }
+  const SplitPlan s = plan_split(M, N, nk);
+  if (s.ksplit > 1 && s.bytes <= ws_bytes)
+    return (9.7 + 1.23 * s.kper + s.ksplit * 2.0 * M * s.ldw * 4 / 6.8e6) / 0.95;
+  return HUGE_VAL;
 }
 
 // Two split-K products in one launch (the layer backward's weight gradients
@@ -2082,9 +2122,11 @@ PairSplitPlan plan_split_pair(int64_t M1, int64_t N1, int nk1, int64_t M2, int64
     }
   }
   if (pick[0] == 0) return r;
-  // the two products apart on small tiles, where both take them
+  // the two products apart on small tiles, where both take them: faster by 24 to
+  // 4 % in 27 layer backwards where those are predicted below 1.25 us a K-tile
+  // time of this plan, level up to 1.42, up to 20 % slower above
   const MidPlan mid[2] = {plan_mid(M1, N1, nk1, 0, INT64_MAX), plan_mid(M2, N2, nk2, 0, INT64_MAX)};
-  constexpr double kTileUs = 1.2;
+  constexpr double kTileUs = 1.35;
   if (mid[0].bm > 0 && mid[1].bm > 0 && mid[0].us + mid[1].us < best * kTileUs) return r;
   r.bytes = kFixCounterBytes;
   for (int i = 0; i < 2; ++i) {
@@ -2473,10 +2515,10 @@ int gemm_ws_impl(int dtype, int64_t M, int64_t N, int64_t K, const void* A, int6
   };
   a.pp = no_wrap(a.a[0]) && no_wrap(a.b[0]) && no_wrap(a.a[1]) && no_wrap(a.b[1]);
   // small tiles (a K split only with a workspace for its partials)
-  const MidPlan mp = a.pp ? plan_mid(M, N, a.nk[0] + a.nk[1], 0,
-                                     workspace != nullptr && aligned16(workspace) ? workspace_bytes : 0)
-                          : MidPlan();
-  if (mp.bm > 0) {
+  const int nk_all = a.nk[0] + a.nk[1];
+  const int64_t ws_have = workspace != nullptr && aligned16(workspace) ? workspace_bytes : 0;
+  const MidPlan mp = a.pp ? plan_mid(M, N, nk_all, 0, ws_have) : MidPlan();
+  if (mp.bm > 0 && mp.us <= wide_us(M, N, nk_all, a.nk[1] > 0, la == 1, ws_have)) {
     GemmArgs run = a;
     run.tiles_m = static_cast<int>((M + mp.bm - 1) / mp.bm);
     run.tiles_n = static_cast<int>((N + mp.bn - 1) / mp.bn);
@@ -2502,18 +2544,7 @@ int gemm_ws_impl(int dtype, int64_t M, int64_t N, int64_t K, const void* A, int6
                                                         ldc, a.vec_store, a.res, a.ldres);
     return check_launch("splitk_reduce_kernel");
   }
-  // 128-row tiles when 256 x 256 tiles would fill more than a quarter but at
-  // most half of the CUs and K is short (the 130m layer's D: 96 tiles, 32 K
-  // tiles): twice the tiles run whole, where 256 x 256 tiles need a two-part
-  // K split whose f32 partial tile (256 KB) passes through one CU per tile
-  // (45 -> 40 us).  A 128-row tile runs its K tiles at ~0.7 of the 256-row
-  // tile's rate per FLOP (half the MFMA work per phase, more than half the
-  // fragment reads), so for long K the split wins (the 130m dX, 64 K tiles:
-  // 72 us split against 78 us).
-  const int64_t cus = cu_count();
-  const int64_t tiles256 = static_cast<int64_t>(a.tiles_m) * a.tiles_n;
-  const bool short_whole = a.pp && la == 1 && 4 * tiles256 > cus && 2 * tiles256 <= cus &&
-                           a.nk[0] + a.nk[1] <= kShortMaxKTiles;
+  const bool short_whole = a.pp && la == 1 && short_whole_ok(M, N, a.nk[0] + a.nk[1]);
   // 128-row tiles in two K parts instead of a K split (see plan_fix_short)
   const FixPlan sfp = a.pp && la == 1 && !short_whole ? plan_fix_short(M, N, a.nk[0] + a.nk[1]) : FixPlan();
   const bool short_fix = sfp.tail > 0 && workspace != nullptr && workspace_bytes >= sfp.bytes &&

@@ -87,3 +87,16 @@ def test_without_workspace():
     N.call("moc_gemm_ws", N.MOC_BF16, m, n, k, a.data_ptr(), a.stride(0), 1, b.data_ptr(), b.stride(0), 1, 0,
            None, 0, 0, None, 0, 0, out.data_ptr(), n, N.MOC_BF16, None, 0, N.stream_of(a))
     _check(out, a.double() @ b.double(), a.double().abs() @ b.double().abs(), k)
+
+
+@pytest.mark.parametrize("m,n,k", [(7086, 704, 1699), (2048, 2560, 520), (9216, 328, 1376), (3346, 1216, 2824),
+                                   (3604, 712, 5544)])
+@pytest.mark.parametrize("b_kc", [True, False])
+def test_plans_on_either_side_of_the_small_tiles_line(m, n, k, b_kc):
+    """128-row tiles, small tiles, 128-row tiles in two parts, a K split."""
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a, b = _mat(m, k, gen), _mat(k, n, gen, not b_kc)
+    ref, mags = a.double() @ b.double(), a.double().abs() @ b.double().abs()
+    _check(K.gemm(a, b), ref, mags, k)
+    res = _mat(m, n, gen)
+    assert torch.equal(K.gemm(a, b, residual=res), (K.gemm(a, b).float() + res.float()).to(BF))
