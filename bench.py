@@ -134,8 +134,9 @@ def cfg5_bench(steps: int, only: str | None = None) -> dict:
     benchmark_training_throughput.py:135), then `steps` timed steps; peak
     memory over the timed steps (the method of
     benchmark_training_throughput.py:51-114 and benchmark_memory.py:51-107).
-    Attention, norms and embeddings are stock PyTorch; the FFN is this
-    build's.  Beside the wall-clock step: the model's algorithmic FLOP over
+    The dense row is stock PyTorch throughout.  The MoC rows run this library's
+    attention half, LM head and loss too, so their ratio to it is not the
+    FFN's alone.  Beside the wall-clock step: the model's algorithmic FLOP over
     it, and one FFN layer of the step's shape timed on its own (GPU-bound,
     so the two FFNs compare without the host's launch time, which at this
     size is close to the GPU's work).  Rows: moc_gcp (the FFN's pre-norm and

@@ -212,7 +212,7 @@ class InferenceMoCSwiGLUFFN(nn.Module):
         """2:8 batches that run as dense products (K.ffn_infer) instead of the
         packed gate/up epilogue and the structured-sparse Down, whose tiles of
         256 tokens leave CUs idle: 2048 -> 5464 at 48 / 200 / 512 / 700 tokens
-        80 / 64 / 75 / 77 us packed, 32 / 45 / 64 / 85 dense; 1024 -> 2736 at
+        80 / 64 / 75 / 77 us packed, 36 / 45 / 64 / 85 dense; 1024 -> 2736 at
         1024 / 1500 tokens 51 / 58 and 43 / 60; 512 -> 1376 at 4096 45 and 41."""
         c = self.config
         return nb > 16 and (nb <= 512 or nb * c.hidden_size * c.intermediate_size <= 3 << 30)
