@@ -299,6 +299,14 @@ class DecoderModel(nn.Module):
                 and n.weight.shape == x.shape[-1:] and head.weight.shape[1:] == x.shape[-1:])
 
 
+def _set_position(pos: torch.Tensor, p: int, max_seq: int) -> None:
+    """pos <- p, refused outside the cache: the fused attention half has no
+    cache row there and gives NaN."""
+    if isinstance(p, int) and not 0 <= p < max_seq:
+        raise ValueError(f"position {p} is outside the cache of {max_seq}")
+    pos.fill_(p)
+
+
 def make_step(model: DecoderModel, scope: str) -> Callable[[torch.Tensor, int], torch.Tensor]:
     """A callable (token ids [1, 1], position) -> logits [1, 1, vocab].
     "whole_graph" captures one step (after warm-up launches on a side
@@ -307,7 +315,7 @@ def make_step(model: DecoderModel, scope: str) -> Callable[[torch.Tensor, int], 
     pos = torch.zeros((), dtype=torch.int64, device=dev)
     if scope == "eager":
         def step(tokens: torch.Tensor, p: int) -> torch.Tensor:
-            pos.fill_(p)
+            _set_position(pos, p, model.cfg.max_seq)
             return model.forward_step(tokens, pos)
         return step
     if scope == "layer_graph":
@@ -329,7 +337,7 @@ def make_step(model: DecoderModel, scope: str) -> Callable[[torch.Tensor, int], 
 
     def step(tokens: torch.Tensor, p: int) -> torch.Tensor:
         tok.copy_(tokens)
-        pos.fill_(p)
+        _set_position(pos, p, model.cfg.max_seq)
         graph.replay()
         return logits
 
@@ -368,7 +376,7 @@ def _layer_graph_step(model: DecoderModel, pos: torch.Tensor) -> Callable[[torch
 
     @torch.no_grad()
     def step(tokens: torch.Tensor, p: int) -> torch.Tensor:
-        pos.fill_(p)
+        _set_position(pos, p, model.cfg.max_seq)
         xs[0].copy_(model.embed(tokens))
         for g in graphs:
             g.replay()

@@ -10,7 +10,7 @@ from torch.nn.modules.module import register_module_forward_hook
 from moc_amd import MoCConfig, build_model
 from moc_amd.block import _own_head_dw, attention_half_ok, lm_head_ok
 from moc_amd.ffn import block_ffn_f32_ok, block_ffn_ok
-from moc_amd.inference.decode_model import DecodeConfig, DecoderModel
+from moc_amd.inference.decode_model import DecodeConfig, DecoderModel, make_step
 from moc_amd.inference.decode_model import RMSNorm as DecodeNorm
 from moc_amd.model import CausalSelfAttention, RMSNorm, TransformerBlock
 
@@ -328,3 +328,29 @@ def test_attention_half_leaves_long_sequences_to_the_library(on_device):
 def test_head_weight_gradient_takes_the_engine_where_its_rounds_fill(d, vocab, own):
     """Each side is the faster one measured (_own_head_dw)."""
     assert _own_head_dw(d, vocab) == own
+
+
+@pytest.mark.parametrize("p", [-1, 8, 100])
+def test_decode_step_refuses_a_position_outside_the_cache(p):
+    """The fused half would return NaN, where the stock composition's indexing refuses."""
+    cfg = DecodeConfig(hidden=64, intermediate=176, heads=4, layers=1, vocab=64, k=32, max_seq=8)
+    m = DecoderModel("dense", cfg)
+    m.allocate_cache()
+    step = make_step(m, "eager")
+    assert step(torch.zeros(1, 1, dtype=torch.int64), 7).shape == (1, 1, 64)
+    with pytest.raises(ValueError, match="position"):
+        step(torch.zeros(1, 1, dtype=torch.int64), p)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scope", ["eager", "layer_graph", "whole_graph"])
+def test_decode_step_refuses_a_position_in_every_scope(scope):
+    cfg = DecodeConfig(hidden=256, intermediate=704, heads=4, layers=2, vocab=64, k=128, max_seq=8)
+    m = DecoderModel("global_moc", cfg).to("cuda", BF).init_weights(1)
+    m.allocate_cache()
+    step = make_step(m, scope)
+    tok = torch.zeros(1, 1, dtype=torch.int64, device="cuda")
+    assert torch.isfinite(step(tok, 7)).all()
+    for p in (-1, 8):
+        with pytest.raises(ValueError, match="position"):
+            step(tok, p)
