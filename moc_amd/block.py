@@ -58,6 +58,12 @@ def runs_stock(m: nn.Module, name: str = "forward") -> bool:
     return name not in m.__dict__ and getattr(type(m), name) in _STOCK
 
 
+def plain(*tensors) -> bool:
+    """Tensors whose storage holds their values, which the kernels read: no
+    subclass (sharded, quantised, ...) with operators of its own."""
+    return all(type(t) is torch.Tensor or type(t) is nn.Parameter for t in tensors)
+
+
 def bare(*modules) -> bool:
     """The modules that a fused half does not call have the forward it computes
     and no hooks, their own or those registered for every module."""
@@ -119,10 +125,10 @@ def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:
             cos.dim() != 2 or cos.shape[0] < x.shape[1] or cos.shape[1] != attn.head_dim // 2 or \
             attn.rope_sin.shape != cos.shape:
         return False
-    if x.is_contiguous() and x.data_ptr() % 16:
+    read = norm.weight, qkv.weight, out.weight, attn.rope_cos, attn.rope_sin
+    if not plain(x, *read) or (x.is_contiguous() and x.data_ptr() % 16):
         return False
-    return all(t.dtype == dt and t.is_contiguous() and t.device == x.device and t.data_ptr() % 16 == 0
-               for t in (norm.weight, qkv.weight, out.weight, attn.rope_cos, attn.rope_sin))
+    return all(t.dtype == dt and t.is_contiguous() and t.device == x.device and t.data_ptr() % 16 == 0 for t in read)
 
 
 def attention_half(x, norm, attn) -> torch.Tensor:
@@ -213,7 +219,8 @@ def lm_head_ok(h, norm, norm_type, head, weight) -> bool:
     if head is not None and (type(head) is not nn.Linear or head.bias is not None or not bare(head)):
         return False
     d = h.shape[-1]
-    if d % 8 or d > 4096 or weight.dim() != 2 or weight.shape[0] % 8 or h.numel() < 2 * d:
+    if not plain(h, norm.weight, weight) or d % 8 or d > 4096 or weight.dim() != 2 or weight.shape[0] % 8 or \
+            h.numel() < 2 * d:
         return False
     return all(t.dtype == dt and t.is_contiguous() and t.device == h.device and t.data_ptr() % 16 == 0
                for t in (h, norm.weight, weight)) and norm.weight.shape == (d,) and weight.shape[1] == d
@@ -293,7 +300,8 @@ class _LMHead(torch.autograd.Function):
 def next_token_loss_ok(logits, labels) -> bool:
     """True if next_token_loss takes these: bf16 device logits whose stock loss
     is f32 (autocast) or bf16, int64 labels of their shape."""
-    return (logits.is_cuda and logits.dtype == BF16 and logits.dim() == 3 and logits.shape[1] >= 2
+    return (plain(logits, labels) and logits.is_cuda and logits.dtype == BF16 and logits.dim() == 3
+            and logits.shape[1] >= 2
             and logits.is_contiguous() and logits.data_ptr() % 16 == 0 and logits.numel() > 0
             and logits.shape[2] % 8 == 0 and logits.shape[2] <= 65536 and logits.shape[0] * logits.shape[1] <= 1 << 22
             and labels.device == logits.device and labels.dtype == torch.int64

@@ -37,7 +37,7 @@ import torch.nn as nn
 from torch.nn.modules.module import _has_any_global_hook
 
 from .. import kernels as K
-from ..block import runs_stock, stock_method
+from ..block import plain, runs_stock, stock_method
 from .inference_ffn import InferenceMoCSwiGLUFFN
 
 HIDDEN = 2048
@@ -176,7 +176,8 @@ def _plain(*modules) -> bool:
 def _one_token_native(x: torch.Tensor, *weights) -> bool:
     """One bf16 token of a gradient-free pass outside autocast, with
     contiguous, aligned bf16 weights on its device (the token aligned too)."""
-    return (x.is_cuda and x.dtype == torch.bfloat16 and x.shape[:2] == (1, 1) and not torch.is_grad_enabled()
+    return (plain(x, *weights) and x.is_cuda and x.dtype == torch.bfloat16 and x.shape[:2] == (1, 1)
+            and not torch.is_grad_enabled()
             and not torch.is_autocast_enabled("cuda") and x.data_ptr() % 16 == 0
             and all(w.dtype == torch.bfloat16 and w.device == x.device and w.is_contiguous()
                     and w.data_ptr() % 16 == 0 for w in weights))

@@ -8,7 +8,7 @@ import torch.nn as nn
 from torch.nn.modules.module import register_module_forward_hook
 
 from moc_amd import MoCConfig, build_model
-from moc_amd.block import _own_head_dw, attention_half_ok, lm_head_ok
+from moc_amd.block import _own_head_dw, attention_half_ok, lm_head_ok, next_token_loss_ok
 from moc_amd.ffn import block_ffn_f32_ok, block_ffn_ok
 from moc_amd.inference.decode_model import DecodeConfig, DecoderModel, make_step
 from moc_amd.inference.decode_model import RMSNorm as DecodeNorm
@@ -354,3 +354,56 @@ def test_decode_step_refuses_a_position_in_every_scope(scope):
     for p in (-1, 8):
         with pytest.raises(ValueError, match="position"):
             step(tok, p)
+
+
+class _Wrapped(torch.Tensor):
+    """Stands for a tensor type of its own (sharded, quantised): its storage is not what the kernels read."""
+
+
+def _wrap(m, name="weight"):
+    old = getattr(m, name)
+    if isinstance(old, nn.Parameter):
+        setattr(m, name, nn.Parameter(old.detach().as_subclass(_Wrapped)))
+    else:
+        setattr(m, name, old.as_subclass(_Wrapped))
+
+
+@pytest.mark.parametrize("part", ["attn_norm.weight", "attn.qkv_proj.weight", "attn.out_proj.weight", "attn.rope_cos", "x"])
+def test_attention_half_leaves_other_tensor_types_alone(on_device, part):
+    blk, x = _block(), torch.zeros(2, 16, 256, dtype=BF)
+    if part == "x":
+        x = x.as_subclass(_Wrapped)
+    else:
+        mod, name = part.rsplit(".", 1)
+        _wrap(blk.get_submodule(mod), name)
+    assert not _attn_ok(blk, x)
+
+
+@pytest.mark.parametrize("part", ["norm", "lm_head", "h"])
+def test_lm_head_leaves_other_tensor_types_alone(on_device, part):
+    norm, head, h = RMSNorm(64).to(BF), _linear(64, 128), torch.zeros(1, 4, 64, dtype=BF)
+    if part == "h":
+        h = h.as_subclass(_Wrapped)
+    else:
+        _wrap(norm if part == "norm" else head)
+    assert not lm_head_ok(h, norm, RMSNorm, head, head.weight)
+
+
+def test_loss_leaves_other_tensor_types_alone(on_device):
+    x, labels = torch.zeros(2, 4, 64, dtype=BF), torch.zeros(2, 4, dtype=torch.int64)
+    assert next_token_loss_ok(x, labels)
+    assert not next_token_loss_ok(x.as_subclass(_Wrapped), labels)
+    assert not next_token_loss_ok(x, labels.as_subclass(_Wrapped))
+
+
+def test_decode_step_leaves_other_tensor_types_alone(on_device):
+    x = torch.zeros(1, 1, 256, dtype=BF)
+    with torch.no_grad():
+        for part in ("attn_norm", "attn.qkv_proj", "attn.out_proj"):
+            layer = _decoder().layers[0]
+            _wrap(layer.get_submodule(part))
+            assert not layer._attn_native(x)
+        for part in ("final_norm", "lm_head"):
+            model = _decoder()
+            _wrap(getattr(model, part))
+            assert not model._head_native(x)
