@@ -776,7 +776,9 @@ class _MoCBlockF32Function(torch.autograd.Function):
             return _block_graph_grads(ctx, (h, norm_w, gate_w, up_w, down_w), idx, dout)
         h2 = h.reshape(-1, h.shape[-1])
         d2 = dout.reshape(h2.shape).contiguous()
-        if ctx.native and d2.data_ptr() % 16 == 0 and d2.dtype == torch.float32 and (
+        if d2.data_ptr() % 16:  # a view into a larger gradient
+            d2 = d2.clone()
+        if ctx.native and d2.dtype == torch.float32 and (
                 not ctx.gcp or K.row_pitch(ctx.inter, torch.bfloat16) <= 8192):
             dh, dnw, dwg, dwu, dwd = _block_backward_f32_native(d2, h2, xn, rstd, norm_w, idx, g_s, u_s, s_s, z_s,
                                                                 gate_w, up_w, down_w, ctx.gcp)

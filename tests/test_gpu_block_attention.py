@@ -363,3 +363,21 @@ def test_rope_attention_rounds_where_the_library_attention_does(seq, dim, table)
     q, k = (rotate_pairs(t, cos, sin).to(BF) for t in (q, k))
     r = torch.nn.functional.scaled_dot_product_attention(q, k, v, is_causal=True)
     assert (o != r.permute(0, 2, 1, 3).reshape(o.shape)).float().mean() <= 5e-3
+
+
+@pytest.mark.parametrize("dtype,inter", [(BF, 512), (F32, 512), (F32, 333)])
+def test_block_takes_a_gradient_off_the_16_byte_grid(dtype, inter):
+    """The gradient of a concatenation is a view into it: that of an aligned copy."""
+    torch.manual_seed(9)
+    cfg = MoCConfig(hidden_size=128, intermediate_size=inter, num_hidden_layers=1, num_attention_heads=2,
+                    vocab_size=32)
+    blk = TransformerBlock(cfg, "moc").to("cuda", dtype)
+    x = torch.randn(2, 20, 128, device="cuda").to(dtype).requires_grad_()
+    dy = torch.randn(2, 20, 128, device="cuda").to(dtype)
+    off = torch.cat((dy.new_zeros(1), dy.flatten()))[1:].view(dy.shape)
+    assert off.data_ptr() % 16 and off.is_contiguous()
+    with torch.autocast("cuda", dtype=BF, enabled=dtype == F32):
+        y = blk(x)
+    want = torch.autograd.grad(y, [x, *blk.parameters()], dy, retain_graph=True)
+    got = torch.autograd.grad(y, [x, *blk.parameters()], off)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
