@@ -88,6 +88,11 @@ def rms_norm_f32(x, w, eps: float):
     return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + eps) * w.float()
 
 
+# Bytes of a bf16 operand the engine addresses (32-bit offsets); larger products
+# are the library's.
+_OPERAND_BYTES = (1 << 31) - 1024
+
+
 # Longest sequence of the fused half; from there on the stock composition over
 # the library's attention is as fast or faster.  Stock time over fused, forward +
 # backward, 4096 tokens a pass (the last column one sequence of 8192):
@@ -118,7 +123,7 @@ def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:
         return False
     d = x.shape[-1]
     if attn.head_dim not in (64, 128) or d != attn.num_heads * attn.head_dim or d > 4096 or x.numel() < 2 * d or \
-            x.shape[0] > 65535 or x.shape[1] > MAX_SEQ:
+            x.shape[0] > 65535 or x.shape[1] > MAX_SEQ or 3 * x.numel() * 2 >= _OPERAND_BYTES:
         return False
     cos = attn.rope_cos
     if norm.weight.shape != (d,) or qkv.weight.shape != (3 * d, d) or out.weight.shape != (d, d) or \
@@ -231,17 +236,17 @@ def lm_head(h, norm, weight) -> torch.Tensor:
     return _LMHead.apply(h, norm.weight, weight, float(norm.eps))
 
 
-def _own_head_dx(tokens: int, d: int) -> bool:
+def _own_head_dx(tokens: int, d: int, vocab: int) -> bool:
     """dX contracts over the vocabulary into few tiles: the library's product
     leaves most CUs idle, the engine's splits K.  Library and engine, us, of 32000
     words: 93 / 44 (16 tokens, d 512), 104 / 32 (512, 512), 289 / 127 (4096,
     512), 325 / 227 (4096, 1024), 427 / 406 (4096, 2048), the last of the range
     where the engine was ahead.  1000 to 128256 words: the engine at most 4 %
     behind anywhere in it (8192 words, d 1024, 8192 tokens: 117 / 121)."""
-    return tokens * d <= 1 << 23
+    return tokens * d <= 1 << 23 and 2 * vocab * max(tokens, d) < _OPERAND_BYTES
 
 
-def _own_head_dw(d: int, vocab: int) -> bool:
+def _own_head_dw(d: int, vocab: int, tokens: int) -> bool:
     """dW on the engine where its 256-wide tiles fill their rounds of 256 CUs:
     0.8 of one round, 0.7 of several.  Library and engine, us, 4096 tokens: 131 /
     108 (32000 words, d 512: 250 tiles), 109 / 108 (26624: 208), 249 / 210 (32000,
@@ -252,7 +257,8 @@ def _own_head_dw(d: int, vocab: int) -> bool:
     and the library keeps them."""
     tiles = -(-d // 256) * -(-vocab // 256)
     rounds = -(-tiles // 256)
-    return d >= 512 and vocab >= 16384 and tiles >= (0.8 if rounds == 1 else 0.7) * 256 * rounds
+    return (d >= 512 and vocab >= 16384 and tiles >= (0.8 if rounds == 1 else 0.7) * 256 * rounds
+            and 2 * tokens * max(vocab, d) < _OPERAND_BYTES)
 
 
 class _LMHead(torch.autograd.Function):
@@ -288,11 +294,11 @@ class _LMHead(torch.autograd.Function):
         h2, g2 = h.reshape(-1, d), g.contiguous().reshape(-1, vocab)
         dh = dnw = dw = None
         if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-            dxn = K.gemm(g2, wb) if _own_head_dx(h2.shape[0], d) else torch.matmul(g2, wb)
+            dxn = K.gemm(g2, wb) if _own_head_dx(h2.shape[0], d, vocab) else torch.matmul(g2, wb)
             dh, dnw = (K.rmsnorm_backward_f32 if h.dtype == F32 else K.rmsnorm_backward)(h2, norm_w, rstd, dxn)
             dh = dh.reshape(h.shape)
         if ctx.needs_input_grad[2]:
-            dw = (K.gemm(g2.t(), xn, out_dtype=weight.dtype) if _own_head_dw(d, vocab)
+            dw = (K.gemm(g2.t(), xn, out_dtype=weight.dtype) if _own_head_dw(d, vocab, h2.shape[0])
                   else torch.matmul(g2.t(), xn).to(weight.dtype))
         return dh, dnw, dw, None
 

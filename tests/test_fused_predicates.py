@@ -8,7 +8,7 @@ import torch.nn as nn
 from torch.nn.modules.module import register_module_forward_hook
 
 from moc_amd import MoCConfig, build_model
-from moc_amd.block import _own_head_dw, attention_half_ok, lm_head_ok, next_token_loss_ok
+from moc_amd.block import _own_head_dw, _own_head_dx, attention_half_ok, lm_head_ok, next_token_loss_ok
 from moc_amd.ffn import block_ffn_f32_ok, block_ffn_ok
 from moc_amd.inference.decode_model import DecodeConfig, DecoderModel, make_step
 from moc_amd.inference.decode_model import RMSNorm as DecodeNorm
@@ -327,7 +327,7 @@ def test_attention_half_leaves_long_sequences_to_the_library(on_device):
                                          (1024, 8192, False)])
 def test_head_weight_gradient_takes_the_engine_where_its_rounds_fill(d, vocab, own):
     """Each side is the faster one measured (_own_head_dw)."""
-    assert _own_head_dw(d, vocab) == own
+    assert _own_head_dw(d, vocab, 4096) == own
 
 
 @pytest.mark.parametrize("p", [-1, 8, 100])
@@ -407,3 +407,17 @@ def test_decode_step_leaves_other_tensor_types_alone(on_device):
             model = _decoder()
             _wrap(getattr(model, part))
             assert not model._head_native(x)
+
+
+def test_attention_half_leaves_operands_of_2_gib_to_the_library(on_device):
+    """The engine addresses an operand with 32 bits: q/k/v rows of 1536 bytes here."""
+    blk = _block()
+    x = torch.zeros(1, dtype=BF).expand(43692, 32, 256)
+    assert _attn_ok(blk, x[:43000]) and not _attn_ok(blk, x)
+
+
+@pytest.mark.parametrize("tokens,d,vocab,dx,dw", [(32768, 256, 32000, True, False), (65536, 128, 32000, False, False),
+                                                  (4096, 2048, 32000, True, True), (65536, 1024, 32000, False, False),
+                                                  (2048, 4096, 262144, False, True), (2048, 4096, 131072, True, True), (2048, 4096, 524288, False, False)])
+def test_head_gradients_leave_operands_of_2_gib_to_the_library(tokens, d, vocab, dx, dw):
+    assert (_own_head_dx(tokens, d, vocab), _own_head_dw(d, vocab, tokens)) == (dx, dw)

@@ -248,3 +248,17 @@ def test_logits_take_writes_in_place(dtype):
     grads = [torch.autograd.grad(y, m.lm_head.weight, torch.ones_like(y))[0] for y in (got, want)]
     assert torch.equal(got, want) and torch.equal(*grads)
     assert (grads[0][7] == 0).all()
+
+
+@pytest.mark.parametrize("tokens,d,vocab", [(70000, 512, 16384), (70000, 512, 32000)])
+def test_lm_head_gradients_of_more_than_2_gib_of_logits(tokens, d, vocab):
+    g = torch.Generator(device="cuda").manual_seed(8)
+    h = torch.randn(1, tokens, d, generator=g, device="cuda").to(BF).requires_grad_()
+    w = (torch.randn(vocab, d, generator=g, device="cuda") / d ** 0.5).to(BF).requires_grad_()
+    norm = RMSNorm(d).to("cuda", BF)
+    dy = torch.randn(1, tokens, vocab, generator=g, device="cuda", dtype=BF)
+    got = torch.autograd.grad(lm_head(h, norm, w), (h, norm.weight, w), dy)
+    half = [torch.autograd.grad(lm_head(h[:, s], norm, w), (h, norm.weight, w), dy[:, s])
+            for s in (slice(0, 35000), slice(35000, None))]
+    for a, b, c in zip(got, *half):  # the halves' weight gradients are rounded, and their sum, which a's is not
+        assert (a.float() - (b.float() + c.float())).norm() <= 3 * 2.0 ** -9 * a.float().norm()
