@@ -88,11 +88,6 @@ def rms_norm_f32(x, w, eps: float):
     return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + eps) * w.float()
 
 
-# Bytes of a bf16 operand the engine addresses (32-bit offsets); larger products
-# are the library's.
-_OPERAND_BYTES = (1 << 31) - 1024
-
-
 # Longest sequence of the fused half; from there on the stock composition over
 # the library's attention is as fast or faster.  Stock time over fused, forward +
 # backward, 4096 tokens a pass (the last column one sequence of 8192):
@@ -123,7 +118,7 @@ def attention_half_ok(x, norm, norm_type, attn, attn_type) -> bool:
         return False
     d = x.shape[-1]
     if attn.head_dim not in (64, 128) or d != attn.num_heads * attn.head_dim or d > 4096 or x.numel() < 2 * d or \
-            x.shape[0] > 65535 or x.shape[1] > MAX_SEQ or 3 * x.numel() * 2 >= _OPERAND_BYTES:
+            x.shape[0] > 65535 or x.shape[1] > MAX_SEQ or 3 * x.numel() * 2 >= K.OPERAND_BYTES:
         return False
     cos = attn.rope_cos
     if norm.weight.shape != (d,) or qkv.weight.shape != (3 * d, d) or out.weight.shape != (d, d) or \
@@ -243,7 +238,7 @@ def _own_head_dx(tokens: int, d: int, vocab: int) -> bool:
     512), 325 / 227 (4096, 1024), 427 / 406 (4096, 2048), the last of the range
     where the engine was ahead.  1000 to 128256 words: the engine at most 4 %
     behind anywhere in it (8192 words, d 1024, 8192 tokens: 117 / 121)."""
-    return tokens * d <= 1 << 23 and 2 * vocab * max(tokens, d) < _OPERAND_BYTES
+    return tokens * d <= 1 << 23 and 2 * vocab * max(tokens, d) < K.OPERAND_BYTES
 
 
 def _own_head_dw(d: int, vocab: int, tokens: int) -> bool:
@@ -258,7 +253,7 @@ def _own_head_dw(d: int, vocab: int, tokens: int) -> bool:
     tiles = -(-d // 256) * -(-vocab // 256)
     rounds = -(-tiles // 256)
     return (d >= 512 and vocab >= 16384 and tiles >= (0.8 if rounds == 1 else 0.7) * 256 * rounds
-            and 2 * tokens * max(vocab, d) < _OPERAND_BYTES)
+            and 2 * tokens * max(vocab, d) < K.OPERAND_BYTES)
 
 
 class _LMHead(torch.autograd.Function):

@@ -62,6 +62,9 @@ def cu_count(device_index: int) -> int:
     return n
 
 
+# Bytes of a bf16 GEMM operand that the engine addresses (32-bit offsets).
+OPERAND_BYTES = (1 << 31) - 1024
+
 _unsafe_view = torch.ops.aten._unsafe_view.default
 
 
@@ -761,10 +764,18 @@ def global_after_gate(x, gate_scores, up_weight, down_weight_t, k: int, *, works
         # launches, like the reference's op, which accepts any batch
         # (optimized_global_moc_ext.cu:457-540).  U and Down as dense products:
         # the tokens' selections overlap (see moc_ffn_infer_bf16)
+        r = None if residual is None else residual.reshape(nb, hidden)
+        most = (OPERAND_BYTES - 1) // (2 * max(row_pitch(inter, torch.bfloat16), round_up(hidden, 8)))
+        if nb > most:  # in parts whose products' operands the engine addresses
+            step = -(-nb // -(-nb // most))
+            yy = torch.cat([global_after_gate(x[a:a + step], g[a:a + step], wu, wdt, k,
+                                              residual=None if r is None else r[a:a + step],
+                                              idx_out=None if idx_out is None else idx_out[a:a + step])
+                            for a in range(0, nb, step)])
+            return yy if out is None else out.copy_(yy)
         vals, idx, _ = topk_rows(g, int(k), idx_dtype=torch.int32)
         u = linear(x, wu, out=padded_empty(nb, inter, torch.bfloat16, x.device))
         z = sparse_forward_aux(vals, idx, u, inter, want_s=False, want_z=False)[3]
-        r = None if residual is None else residual.reshape(nb, hidden)
         if r is None or r.dtype == torch.bfloat16:
             yy = gemm(z, wdt, residual=r)
         else:  # the sum in the type that residual and layer promote to
@@ -933,6 +944,7 @@ def ffn_infer_fits(x2d: torch.Tensor, gate_weight, up_weight, down_weight_t) -> 
     nb, hidden = x2d.shape
     inter = gate_weight.shape[0]
     return (x2d.is_cuda and nb >= 1 and hidden % 8 == 0 and inter <= 16384
+            and 2 * nb * max(row_pitch(inter, torch.bfloat16), hidden) < OPERAND_BYTES
             and x2d.dtype == gate_weight.dtype == up_weight.dtype == down_weight_t.dtype == torch.bfloat16
             and gate_weight.shape == up_weight.shape == down_weight_t.shape == (inter, hidden)
             and gate_weight.is_contiguous() and up_weight.is_contiguous()

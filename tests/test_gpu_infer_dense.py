@@ -154,3 +154,24 @@ def test_after_gate_adds_a_residual_of_any_type(dtype):
     out = torch.empty(20, 64, dtype=BF, device="cuda")
     assert K.global_after_gate(x, g, w[1], wdt, 50, residual=res, out=out) is out
     assert torch.equal(out, want.to(BF))
+
+
+@pytest.mark.parametrize("residual", [False, True])
+def test_global_layer_of_more_than_2_gib_of_channels(residual):
+    """More tokens than a product's operands may hold: the layer in parts."""
+    nb, hidden, inter, k = 140000, 64, 8000, 8
+    x, w = _case(nb, hidden, inter, 13)
+    m = InferenceMoCSwiGLUFFN(hidden, inter, k).to("cuda", BF)
+    for p, t in zip((m.gate_proj, m.up_proj, m.down_proj), w):
+        p.weight.data.copy_(t)
+    parts = slice(0, 60000), slice(60000, 120000), slice(120000, None)
+    if residual:
+        wdt, g = K.down_weight_t_for_decode(w[2]), K.linear(x, w[0])
+        idx = torch.empty(nb, k, dtype=torch.int32, device="cuda")
+        got = K.global_after_gate(x, g, w[1], wdt, k, residual=x, idx_out=idx)
+        want = [K.global_after_gate(x[s], g[s], w[1], wdt, k, residual=x[s]) for s in parts]
+        assert torch.equal(idx, K.topk_rows(g, k, idx_dtype=torch.int32)[1])
+    else:
+        assert not K.ffn_infer_fits(x, w[0], w[1], K.down_weight_t_for_decode(w[2]))
+        got, want = m(x), [m(x[s]) for s in parts]
+    assert torch.equal(got, torch.cat(want))
