@@ -82,8 +82,8 @@ class StandardSwiGLUFFN(nn.Module):
 def _weights_fit(d: int, gate_w, up_w, down_w) -> bool:
     """Weights [inter, d], [inter, d] and [any, inter]: the kernels take d and
     inter from x and gate_w, the rest through bare pointers."""
-    return (gate_w.dim() == 2 and gate_w.shape[1] == d and up_w.shape == gate_w.shape
-            and down_w.dim() == 2 and down_w.shape[1] == gate_w.shape[0])
+    g = gate_w.shape
+    return len(g) == 2 and g[1] == d and up_w.shape == g and down_w.dim() == 2 and down_w.size(1) == g[0]
 
 
 def _check_inputs(x, gate_w, up_w, down_w, strict_aux: bool, index_save_dtype):
@@ -189,7 +189,7 @@ def _layer_forward(x, x2, gate_w, up_w, down_w, k, selection: str, idx_dtype, sa
     s_s = torch.empty((rows, kk), dtype=dt, device=dev) if save_s else None
     z_s = torch.empty((rows, kk), dtype=dt, device=dev) if save_s else None
     d_out = down_w.shape[0]
-    out = torch.empty((rows, d_out), dtype=dt, device=dev)
+    out = torch.empty((*x.shape[:-1], d_out), dtype=dt, device=dev)
     query = "moc_ffn_forward_f32_workspace_size" if f32 else "moc_ffn_forward_workspace_size"
     nbytes = _layer_ws_bytes(("f", f32, dev.index, rows, d, inter), query, rows, d, inter)
     ws = K._gemm_workspace(dev, nbytes) if nbytes > 0 else None
@@ -200,7 +200,7 @@ def _layer_forward(x, x2, gate_w, up_w, down_w, k, selection: str, idx_dtype, sa
              u_s.data_ptr(), N.ptr(s_s), N.ptr(z_s), out.data_ptr(), d_out, N.ptr(ws), nbytes,
              N.stream_of(x2))
     shp = (*x.shape[:-1], kk)
-    return (K.unaliased(out, (*x.shape[:-1], d_out)), idx.reshape(shp), vals.reshape(shp), u_s.reshape(shp),
+    return (out, idx.reshape(shp), vals.reshape(shp), u_s.reshape(shp),
             None if s_s is None else s_s.reshape(shp), None if z_s is None else z_s.reshape(shp))
 
 
@@ -682,7 +682,7 @@ class _MoCBlockFunction(torch.autograd.Function):
         mask = None
         if not bitmask and _block_native(h2, gate_w, up_w, down_w):
             out, idx, vals, u_s, s_s, z_s, rstd = _block_forward_native(
-                h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s=not gcp)
+                h, h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s=not gcp)
         else:
             xn, rstd = K.rmsnorm_rows(h2, norm_w, eps)
             out, idx, vals, u_s, s_s, z_s, *mk = _forward_common(
@@ -746,7 +746,7 @@ class _MoCBlockF32Function(torch.autograd.Function):
         native = not bitmask and _block_f32_native(h2, gate_w, down_w)
         if native:
             out, idx, vals, u_s, s_s, z_s, xn, rstd = _block_forward_f32_native(
-                h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s=not gcp)
+                h, h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s=not gcp)
             mask = ()
         else:
             xn, rstd = K.rmsnorm_rows_f32(h2, norm_w, eps)
@@ -799,7 +799,7 @@ def _block_f32_native(h2, gate_w, down_w) -> bool:
             and h2.is_contiguous() and _side_for(h2.device, rows, inter) is None)
 
 
-def _block_forward_f32_native(h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s):
+def _block_forward_f32_native(h, h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s):
     """moc_ffn_block_forward_f32: casts, norm, FFN and residual in one call."""
     rows, d = h2.shape
     inter = gate_w.shape[0]
@@ -812,7 +812,7 @@ def _block_forward_f32_native(h2, norm_w, eps, gate_w, up_w, down_w, k, selectio
     gu = torch.empty((2, rows, pitch), dtype=bf16, device=dev)
     sel = [torch.empty((rows, kk), dtype=bf16, device=dev) for _ in range(4 if save_s else 2)]
     idx = torch.empty((rows, kk), dtype=idx_dtype, device=dev)
-    out = torch.empty_like(h2)
+    out = torch.empty_like(h)
     ncast = _layer_ws_bytes(("c", rows, d, inter), "moc_ffn_block_f32_cast_size", rows, d, inter)
     cast = torch.empty(ncast, dtype=torch.uint8, device=dev)
     nbytes = _layer_ws_bytes(("f", False, dev.index, rows, d, inter), "moc_ffn_forward_workspace_size",
@@ -863,7 +863,7 @@ def _block_backward_f32_native(dout, h2, xn, rstd, norm_w, idx, g_s, u_s, s_s, z
     return dh, dnw, dwg, dwu, dwd
 
 
-def _block_forward_native(h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s):
+def _block_forward_native(h, h2, norm_w, eps, gate_w, up_w, down_w, k, selection, idx_dtype, save_s):
     """moc_ffn_block_forward_bf16: the norm, the FFN and the residual add in
     one call (the launches of the unfused path in the same order)."""
     rows, d = h2.shape
@@ -881,7 +881,7 @@ def _block_forward_native(h2, norm_w, eps, gate_w, up_w, down_w, k, selection, i
     u_s = torch.empty((rows, kk), dtype=dt, device=dev)
     s_s = torch.empty((rows, kk), dtype=dt, device=dev) if save_s else None
     z_s = torch.empty((rows, kk), dtype=dt, device=dev) if save_s else None
-    out = torch.empty((rows, d), dtype=dt, device=dev)
+    out = torch.empty(h.shape, dtype=dt, device=dev)
     nbytes = _layer_ws_bytes(("f", False, dev.index, rows, d, inter), "moc_ffn_forward_workspace_size",
                              rows, d, inter)
     ws = K._gemm_workspace(dev, nbytes) if nbytes > 0 else None

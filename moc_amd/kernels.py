@@ -69,10 +69,10 @@ _unsafe_view = torch.ops.aten._unsafe_view.default
 
 
 def unaliased(t: torch.Tensor, shape) -> torch.Tensor:
-    """t, made by the caller and used nowhere else, in another shape and no
-    view of t: what a custom Function returns.  Autograd lets no result of a
+    """t, made by the caller, no view and used nowhere else, in another shape and
+    no view of t: what a custom Function returns.  Autograd lets no result of a
     Function that is a view be written in place."""
-    return _unsafe_view(t, shape)
+    return t if t.shape == shape else _unsafe_view(t, shape)
 
 
 def gemm_tiles(m: int, n: int) -> int:
@@ -944,7 +944,7 @@ def ffn_infer_fits(x2d: torch.Tensor, gate_weight, up_weight, down_weight_t) -> 
     nb, hidden = x2d.shape
     inter = gate_weight.shape[0]
     return (x2d.is_cuda and nb >= 1 and hidden % 8 == 0 and inter <= 16384
-            and 2 * nb * max(row_pitch(inter, torch.bfloat16), hidden) < OPERAND_BYTES
+            and 2 * nb * max(inter + 64, hidden) < OPERAND_BYTES
             and x2d.dtype == gate_weight.dtype == up_weight.dtype == down_weight_t.dtype == torch.bfloat16
             and gate_weight.shape == up_weight.shape == down_weight_t.shape == (inter, hidden)
             and gate_weight.is_contiguous() and up_weight.is_contiguous()
