@@ -262,3 +262,17 @@ def test_lm_head_gradients_of_more_than_2_gib_of_logits(tokens, d, vocab):
             for s in (slice(0, 35000), slice(35000, None))]
     for a, b, c in zip(got, *half):  # the halves' weight gradients are rounded, and their sum, which a's is not
         assert (a.float() - (b.float() + c.float())).norm() <= 3 * 2.0 ** -9 * a.float().norm()
+
+
+def test_entry_without_a_copy():
+    """moc_next_token_loss_forward: the same loss and row values as with the copy, which is the logits."""
+    from moc_amd import _native as N
+    x = torch.randn(2, 5, 4104, device="cuda").to(BF)
+    labels = torch.randint(0, 4104, (2, 5), device="cuda")
+    labels[1, 3] = -100
+    keep, bufs, losses = torch.zeros_like(x), torch.zeros(2, 21, device="cuda"), torch.zeros(2, device="cuda")
+    for i, name in enumerate(("moc_next_token_loss_forward", "moc_next_token_loss_forward_keep")):
+        p = bufs[i].data_ptr()
+        N.call(name, x.data_ptr(), 4104, 2, 5, 4104, labels.data_ptr(), -100, p, p + 40, losses[i].data_ptr(),
+               N.MOC_F32, p + 80, *((keep.data_ptr(), 4104) if i else ()), N.stream_of(x))
+    assert torch.equal(bufs[0], bufs[1]) and torch.equal(losses[0], losses[1]) and torch.equal(keep, x)
